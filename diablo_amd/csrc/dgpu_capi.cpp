@@ -46,7 +46,7 @@ struct dgpu_ctx {
     cx<double> *d_iptw = nullptr;
     cx<float> *d_iptwf = nullptr;
     int ld = 0;      // row length of the intermediates (>= mk, multiple of 8)
-    int xchunk = 64; // planes per block of the fused x kernel (set at creation)
+    int xchunk = 64; // planes per block of the fused x kernel (xfused_auto_chunk's at creation)
     int colnw = 8;   // waves per block of the segmented column kernels; 0: whole-column sweeps
     int colfuse = -1;     // fused column kernel: -1 where NY >= 160 (FP64: at 8 waves), 0 never, 1 where it fits
     // mixed paths: FP32 transforms, intermediates and nonlinear terms
@@ -513,11 +513,6 @@ int32_t dgpu_create(const dgpu_params *p, dgpu_ctx **out)
             delete c;
             return DGPU_E_ARG;
         }
-        // planes per block: what dgpu_autotune measures best at 384x257x384
-        // (64 in FP64, 32 with the FP32 transforms: three full rounds of
-        // resident blocks either way, at two and four blocks per CU)
-        c->xchunk = c->mixed ? 32 : 64;
-        if (xc && std::atoi(xc) > 0) c->xchunk = std::atoi(xc);
         // column stage: DGPU_COLSEG=0 selects the whole-column sweeps,
         // DGPU_COLSEG_NW the waves per block of the segmented kernels
         const char *cs = std::getenv("DGPU_COLSEG"), *cw = std::getenv("DGPU_COLSEG_NW");
@@ -539,6 +534,13 @@ int32_t dgpu_create(const dgpu_params *p, dgpu_ctx **out)
         const char *zs = std::getenv("DGPU_ZSWZ");  // 0 turns the column-batch swizzle off
         c->ipz.cswz = (zs && std::atoi(zs) == 0) ? 0 : dgpu::ip_pick_cswz(c->ipz, zw);
         c->ld = (g.mk + 7) / 8 * 8;
+        if (xc && std::atoi(xc) > 0) {
+            c->xchunk = std::atoi(xc);
+        } else {
+            const int jlo = g.nth ? std::min(2, c->jstart_th[0]) : 2;
+            c->xchunk = c->mixed ? dgpu::xfused_auto_chunk<float>(g, c->ipx, jlo, g.ny)
+                                 : dgpu::xfused_auto_chunk<double>(g, c->ipx, jlo, g.ny);
+        }
     }
     int rc = 0;
     auto bail = [&](int code) { rc = code; dgpu_destroy(c); return code; };
@@ -2138,6 +2140,9 @@ static int ens_build_groups(dgpu_ensemble *e)
         std::vector<dgpu::ScatDesc<double, float>> sc;
         for (int i : gr.idx) {
             dgpu_ctx *c = e->m[i];
+            // the group's launches fill the GPU with whole sweeps of many
+            // members: longer chunks than a member alone would take
+            if (!std::getenv("DGPU_XCHUNK")) c->xchunk = mixed ? 32 : 64;
             const int jlo = member_jlo(c), ny = c->g.ny;
             gr.max_planes = std::max(gr.max_planes, ny + 2);
             gr.max_span = std::max(gr.max_span, ny - jlo + 1);

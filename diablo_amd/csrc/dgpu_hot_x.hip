@@ -3,6 +3,9 @@
 // (for/courant.f:35-44), on the in-place transforms of dgpu_fft.hpp.
 #include "dgpu_hot.hpp"
 
+#include <algorithm>
+#include <cmath>
+
 namespace dgpu {
 
 // -------------------------------------------------------------------------
@@ -456,13 +459,55 @@ static int xfused_zrows(const IpLen &fx, int nz, int mk)
     return zr;
 }
 
+// Planes per block when the caller leaves the choice (dgpu_create): the fewest
+// rounds of resident blocks times a block's iterations.  A block of c planes
+// runs about c + 1.5 iterations (two of its c + 2 backward planes share one
+// pass), and an iteration takes nearly the same time whether a CU holds one
+// block or all that fit, so up to one full round only the chunk's length
+// counts.  Beyond it a round that is partly empty costs a whole one while the
+// rounds are few; over many rounds blocks even that out by half.  On small
+// grids the former fixed 64 (FP64) / 32 planes left most CUs without a block:
+// one RK3 step at 64x65x64 FP64 1502 -> 219 us (2 planes), 96x81x108 1984 ->
+// 520, 192x129x192 2819 -> 1840; at 384x257x384 the rule gives the 64 (FP64)
+// and 32 (FP32) planes measured best there.
+static int xfused_rule(long rows, int planes, long slots)
+{
+    int best = planes;
+    double best_cost = 1e300;
+    for (int n = 1; n <= planes; ++n) {
+        const int c = (planes + n - 1) / n;
+        const long blocks = rows * ((planes + c - 1) / c);
+        const double r = (double)blocks / (double)slots, up = std::ceil(r);
+        const double rounds = r <= 3.0 ? std::max(1.0, up) : r + 0.5 * (up - r);
+        const double cost = rounds * (c + 1.5);
+        if (cost < best_cost * (1.0 - 1e-9)) {
+            best_cost = cost;
+            best = c;
+        }
+    }
+    return best;
+}
+
+// Blocks of a kernel that the whole device holds at once.
+template <class K>
+static long xfused_slots(K kernel, int threads, size_t lds)
+{
+    int per = 0, dev = 0, cus = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, lds) != hipSuccess || per < 1) per = 1;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+        cus = 256;
+    (void)hipGetLastError();
+    return (long)per * cus;
+}
+
+// pick: nothing is launched, *pick receives the rule's planes per block
 template <typename T, int E, int NTH, int PID>
 static void xfused_ip_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, int ld, const cx<T> *zt,
                         long zt_fs, cx<T> *wt, long wt_fs, const double *dy, const double *dyf, const double *kx,
-                        int jlo, int jhi, int chunk)
+                        int jlo, int jhi, int chunk, int *pick)
 {
     using C = XCount<NTH>;
-    const int nchunks = (jhi - jlo + 1 + chunk - 1) / chunk;
     const int zr = xfused_zrows<T, NTH>(fx, g.nz, g.mk);
     const int threads = zr * fx.t * (C::npi + C::npo);
     const size_t lds =
@@ -473,6 +518,12 @@ static void xfused_ip_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T
                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         attr = true;
     }
+    if (pick) {
+        *pick = xfused_rule((g.nz + zr - 1) / zr, jhi - jlo + 1,
+                            xfused_slots(&k_xfused_ip<T, E, NTH, PID>, threads, lds));
+        return;
+    }
+    const int nchunks = (jhi - jlo + 1 + chunk - 1) / chunk;
     const long ps = (long)g.nz * ld;
     hipLaunchKernelGGL((k_xfused_ip<T, E, NTH, PID>), dim3((g.nz + zr - 1) / zr, nchunks), dim3(threads), lds, s, fx,
                        tw, g.mk, ld, zt, zt_fs, ps, wt, wt_fs, ps, dy, dyf, kx, jlo, jhi, chunk, zr, g.nz);
@@ -482,22 +533,24 @@ static void xfused_ip_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T
 // The single-run x kernel is built for the 384 and 256 plans (the ensembles
 // use the batched kernel) with one scalar; other shapes run on runtime plans.
 template <typename T>
-void launch_xfused_ip(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, int ld, const cx<T> *zt,
-                      long zt_fs, cx<T> *wt, long wt_fs, const double *dy, const double *dyf, const double *kx,
-                      int jlo, int jhi, int chunk)
+static void xfused_ip_any(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, int ld, const cx<T> *zt,
+                          long zt_fs, cx<T> *wt, long wt_fs, const double *dy, const double *dyf, const double *kx,
+                          int jlo, int jhi, int chunk, int *pick)
 {
     if (g.nth == 1 && with_pid(const_plan_id(fx), XPidsSingle<T>{}, [&](auto pc) {
             constexpr int P = decltype(pc)::value;
             xfused_ip_e<T, kConstPlanSpecs[P].e, 1, P>(s, g, fx, tw, ld, zt, zt_fs, wt, wt_fs, dy, dyf, kx, jlo, jhi,
-                                                       chunk);
+                                                       chunk, pick);
         }))
         return;
 #define DGPU_XF(EE_)                                                                                             \
     do {                                                                                                         \
         if (g.nth == 0)                                                                                          \
-            xfused_ip_e<T, EE_, 0, 0>(s, g, fx, tw, ld, zt, zt_fs, wt, wt_fs, dy, dyf, kx, jlo, jhi, chunk);     \
+            xfused_ip_e<T, EE_, 0, 0>(s, g, fx, tw, ld, zt, zt_fs, wt, wt_fs, dy, dyf, kx, jlo, jhi, chunk,      \
+                                      pick);                                                                     \
         else                                                                                                     \
-            xfused_ip_e<T, EE_, 1, 0>(s, g, fx, tw, ld, zt, zt_fs, wt, wt_fs, dy, dyf, kx, jlo, jhi, chunk);     \
+            xfused_ip_e<T, EE_, 1, 0>(s, g, fx, tw, ld, zt, zt_fs, wt, wt_fs, dy, dyf, kx, jlo, jhi, chunk,      \
+                                      pick);                                                                     \
     } while (0)
     switch (fx.e) {
     case 4: DGPU_XF(4); break;
@@ -510,6 +563,22 @@ void launch_xfused_ip(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> 
     default: break;
     }
 #undef DGPU_XF
+}
+
+template <typename T>
+void launch_xfused_ip(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, int ld, const cx<T> *zt,
+                      long zt_fs, cx<T> *wt, long wt_fs, const double *dy, const double *dyf, const double *kx,
+                      int jlo, int jhi, int chunk)
+{
+    xfused_ip_any<T>(s, g, fx, tw, ld, zt, zt_fs, wt, wt_fs, dy, dyf, kx, jlo, jhi, chunk, nullptr);
+}
+
+template <typename T>
+int xfused_auto_chunk(const Geo &g, const IpLen &fx, int jlo, int jhi)
+{
+    int c = 0;
+    xfused_ip_any<T>(nullptr, g, fx, nullptr, 0, nullptr, 0, nullptr, 0, nullptr, nullptr, nullptr, jlo, jhi, 1, &c);
+    return c > 0 ? c : 32;
 }
 
 template <typename T, int E, int NTH, int PID>
@@ -595,6 +664,8 @@ void launch_vmax_ip(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *t
     DGPU_DISPATCH_IPE(fx.e, (vmax_ip_e<T, EE>(s, g, fx, tw, ld, zt, zt_fs, part, out)));
 }
 
+template int xfused_auto_chunk<double>(const Geo &, const IpLen &, int, int);
+template int xfused_auto_chunk<float>(const Geo &, const IpLen &, int, int);
 template void launch_vmax_ip<double>(hipStream_t, const Geo &, const IpLen &, const cx<double> *, int,
                                      const cx<double> *, long, double *, double *);
 template void launch_vmax_ip<float>(hipStream_t, const Geo &, const IpLen &, const cx<float> *, int,
