@@ -97,7 +97,14 @@ struct dgpu_ctx {
     bool zdft = false;
     uint16_t *d_zdft = nullptr;
     dgpu::ZdftTab zinv_tab{}, zfwd_tab{};
-    double *d_les = nullptr;   // LES work planes, NU_T, SGS force, filter widths
+    // pair planes (dgpu_pairs.hip): FP64 x plan and twiddles, slots of x and z
+    // in natural order, npairs physical pairs
+    dgpu::IpLen ipx64{};
+    cx<double> *d_pairtw = nullptr;
+    int *d_perm = nullptr;
+    cx<double> *d_pairs = nullptr;
+    int npairs = 0;
+    double *d_les = nullptr;   // LES: NU_T, wall rows, saved rows, per-row constants
     bool les = false, les_model = false;  // input.dat's LES; les_chan called in each substep
     // CN tables: [stage 0..2][sys][NY+2][kRow]
     double *d_cn = nullptr;
@@ -737,7 +744,8 @@ int32_t dgpu_destroy(dgpu_ctx *c)
     void *bufs[] = {c->d_vec, c->d_tw, c->d_state, c->d_pmult, c->d_pinv, c->d_rd, c->d_nlptr, c->d_zt, c->d_wt,
                     c->d_fa, c->d_fb, c->d_iptw, c->d_iptwf, c->d_ztf, c->d_wtf, c->d_nlf, c->d_nlptrf,
                     c->d_fort, c->d_cn, c->d_codes, c->d_c1, c->d_state32, c->d_side, c->d_map,
-                    c->d_pmultf, c->d_pinvf, c->d_gs32, c->d_stats, c->d_vmax_part, c->d_vmax, c->d_file, c->d_les, c->d_zdft};
+                    c->d_pmultf, c->d_pinvf, c->d_gs32, c->d_stats, c->d_vmax_part, c->d_vmax, c->d_file, c->d_les, c->d_zdft,
+                    c->d_pairtw, c->d_perm, c->d_pairs};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     if (c->side_stream) {
@@ -1098,94 +1106,196 @@ int32_t dgpu_get_column_shape(const dgpu_ctx *c, int32_t *waves, int32_t *fused)
 // ---------------------------------------------------------------------------
 // LES (for/les.f, for/channel.f:303-386, 628-659, 748-1003)
 // ---------------------------------------------------------------------------
-// Work planes, Fortran layout (NX+2) x (NZ+2) x (NY+2) doubles each:
-//   0-7   S_ij (3-7, 1) and U1, U3 (0, 2) for the model; in the substep
-//         physical U1, U2, U3, R1, R2, R3 (0-5) and Thomas scratch (6, 7)
-//   8-12  the stress parts to transform; in the substep CS1 (8), TH (9), RTH
-//         (10), Thomas scratch (8, 11, 12, with 14-16 once the SGS force is
-//         spent)
-//   13    NU_T (kept between substeps; KAPPA_T equals it)
-//   14-17 the SGS force for CF1, CF2, CF3, CFTH (kept modes)
-//   18    rows 1 and NY of CU1, CU3 before les_chan's BCs (kept modes)
-// then DELTA_YF, DELTA_Y.
-static const int kLesBufs = 19;
+// d_les holds NU_T on pair planes (kept between substeps; KAPPA_T equals it),
+// the wall rows after APPLY_BC_VEL_PHYS (k_les_bc_rows), rows 1 and NY of CU1
+// and CU3 before les_chan's BCs (kept modes), and the per-row constants of
+// k_les_prod.  Pair planes 0-5 are the fields of dgpu_les.hip (2-5 also the
+// solves' scratch, once k_les_prod has run), 6 and 7 the right-hand sides.
+static const int kLesPairs = 8;
 
-static size_t les_n(const dgpu_ctx *c)
+static long pair_plane(const dgpu_ctx *c) { return (long)c->g.nx * c->g.nz; }
+static long pair_fs(const dgpu_ctx *c) { return pair_plane(c) * (c->g.ny + 2); }
+static cx<double> *pair_buf(dgpu_ctx *c, int q) { return c->d_pairs + (size_t)q * pair_fs(c); }
+
+// The FP64 x plan of the pair transforms (the context's own in FP64 contexts;
+// mixed ones plan for 16 values per thread, which FP64 would spill) and n pair
+// planes.
+static int ensure_pairs(dgpu_ctx *c, int n)
 {
-    return (size_t)(c->g.nx + 2) * (c->g.nz + 2) * (c->g.ny + 2);
+    const dgpu::Geo &g = c->g;
+    if (!c->d_pairtw) {
+        dgpu::IpLen f = c->ipx;
+        if (c->mixed) {
+            if (!dgpu::ip_plan_x(g.nx, 0, 12, 128, f)) return fail(c, DGPU_E_ARG, "no FP64 plan for NX");
+            dgpu::ip_pick_swizzle(f, 4);
+        }
+        std::vector<cx<double>> tw;
+        dgpu::ip_twiddles(f, tw);
+        std::vector<int> perm(g.nz + g.nx);
+        for (int k = 0; k < g.nz; ++k) perm[k] = dgpu::pair_zpos(c->ipz, k);
+        for (int i = 0; i < g.nx; ++i) perm[g.nz + i] = dgpu::pair_slot(f, i);
+        if (!c->d_perm) HIPCHK(c, hipMalloc(&c->d_perm, sizeof(int) * perm.size()));
+        HIPCHK(c, hipMemcpy(c->d_perm, perm.data(), sizeof(int) * perm.size(), hipMemcpyHostToDevice));
+        cx<double> *d = nullptr;
+        HIPCHK(c, hipMalloc(&d, sizeof(cx<double>) * tw.size()));
+        if (hipMemcpy(d, tw.data(), sizeof(cx<double>) * tw.size(), hipMemcpyHostToDevice) != hipSuccess) {
+            (void)hipFree(d);
+            return fail(c, DGPU_E_HIP, "pair twiddles");
+        }
+        c->ipx64 = f;
+        c->d_pairtw = d;
+    }
+    if (c->npairs < n) {
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        if (c->d_pairs) HIPCHK(c, hipFree(c->d_pairs));
+        c->d_pairs = nullptr;
+        c->npairs = 0;
+        HIPCHK(c, hipMalloc(&c->d_pairs, sizeof(cx<double>) * (size_t)n * pair_fs(c)));
+        c->npairs = n;
+    }
+    return DGPU_OK;
 }
 
-static double *les_buf(dgpu_ctx *c, int q) { return c->d_les + (size_t)q * les_n(c); }
+// Kept modes of CU1-3, CTH (and, with grads, their z derivatives) to the rows
+// Wt, fields 0..nin-1 (nin..2 nin-1).
+static int pairs_z(dgpu_ctx *c, bool grads)
+{
+    const int nin = 3 + c->g.nth;
+    dgpu::ZSrc z{};
+    z.n = grads ? 2 * nin : nin;
+    for (int q = 0; q < z.n; ++q) {
+        z.p[q] = q % nin < 3 ? c->cu[q % nin] : c->cth[0];
+        z.dz[q] = q >= nin;
+    }
+    dgpu::launch_zinv_src(c->stream, c->g, c->ipz, c->d_iptw + c->ipx.twn, z, c->d_wt, c->zfs, c->ld, c->d_kz, 0,
+                          c->g.ny + 2);
+    return check_launch(c, "zinv(pairs)");
+}
+
+static int pairs_x(dgpu_ctx *c, const dgpu::PairSrc &src, const cx<double> *zt, int first)
+{
+    dgpu::PairDst dst{};
+    for (int q = 0; q < src.n; ++q) dst.p[q] = pair_buf(c, first + q);
+    dgpu::launch_pairs_inv(c->stream, c->g, c->ipx64, c->d_pairtw, c->ld, zt, c->zfs, src, dst, c->d_kx, 0,
+                           c->g.ny + 2);
+    return check_launch(c, "x inverse(pairs)");
+}
+
+// (U1, U2), (U3, TH) of Wt's first fields
+static dgpu::PairSrc pairs_of_fields(const dgpu_ctx *c)
+{
+    return dgpu::PairSrc{{0, 2}, {-1, -1}, {1, c->g.nth ? 3 : -1}, {-1, -1}, 2};
+}
+
+struct LesMem {
+    double *nut;         // NU_T
+    cx<double> *bc;      // [2][4][NZ*NX]
+    cx<double> *pre;     // [4][ps]
+    double *tab;         // [NY+2][8]
+    size_t bytes;
+};
+static LesMem les_mem(const dgpu_ctx *c)
+{
+    LesMem m;
+    char *b = reinterpret_cast<char *>(c->d_les);
+    size_t at = 0;
+    auto take = [&](size_t n) {
+        char *p = b ? b + at : nullptr;
+        at += (n + 255) / 256 * 256;
+        return p;
+    };
+    m.nut = reinterpret_cast<double *>(take(sizeof(double) * pair_fs(c)));
+    m.bc = reinterpret_cast<cx<double> *>(take(sizeof(cx<double>) * 8 * pair_plane(c)));
+    m.pre = reinterpret_cast<cx<double> *>(take(sizeof(cx<double>) * 4 * c->g.ps));
+    m.tab = reinterpret_cast<double *>(take(sizeof(double) * 8 * (c->g.ny + 2)));
+    m.bytes = at;
+    return m;
+}
 
 static int ensure_les(dgpu_ctx *c)
 {
+    if (int rc = ensure_pairs(c, kLesPairs)) return rc;
     if (c->d_les) return DGPU_OK;
     const dgpu::Geo &g = c->g;
     const int NY = g.ny;
-    const size_t n = les_n(c);
-    HIPCHK(c, hipMalloc(&c->d_les, (kLesBufs * n + 2 * (size_t)(NY + 2)) * sizeof(double)));
-    // NU_T's padding and the unset rows of the work planes stay zero
-    HIPCHK(c, hipMemsetAsync(c->d_les, 0, kLesBufs * n * sizeof(double), c->stream));
-    // filter widths with -2 C_SMAG^2 absorbed (for/les.f:200-223):
-    // C_SMAG = 0.13, beta_sgs = 1, DELTA = (DX DY 2 DZ)^(1/3)
+    const size_t bytes = les_mem(c).bytes;
+    void *mem = nullptr;
+    HIPCHK(c, hipMalloc(&mem, bytes));
+    c->d_les = reinterpret_cast<double *>(mem);
+    // NU_T starts at zero; its rows outside k_les_prod's stay zero
+    HIPCHK(c, hipMemsetAsync(mem, 0, bytes, c->stream));
+    // per-row constants; filter widths with -2 C_SMAG^2 absorbed
+    // (for/les.f:200-223): C_SMAG = 0.13, beta_sgs = 1, DELTA = (DX DY 2 DZ)^(1/3)
     const double C_SMAG = 0.13, beta_sgs = 1.0;
     const double dx = c->p.lx / g.nx, dz = c->p.lz / g.nz;
-    std::vector<double> dl(2 * (size_t)(NY + 2), 0.0);
-    for (int j = 1; j <= NY + 1; ++j) {
-        dl[j] = -2.0 * std::pow(C_SMAG, 2.0) * std::pow(dx * beta_sgs * c->dyf[j] * 2.0 * dz * beta_sgs, 2.0 / 3.0);
-        dl[NY + 2 + j] =
-            -2.0 * std::pow(C_SMAG, 2.0) * std::pow(dx * beta_sgs * c->dy[j] * 2.0 * dz * beta_sgs, 2.0 / 3.0);
+    const std::vector<double> &DY = c->dy, &DYF = c->dyf;
+    std::vector<double> t(8 * (size_t)(NY + 2), 0.0);
+    for (int j = 0; j <= NY + 1; ++j) {
+        double *r = &t[8 * (size_t)j];
+        r[0] = DYF[j] != 0.0 ? 1.0 / DYF[j] : 0.0;
+        r[1] = DY[j] != 0.0 ? 1.0 / DY[j] : 0.0;
+        r[2] = 0.5 * r[0];
+        if (j < 1) continue;
+        r[3] = DYF[j - 1] / (2.0 * DY[j]);
+        r[4] = DYF[j] / (2.0 * DY[j]);
+        r[5] = -2.0 * std::pow(C_SMAG, 2.0) * std::pow(dx * beta_sgs * DYF[j] * 2.0 * dz * beta_sgs, 2.0 / 3.0);
+        r[6] = -2.0 * std::pow(C_SMAG, 2.0) * std::pow(dx * beta_sgs * DY[j] * 2.0 * dz * beta_sgs, 2.0 / 3.0);
     }
-    HIPCHK(c, hipMemcpyAsync(c->d_les + kLesBufs * n, dl.data(), dl.size() * sizeof(double), hipMemcpyHostToDevice,
-                             c->stream));
+    HIPCHK(c, hipMemcpyAsync(les_mem(c).tab, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return DGPU_OK;
 }
 
 // les_chan with LES_MODEL_TYPE = 1 (for/les.f:1-331) at NPROCY = 1: the
-// velocity BCs and APPLY_BC_LES on the state, S_ij and U1, U3 to physical
-// space, |S| and NU_T, tau_ij back to Fourier space and its divergence
-// subtracted from f1-f3 (the reference's CF1-3), then the explicit cross
-// terms NU_T dU/dy added to f2.  fresh: f1-f3 start from zero (the SGS
-// force alone) and need no clear beforehand.
-static int les_model(dgpu_ctx *c, cx<double> *f1, cx<double> *f2, cx<double> *f3, bool fresh)
+// velocity BCs and APPLY_BC_LES on the state, its physical fields and
+// gradients, then the model and, unless force asks for the SGS force alone,
+// RK_CHAN_1's products and the scalar's eddy flux: the nonlinear terms (x, y,
+// z momentum, scalar) of rows jlo..NY in c->nl, NU_T in d_les, the physical
+// wall rows after APPLY_BC_VEL_PHYS in d_les.
+static int les_terms(dgpu_ctx *c, int jlo, bool force)
 {
     const dgpu::Geo &g = c->g;
-    const int NY = g.ny;
-    const size_t n = les_n(c);
-    const double *delta_yf = c->d_les + kLesBufs * n, *delta_y = delta_yf + (NY + 2);
-    dgpu::LesPtrs S, O;
-    // S_ij in planes 3-7 and 1, U1 and U3 in planes 0 and 2 (where the
-    // substep keeps its physical U1, U3)
-    const int splane[8] = {3, 4, 5, 6, 7, 1, 0, 2};
-    for (int q = 0; q < 8; ++q) S.p[q] = les_buf(c, splane[q]);
-    for (int q = 0; q < 6; ++q) O.p[q] = les_buf(c, 8 + q);
-    O.p[6] = O.p[7] = nullptr;
+    const int nin = 3 + g.nth;
+    const LesMem m = les_mem(c);
     dgpu::launch_apply_bc_vel(c->stream, g, c->cu[0], c->cu[1], c->cu[2], c->d_codes, c->d_c1, c->d_dy, c->d_dyf);
     if (int rc = check_launch(c, "apply_bc_vel")) return rc;
     dgpu::launch_les_bc(c->stream, g, c->cu[0], c->cu[2], c->p.u_bc_ymin, c->p.u_bc_ymax, c->p.w_bc_ymin,
                         c->p.w_bc_ymax);
     if (int rc = check_launch(c, "les_bc")) return rc;
-    dgpu::launch_les_strain(c->stream, g, c->cu[0], c->cu[1], c->cu[2], c->d_kx, c->d_kz, c->d_dy, c->d_dyf, S);
-    if (int rc = check_launch(c, "les_strain")) return rc;
-    for (int q = 0; q < 8; ++q)
-        if (int rc = fort_to_physical(c, S.p[q], 0, NY + 1)) return rc;
-    dgpu::launch_les_nut(c->stream, g, S, O, c->cu[0], c->cu[2], c->d_dy, c->d_dyf, delta_y, c->jstart, c->jend);
-    if (int rc = check_launch(c, "les_nut")) return rc;
-    for (int q = 0; q < 5; ++q)
-        if (int rc = fort_to_fourier(c, O.p[q], 0, NY + 1)) return rc;
-    // CF1, CF3 on J1 = JSTART .. J2 = NY-1 (the RANKY = NPROCY-1 bounds, for/les.f:46-50)
-    dgpu::launch_les_cf(c->stream, g, O, f1, f2, f3, c->d_kx, c->d_kz, c->d_dyf, delta_y, delta_yf, c->jstart,
-                        NY - 1, fresh);
-    if (int rc = check_launch(c, "les_cf")) return rc;
-    for (int pass = 0; pass < 2; ++pass) {
-        dgpu::launch_les_cross_src(c->stream, g, O.p[5], S.p[6 + pass], c->d_dy, O.p[0]);
-        if (int rc = check_launch(c, "les_cross_src")) return rc;
-        if (int rc = fort_to_fourier(c, O.p[0], 2, NY)) return rc;
-        dgpu::launch_les_cross_add(c->stream, g, O.p[0], f2, c->d_kx, c->d_kz, pass);
-        if (int rc = check_launch(c, "les_cross_add")) return rc;
+    if (int rc = pairs_z(c, true)) return rc;
+    const int th = g.nth ? 3 : -1, dth = g.nth ? nin + 3 : -1;
+    // pairs 0-5 (dgpu_les.hip): plain rows, x derivatives, z derivatives
+    dgpu::PairSrc src{{0, 2, -1, nin, nin + 1, dth},
+                      {-1, -1, 0, 2, -1, -1},
+                      {1, th, -1, nin + 2, -1, -1},
+                      {-1, -1, 1, -1, th, -1},
+                      g.nth ? 6 : 5};
+    if (int rc = pairs_x(c, src, c->d_wt, 0)) return rc;
+    dgpu::LesBc b;
+    b.u_lo = c->p.u_bc_ymin; b.u_hi = c->p.u_bc_ymax; b.w_lo = c->p.w_bc_ymin; b.w_hi = c->p.w_bc_ymax;
+    b.v_lo = c->p.v_bc_ymin; b.v_hi = c->p.v_bc_ymax;
+    b.u_lo_c = c->p.u_bc_ymin_c1; b.u_hi_c = c->p.u_bc_ymax_c1; b.w_lo_c = c->p.w_bc_ymin_c1;
+    b.w_hi_c = c->p.w_bc_ymax_c1; b.v_lo_c = c->p.v_bc_ymin_c1; b.v_hi_c = c->p.v_bc_ymax_c1;
+    dgpu::launch_les_bc_rows(c->stream, g, pair_buf(c, 0), pair_buf(c, 1), m.bc, b, c->d_dy, c->d_dyf);
+    if (int rc = check_launch(c, "les_bc_rows")) return rc;
+    dgpu::LesProd a{};
+    for (int q = 0; q < src.n; ++q) a.pr[q] = pair_buf(c, q);
+    a.bc = m.bc; a.nut = m.nut; a.wt = c->d_wt; a.wt_fs = c->zfs; a.tab = m.tab;
+    a.cu1 = c->cu[0]; a.cu3 = c->cu[2]; a.kx = c->d_kx; a.ps = g.ps;
+    a.ny = g.ny; a.nz = g.nz; a.jlo = jlo; a.jhi = g.ny; a.force = force ? 1 : 0;
+    dgpu::launch_les_prod(c->stream, g, c->ipx64, c->d_pairtw, c->ld, a);
+    if (int rc = check_launch(c, "les_prod")) return rc;
+    if (!force) {
+        // APPLY_BC_VEL_PHYS_MPI (for/channel.f:309-311) on the state and on the
+        // physical fields the solves take
+        dgpu::launch_les_bc_phys(c->stream, g, c->cu[0], c->cu[1], c->cu[2], b, c->d_dy, c->d_dyf);
+        if (int rc = check_launch(c, "les_bc_phys")) return rc;
+        dgpu::launch_les_bc_put(c->stream, g, pair_buf(c, 0), pair_buf(c, 1), m.bc);
+        if (int rc = check_launch(c, "les_bc_put")) return rc;
     }
-    return DGPU_OK;
+    dgpu::launch_zfwd_nl_ip<double, double>(c->stream, g, c->ipz, c->d_iptw + c->ipx.twn, c->d_wt, c->zfs, c->ld,
+                                            c->d_nlptr, c->d_kz, jlo, g.ny, force ? 3 : nin);
+    return check_launch(c, "zfwd_nl(les)");
 }
 
 int32_t dgpu_les_chan(dgpu_ctx *c, double *nu_t)
@@ -1194,9 +1304,17 @@ int32_t dgpu_les_chan(dgpu_ctx *c, double *nu_t)
     if (int rc = to_master(c)) return rc;
     c->master_dirty = true;
     if (int rc = ensure_les(c)) return rc;
-    if (int rc = les_model(c, c->cf[0], c->cf[1], c->cf[2], false)) return rc;
-    if (nu_t) HIPCHK(c, hipMemcpyAsync(nu_t, les_buf(c, 13), les_n(c) * sizeof(double), hipMemcpyDeviceToHost,
-                                       c->stream));
+    if (nu_t)
+        if (int rc = ensure_fort(c)) return rc;
+    if (int rc = les_terms(c, 2, true)) return rc;
+    for (int q = 0; q < 3; ++q) dgpu::launch_les_addcf(c->stream, c->g, c->cf[q], c->nl[q]);
+    if (int rc = check_launch(c, "les_addcf")) return rc;
+    if (nu_t) {
+        const size_t n = (size_t)(c->g.nx + 2) * (c->g.nz + 2) * (c->g.ny + 2);
+        dgpu::launch_les_nut_out(c->stream, c->g, les_mem(c).nut, c->d_perm, c->d_perm + c->g.nz, c->d_fort);
+        if (int rc = check_launch(c, "les_nut_out")) return rc;
+        HIPCHK(c, hipMemcpyAsync(nu_t, c->d_fort, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    }
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return DGPU_OK;
 }
@@ -1206,16 +1324,11 @@ int32_t dgpu_tke_les(dgpu_ctx *c, double *eps_sgs)
     if (!c || !eps_sgs) return DGPU_E_ARG;
     if (!c->les) return fail(c, DGPU_E_ARG, "tkebudget_chan_les needs LES on");
     if (int rc = to_master(c)) return rc;
-    const dgpu::Geo &g = c->g;
-    const int NY = g.ny;
-    double *U[3] = {les_buf(c, 0), les_buf(c, 1), les_buf(c, 2)};
-    for (int q = 0; q < 3; ++q) {
-        dgpu::launch_les_pack(c->stream, g, c->cu[q], U[q], c->d_kx, c->d_kz, 0, 0, NY + 1);
-        if (int rc = check_launch(c, "les_pack")) return rc;
-        if (int rc = fort_to_physical(c, U[q], 0, NY + 1)) return rc;
-    }
-    double *out = les_buf(c, 6);
-    dgpu::launch_les_eps(c->stream, g, U[0], U[1], U[2], les_buf(c, 13), c->d_dy, c->d_dyf, out);
+    const int NY = c->g.ny;
+    if (int rc = pairs_z(c, false)) return rc;
+    if (int rc = pairs_x(c, pairs_of_fields(c), c->d_wt, 0)) return rc;
+    double *out = reinterpret_cast<double *>(pair_buf(c, 2));
+    dgpu::launch_les_eps(c->stream, c->g, pair_buf(c, 0), pair_buf(c, 1), les_mem(c).nut, c->d_dy, c->d_dyf, out);
     if (int rc = check_launch(c, "les_eps")) return rc;
     HIPCHK(c, hipMemcpyAsync(eps_sgs, out, sizeof(double) * NY, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -1626,81 +1739,40 @@ static int rk_enqueue(dgpu_ctx *c, int rk_step, double time, double temp1, doubl
     return DGPU_OK;
 }
 
-// RK_CHAN_1 with LES = .TRUE. (for/channel.f:62-1073): the explicit terms of
-// the fused path (with the SGS force when the model is called) give the
-// right-hand sides; the Crank-Nicolson solves run in physical space with the
-// eddy viscosity, then REM_DIV_CHAN and the CP update as in the DNS path.
+// RK_CHAN_1 with LES = .TRUE. (for/channel.f:62-1073): the explicit terms (with
+// the model's when it is called) give the right-hand sides; the
+// Crank-Nicolson solves run in physical space with the eddy viscosity, then
+// REM_DIV_CHAN and the CP update as in the DNS path.
 static int les_substep(dgpu_ctx *c, int rk_step, double time, double temp1, double temp3, double temp4,
                        double temp5)
 {
     const dgpu::Geo &g = c->g;
-    const int NY = g.ny;
-    const int nin = 3 + g.nth;
+    const int NY = g.ny, nin = 3 + g.nth;
     const bool courant = rk_step == 3 && c->courant_state == 1;
     const double temp2 = temp4 / 2.0;  // TEMP2 = H_BAR(RK_STEP) / 2
-    double *U[3] = {les_buf(c, 0), les_buf(c, 1), les_buf(c, 2)};
-    double *Rb[3] = {les_buf(c, 3), les_buf(c, 4), les_buf(c, 5)};
-    double *bm = les_buf(c, 6), *gw = les_buf(c, 7), *cs = les_buf(c, 8), *thp = les_buf(c, 9),
-           *rthp = les_buf(c, 10), *nut = les_buf(c, 13);
-    cx<double> *sgs[4];
-    for (int q = 0; q < 4; ++q) sgs[q] = reinterpret_cast<cx<double> *>(les_buf(c, 14 + q));
-    cx<double> *pre = reinterpret_cast<cx<double> *>(les_buf(c, 18));
-    const size_t fsb = sizeof(cx<double>) * (size_t)c->fs;
-    if (c->les_model) {
-        // the model writes the whole of sgs[0..2]; the scalar's part is
-        // accumulated over its own rows
-        if (g.nth) HIPCHK(c, hipMemsetAsync(sgs[3], 0, fsb, c->stream));
-        for (int r = 0; r < 4; ++r)
-            HIPCHK(c, hipMemcpyAsync(pre + (size_t)r * g.ps, c->cu[r < 2 ? 0 : 2] + (size_t)(r % 2 ? NY : 1) * g.ps,
-                                     sizeof(cx<double>) * g.ps, hipMemcpyDeviceToDevice, c->stream));
-        if (int rc = les_model(c, sgs[0], sgs[1], sgs[2], true)) return rc;
-        // APPLY_BC_VEL_PHYS_MPI (for/channel.f:309-311)
-        dgpu::LesBc b;
-        b.u_lo = c->p.u_bc_ymin; b.u_hi = c->p.u_bc_ymax; b.w_lo = c->p.w_bc_ymin; b.w_hi = c->p.w_bc_ymax;
-        b.v_lo = c->p.v_bc_ymin; b.v_hi = c->p.v_bc_ymax;
-        b.u_lo_c = c->p.u_bc_ymin_c1; b.u_hi_c = c->p.u_bc_ymax_c1; b.w_lo_c = c->p.w_bc_ymin_c1;
-        b.w_hi_c = c->p.w_bc_ymax_c1; b.v_lo_c = c->p.v_bc_ymin_c1; b.v_hi_c = c->p.v_bc_ymax_c1;
-        dgpu::launch_les_bc_phys(c->stream, g, c->cu[0], c->cu[1], c->cu[2], b, c->d_dy, c->d_dyf);
-        if (int rc = check_launch(c, "les_bc_phys")) return rc;
-        // and on the model's physical U1, U3 (planes 0, 2), as the reference
-        // applies it to the arrays les_chan left in physical space
-        dgpu::launch_les_bc_phys_planes(c->stream, g, U[0], U[2], b, c->d_dy);
-        if (int rc = check_launch(c, "les_bc_phys_planes")) return rc;
-        // KAPPA_T = NU_T and the scalar's horizontal eddy diffusion, explicit
-        // (for/channel.f:313-375)
-        for (int nth = 0; nth < g.nth; ++nth)
-            for (int dir = 1; dir <= 2; ++dir) {
-                dgpu::launch_les_pack(c->stream, g, c->cth[nth], cs, c->d_kx, c->d_kz, dir, 1, NY + 1);
-                if (int rc = check_launch(c, "les_pack")) return rc;
-                if (int rc = fort_to_physical(c, cs, 0, NY + 1)) return rc;
-                dgpu::launch_les_mul(c->stream, g, cs, nut, 1, NY + 1);
-                if (int rc = check_launch(c, "les_mul")) return rc;
-                if (int rc = fort_to_fourier(c, cs, 0, NY + 1)) return rc;
-                dgpu::launch_les_acc(c->stream, g, sgs[3], cs, c->d_kx, c->d_kz, dir, c->jstart_th[nth],
-                                     c->jend_th[nth]);
-                if (int rc = check_launch(c, "les_acc")) return rc;
-            }
-    }
-    // nonlinear terms (the fused transforms of the DNS path, FP64)
+    const LesMem m = les_mem(c);
+    const cx<double> *twx = c->d_iptw, *twz = c->d_iptw + c->ipx.twn;
     int jlo = 2;
     for (int q = 0; q < g.nth; ++q) jlo = std::min(jlo, c->jstart_th[q]);
-    const long zps = (long)g.nz * c->ld;
-    const cx<double> *twx = c->d_iptw, *twz = c->d_iptw + c->ipx.twn;
-    dgpu::launch_zinv_ip<double, double>(c->stream, g, c->ipz, twz, c->cu[0], c->fs, g.ps, c->d_zt, c->zfs, zps,
-                                         c->ld, 0, g.ny + 2, nin);
-    if (int rc = check_launch(c, "zinv")) return rc;
-    dgpu::launch_xfused_ip<double>(c->stream, g, c->ipx, twx, c->ld, c->d_zt, c->zfs, c->d_wt, c->zfs, c->d_dy,
-                                   c->d_dyf, c->d_kx, jlo, g.ny, c->xchunk);
-    if (int rc = check_launch(c, "xfused")) return rc;
-    dgpu::launch_zfwd_nl_ip<double, double>(c->stream, g, c->ipz, twz, c->d_wt, c->zfs, c->ld, c->d_nlptr, c->d_kz,
-                                            jlo, g.ny, nin);
-    if (int rc = check_launch(c, "zfwd_nl")) return rc;
-    // the SGS force joins the nonlinear terms (slots: x, y, z momentum, scalar)
-    if (c->les_model)
-        for (int q = 0; q < nin; ++q) {
-            dgpu::launch_les_add(c->stream, c->nl[q], sgs[q], c->fs);
-            if (int rc = check_launch(c, "les_add")) return rc;
-        }
+    if (c->les_model) {
+        for (int r = 0; r < 4; ++r)
+            HIPCHK(c, hipMemcpyAsync(m.pre + (size_t)r * g.ps, c->cu[r < 2 ? 0 : 2] + (size_t)(r % 2 ? NY : 1) * g.ps,
+                                     sizeof(cx<double>) * g.ps, hipMemcpyDeviceToDevice, c->stream));
+        if (int rc = les_terms(c, jlo, false)) return rc;
+    } else {
+        // the fused products of the DNS path; the physical fields for the solves
+        // come from the same z-backward rows
+        dgpu::launch_zinv_ip<double, double>(c->stream, g, c->ipz, twz, c->cu[0], c->fs, g.ps, c->d_zt, c->zfs,
+                                             (long)g.nz * c->ld, c->ld, 0, NY + 2, nin);
+        if (int rc = check_launch(c, "zinv")) return rc;
+        dgpu::launch_xfused_ip<double>(c->stream, g, c->ipx, twx, c->ld, c->d_zt, c->zfs, c->d_wt, c->zfs, c->d_dy,
+                                       c->d_dyf, c->d_kx, jlo, NY, c->xchunk);
+        if (int rc = check_launch(c, "xfused")) return rc;
+        dgpu::launch_zfwd_nl_ip<double, double>(c->stream, g, c->ipz, twz, c->d_wt, c->zfs, c->ld, c->d_nlptr,
+                                                c->d_kz, jlo, NY, nin);
+        if (int rc = check_launch(c, "zfwd_nl")) return rc;
+        if (int rc = pairs_x(c, pairs_of_fields(c), c->d_zt, 0)) return rc;
+    }
     // new CF and the right-hand sides (sweep A of the column kernel)
     dgpu::CnArgs A;
     make_cn_args(c, rk_step, time, temp3, temp4, temp5, A);
@@ -1715,71 +1787,60 @@ static int les_substep(dgpu_ctx *c, int rk_step, double time, double temp1, doub
         f.drhodx = g.nth ? c->p.drhodx[0] : 0.0; f.drhodz = g.nth ? c->p.drhodz[0] : 0.0;
         f.jstart = c->jstart; f.jend = c->jend;
         f.jstart_th = g.nth ? c->jstart_th[0] : 1; f.jend_th = g.nth ? c->jend_th[0] : 0;
-        dgpu::launch_les_cf_rows(c->stream, g, pre, c->cu[0], c->cu[2], c->cf[0], c->cf[2],
+        dgpu::launch_les_cf_rows(c->stream, g, m.pre, c->cu[0], c->cu[2], c->cf[0], c->cf[2],
                                  g.nth ? c->cfth[0] : nullptr, c->d_kx2, c->d_kz2, f);
         if (int rc = check_launch(c, "les_cf_rows")) return rc;
     }
-    // physical right-hand sides and fields
-    for (int q = 0; q < 3; ++q) {
-        dgpu::launch_les_pack(c->stream, g, c->nl[q], Rb[q], c->d_kx, c->d_kz, 0, 0, NY + 1);
-        if (int rc = check_launch(c, "les_pack")) return rc;
-        if (int rc = fort_to_physical(c, Rb[q], 0, NY + 1)) return rc;
-        if (c->les_model && q != 1) continue;  // the model's U1, U3 with their BCs
-        dgpu::launch_les_pack(c->stream, g, c->cu[q], U[q], c->d_kx, c->d_kz, 0, 0, NY + 1);
-        if (int rc = check_launch(c, "les_pack")) return rc;
-        if (int rc = fort_to_physical(c, U[q], 0, NY + 1)) return rc;
-    }
-    if (g.nth) {
-        dgpu::launch_les_pack(c->stream, g, c->nl[3], rthp, c->d_kx, c->d_kz, 0, 0, NY + 1);
-        dgpu::launch_les_pack(c->stream, g, c->cth[0], thp, c->d_kx, c->d_kz, 0, 0, NY + 1);
-        if (int rc = check_launch(c, "les_pack")) return rc;
-        if (int rc = fort_to_physical(c, rthp, 0, NY + 1)) return rc;
-        if (int rc = fort_to_physical(c, thp, 0, NY + 1)) return rc;
-    }
+    // physical right-hand sides: pairs 6 (R1, R2) and 7 (R3, RTH)
+    dgpu::ZSrc z{};
+    z.n = nin;
+    for (int q = 0; q < nin; ++q) z.p[q] = c->nl[q];
+    dgpu::launch_zinv_src(c->stream, g, c->ipz, twz, z, c->d_zt, c->zfs, c->ld, c->d_kz, 0, NY + 2);
+    if (int rc = check_launch(c, "zinv(rhs)")) return rc;
+    if (int rc = pairs_x(c, pairs_of_fields(c), c->d_zt, 6)) return rc;
     // implicit solves: TH, U2, U1, U3 (for/channel.f:762-1029), independent,
     // in one launch, each right-hand side with its explicit eddy-viscosity
-    // half (for/channel.f:628-659, 748-760) added on the fly; scratch planes: 6, 7 (work planes of the model), 8, 11,
-    // 12, and 14-16 (the SGS force, already added to the nonlinear terms)
+    // half (for/channel.f:628-659, 748-760) added on the fly
     const double nuv = c->p.nu_v_scale;
-    double *scratch[8] = {bm, gw, les_buf(c, 8), les_buf(c, 11), les_buf(c, 12), les_buf(c, 14), les_buf(c, 15),
-                          les_buf(c, 16)};
     dgpu::LesCnSet set{};
-    auto add = [&](int sys, int jl, int jh, int lo, int hi, double clo, double chi, double cmol, const double *rhs,
-                   double *out) {
-        dgpu::LesCn &a = set.a[set.n];
-        a.sys = sys; a.ny = NY; a.jlo = jl; a.jhi = jh; a.clo = jl - 1; a.chi = jh + 1;
-        if (sys == dgpu::LES_SYS_U2) { a.clo = 1; a.chi = NY + 1; }
+    auto sys = [&](dgpu::LesCn &a, int kind, int jl, int jh, int lo, int hi, double clo, double chi, double cmol) {
+        a.sys = kind; a.ny = NY; a.jlo = jl; a.jhi = jh; a.clo = jl - 1; a.chi = jh + 1;
+        if (kind == dgpu::LES_SYS_U2) { a.clo = 1; a.chi = NY + 1; }
         a.lo = lo; a.hi = hi; a.cmol = cmol; a.temp2 = temp2; a.clo_c = clo; a.chi_c = chi;
-        set.rhs[set.n] = rhs;
-        set.out[set.n] = out;
-        set.bm[set.n] = scratch[2 * set.n];
-        set.gw[set.n] = scratch[2 * set.n + 1];
-        ++set.n;
     };
+    sys(set.a[0][0], dgpu::LES_SYS_U13, c->jstart, c->jend, c->p.u_bc_ymin, c->p.u_bc_ymax, c->p.u_bc_ymin_c1,
+        c->p.u_bc_ymax_c1, temp1 * nuv);
+    sys(set.a[0][1], dgpu::LES_SYS_U2, 2, NY, c->p.v_bc_ymin, c->p.v_bc_ymax, c->p.v_bc_ymin_c1, c->p.v_bc_ymax_c1,
+        temp1 * nuv);
+    sys(set.a[1][0], dgpu::LES_SYS_U13, c->jstart, c->jend, c->p.w_bc_ymin, c->p.w_bc_ymax, c->p.w_bc_ymin_c1,
+        c->p.w_bc_ymax_c1, temp1 * nuv);
     if (g.nth)
-        add(dgpu::LES_SYS_TH, c->jstart_th[0], c->jend_th[0], c->p.th_bc_ymin[0], c->p.th_bc_ymax[0],
-            c->p.th_bc_ymin_c1[0], c->p.th_bc_ymax_c1[0], temp1 / c->p.pr[0] * nuv, rthp, thp);
-    add(dgpu::LES_SYS_U2, 2, NY, c->p.v_bc_ymin, c->p.v_bc_ymax, c->p.v_bc_ymin_c1, c->p.v_bc_ymax_c1, temp1 * nuv,
-        Rb[1], U[1]);
-    add(dgpu::LES_SYS_U13, c->jstart, c->jend, c->p.u_bc_ymin, c->p.u_bc_ymax, c->p.u_bc_ymin_c1, c->p.u_bc_ymax_c1,
-        temp1 * nuv, Rb[0], U[0]);
-    add(dgpu::LES_SYS_U13, c->jstart, c->jend, c->p.w_bc_ymin, c->p.w_bc_ymax, c->p.w_bc_ymin_c1, c->p.w_bc_ymax_c1,
-        temp1 * nuv, Rb[2], U[2]);
-    dgpu::launch_les_cn(c->stream, g, set, nut, c->d_dy, c->d_dyf);
+        sys(set.a[1][1], dgpu::LES_SYS_TH, c->jstart_th[0], c->jend_th[0], c->p.th_bc_ymin[0], c->p.th_bc_ymax[0],
+            c->p.th_bc_ymin_c1[0], c->p.th_bc_ymax_c1[0], temp1 / c->p.pr[0] * nuv);
+    else
+        set.a[1][1].sys = -1;
+    for (int q = 0; q < 2; ++q) {
+        set.rhs[q] = pair_buf(c, 6 + q);
+        set.out[q] = pair_buf(c, q);
+        set.cw[q] = pair_buf(c, 2 + 2 * q);
+        set.gw[q] = pair_buf(c, 3 + 2 * q);
+    }
+    dgpu::launch_les_cn(c->stream, g, set, m.nut, c->d_dy, c->d_dyf);
     if (int rc = check_launch(c, "les_cn")) return rc;
     // COURANT on the physical velocity after the solves (for/channel.f:1037-1040)
     if (courant) {
-        dgpu::launch_les_vmax(c->stream, g, U[0], U[1], U[2], c->d_vmax);
+        dgpu::launch_les_vmax(c->stream, g, pair_buf(c, 0), pair_buf(c, 1), c->d_vmax);
         if (int rc = check_launch(c, "les_vmax")) return rc;
         c->courant_state = 2;
     }
     // back to Fourier space (for/channel.f:1043-1050)
-    for (int q = 0; q < 3 + g.nth; ++q) {
-        double *f = q < 3 ? U[q] : thp;
-        if (int rc = fort_to_fourier(c, f, 0, NY + 1)) return rc;
-        dgpu::launch_unpack_fortran(c->stream, g, f, q < 3 ? c->cu[q] : c->cth[0], 0, NY + 2);
-        if (int rc = check_launch(c, "unpack")) return rc;
-    }
+    dgpu::PairDst ps{{pair_buf(c, 0), pair_buf(c, 1)}};
+    const dgpu::PairOut po{{0, 2}, {1, g.nth ? 3 : -1}, 2};
+    dgpu::launch_pairs_fwd(c->stream, g, c->ipx64, c->d_pairtw, c->ld, ps, c->d_wt, c->zfs, po, 0, NY + 2);
+    if (int rc = check_launch(c, "x forward(pairs)")) return rc;
+    dgpu::ZDst zd{{c->cu[0], c->cu[1], c->cu[2], g.nth ? c->cth[0] : nullptr}, nin};
+    dgpu::launch_zfwd_dst(c->stream, g, c->ipz, twz, c->d_wt, c->zfs, c->ld, zd, 0, NY + 2);
+    if (int rc = check_launch(c, "zfwd(pairs)")) return rc;
     dgpu::RdArgs R;
     fill_rdargs(c, R, 1, temp4);
     dgpu::launch_remdiv<double, double>(c->stream, R, P);

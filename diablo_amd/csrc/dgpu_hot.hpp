@@ -62,6 +62,16 @@ __device__ __forceinline__ const IpLen &plan_ref(const IpLen &rt)
     default: break;                                                \
     }
 
+// the x plans of FP64: at most 12 values per thread
+#define DGPU_DISPATCH_XE64(E_, CALL)                               \
+    switch (E_) {                                                  \
+    case 4: { constexpr int EE = 4; CALL; } break;                 \
+    case 6: { constexpr int EE = 6; CALL; } break;                 \
+    case 8: { constexpr int EE = 8; CALL; } break;                 \
+    case 12: { constexpr int EE = 12; CALL; } break;               \
+    default: break;                                                \
+    }
+
 static inline int z_lw(int t)
 {
     int lw = 0;
@@ -80,6 +90,8 @@ using XPids = std::conditional_t<sizeof(T) == 4, PidList<2, 3, 5, 13, 14, 17>, P
 // the single-context x kernel: the 384 and 256 plans
 template <typename T>
 using XPidsSingle = std::conditional_t<sizeof(T) == 4, PidList<13, 17>, PidList<1, 12>>;
+// the FP64 pair transforms (dgpu_pairs.hip) and the LES products
+using XPids64 = PidList<1, 12>;
 template <typename T>
 using ZPids = PidList<6, 8, 9, 10, 15, 16>;
 
@@ -93,7 +105,50 @@ static bool with_pid(int pid, PidList<P...>, F &&fn)
     return done;
 }
 
+// The last forward (DIT) stage of an x row holding the transform of a + i b
+// (a plan with R_0 = E/2): thread th takes groups th and L0 - th (0 and L0/2
+// for th = 0), so it holds Z(k) and Z(NX - k) of its frequencies, and calls
+// emit(k, Z(k), Z(NX - k)) for the kept ones.
+template <typename T, int E, class F>
+__device__ __forceinline__ void x_split(const IpLen &fx, const cx<T> *row, const cx<T> *tw, int th, int mk, F &&emit)
+{
+    constexpr int R0 = E / 2;
+    const int L0 = fx.span[0], TT = fx.t;
+    const int ga = th, gb = th == 0 ? TT : L0 - th;
+    cx<T> va[R0], vb[R0];
+#pragma unroll
+    for (int q = 0; q < R0; ++q) {
+        va[q] = row[ip_swz(fx, ga + q * L0)];
+        vb[q] = row[ip_swz(fx, gb + q * L0)];
+    }
+    ip_group<T, R0, -1, false>(va, tw + fx.twoff[0], ga);
+    ip_group<T, R0, -1, false>(vb, tw + fx.twoff[0], gb);
+#pragma unroll
+    for (int q = 0; q < R0; ++q) {
+        const int ka = ga + q * L0;
+        if (ka < mk) emit(ka, va[q], ga == 0 ? va[(R0 - q) % R0] : vb[R0 - 1 - q]);
+        const int kb = gb + q * L0;
+        if (kb < mk) emit(kb, vb[q], th == 0 ? vb[R0 - 1 - q] : va[R0 - 1 - q]);
+    }
+}
+
 // Id of the compile-time plan equal to f, or 0 (dgpu_hot_z.hip).
 int const_plan_id(const IpLen &f);
+
+// Planes per block of a sweeping kernel (dgpu_hot_x.hip).
+int sweep_rule(long rows, int planes, long slots);
+
+// Blocks of a kernel that the whole device holds at once.
+template <class K>
+static long kernel_slots(K kernel, int threads, size_t lds)
+{
+    int per = 0, dev = 0, cus = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, lds) != hipSuccess || per < 1) per = 1;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
+        cus = 256;
+    (void)hipGetLastError();
+    return (long)per * cus;
+}
 
 }  // namespace dgpu

@@ -470,7 +470,7 @@ static int xfused_zrows(const IpLen &fx, int nz, int mk)
 // one RK3 step at 64x65x64 FP64 1502 -> 219 us (2 planes), 96x81x108 1984 ->
 // 520, 192x129x192 2819 -> 1840; at 384x257x384 the rule gives the 64 (FP64)
 // and 32 (FP32) planes measured best there.
-static int xfused_rule(long rows, int planes, long slots)
+int sweep_rule(long rows, int planes, long slots)
 {
     int best = planes;
     double best_cost = 1e300;
@@ -486,19 +486,6 @@ static int xfused_rule(long rows, int planes, long slots)
         }
     }
     return best;
-}
-
-// Blocks of a kernel that the whole device holds at once.
-template <class K>
-static long xfused_slots(K kernel, int threads, size_t lds)
-{
-    int per = 0, dev = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, lds) != hipSuccess || per < 1) per = 1;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
-        cus = 256;
-    (void)hipGetLastError();
-    return (long)per * cus;
 }
 
 // pick: nothing is launched, *pick receives the rule's planes per block
@@ -519,8 +506,8 @@ static void xfused_ip_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T
         attr = true;
     }
     if (pick) {
-        *pick = xfused_rule((g.nz + zr - 1) / zr, jhi - jlo + 1,
-                            xfused_slots(&k_xfused_ip<T, E, NTH, PID>, threads, lds));
+        *pick = sweep_rule((g.nz + zr - 1) / zr, jhi - jlo + 1,
+                            kernel_slots(&k_xfused_ip<T, E, NTH, PID>, threads, lds));
         return;
     }
     const int nchunks = (jhi - jlo + 1 + chunk - 1) / chunk;

@@ -25,11 +25,13 @@ namespace dgpu {
 // kept slots straight from the state, the last stage writes Zt rows.
 // grid (column chunks, planes, fields), block W*T, LDS W*NZ values.
 // -------------------------------------------------------------------------
-template <typename T, int E, typename TIN, bool CP>
+// kzv (DZ only): null, or the input is multiplied by i KZ.
+template <typename T, int E, typename TIN, bool CP, bool DZ = false>
 __device__ __forceinline__ void zinv_body(const IpLen &fz, const cx<T> *__restrict__ tw,
                                           const cx<TIN> *__restrict__ in, long in_fs, long in_ps, int mk,
                                           cx<T> *__restrict__ out, long out_fs, long out_ps, int ld, int j0, int nkz,
-                                          int tnkz, int lw, int bx, int by, int bz)
+                                          int tnkz, int lw, int bx, int by, int bz,
+                                          const double *__restrict__ kzv = nullptr)
 {
     extern __shared__ unsigned char smem_raw[];
     cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw);
@@ -51,7 +53,13 @@ __device__ __forceinline__ void zinv_body(const IpLen &fz, const cx<T> *__restri
                 // unconditional load at a valid index, then select: keeps it
                 // one 16-byte access
                 const int s = slot_of_freq(f, nz, nkz, tnkz);
-                const cx<TIN> v = src[(long)max(s, 0) * mk + (col ? i : mk - 1)];
+                cx<TIN> v = src[(long)max(s, 0) * mk + (col ? i : mk - 1)];
+                if constexpr (DZ) {
+                    if (kzv) {
+                        const TIN kz = TIN(kzv[max(s, 0)]);
+                        v = make_cx<TIN>(-kz * v.im, kz * v.re);
+                    }
+                }
                 return (col && s >= 0) ? cvt_<T>(v) : make_cx<T>(0, 0);
             },
             [&](int, int pos, cx<T> v) { x[ip_cswz(fz, pos) * W] = v; });
@@ -87,6 +95,64 @@ __global__ void __launch_bounds__(256) k_zinv_ip(IpLen fz, const cx<T> *__restri
     if (plane >= nplanes) return;
     zinv_body<T, E, TIN, PID != 0>(plan_ref<PID>(fz), tw, in, in_fs, in_ps, mk, out, out_fs, out_ps, ld, j0, nkz,
                                    tnkz, lw, chunk, plane, blockIdx.z);
+}
+
+// The same for fields anywhere in memory, each plain or differentiated in z
+// (dgpu_pairs.hip's inputs).
+template <int E, int PID>
+__global__ void __launch_bounds__(256) k_zinv_src(IpLen fz, const cx<double> *__restrict__ tw, ZSrc src, long in_ps,
+                                                   int mk, cx<double> *__restrict__ out, long out_fs, long out_ps,
+                                                   int ld, int j0, int nkz, int tnkz, int lw, int nchunks,
+                                                   int nplanes, const double *__restrict__ kzv)
+{
+    int chunk, plane;
+    if (!plane_chunk(blockIdx.x, nchunks, nplanes, chunk, plane)) return;
+    const int f = blockIdx.z;
+    zinv_body<double, E, double, PID != 0, true>(plan_ref<PID>(fz), tw, src.p[f], 0, in_ps, mk, out + f * out_fs, 0,
+                                                 out_ps, ld, j0, nkz, tnkz, lw, chunk, plane, 0,
+                                                 src.dz[f] ? kzv : nullptr);
+}
+
+// z forward (DIT) of one Wt field per output, no derivative: the kept slots
+// of dst.p[o], 1/NZ applied.
+template <int E, int PID>
+__global__ void __launch_bounds__(256) k_zfwd_dst(IpLen frt, const cx<double> *__restrict__ tw,
+                                                   const cx<double> *__restrict__ wt, long wt_fs, long wt_ps, int ld,
+                                                   int mk, ZDst dst, long ps, int j0, int nkz, int tnkz, int lw,
+                                                   int nchunks, int nplanes)
+{
+    extern __shared__ unsigned char smem_raw[];
+    cx<double> *lds = reinterpret_cast<cx<double> *>(smem_raw);
+    const IpLen &fz = plan_ref<PID>(frt);
+    int chunk, plane;
+    if (!plane_chunk(blockIdx.x, nchunks, nplanes, chunk, plane)) return;
+    const int W = 1 << lw, tid = threadIdx.x, b = tid & (W - 1), th = tid >> lw;
+    const int i = chunk * W + b, j = j0 + plane, o = blockIdx.z, nz = fz.n, S = fz.nstages;
+    const bool col = i < mk;
+    const cx<double> *src = wt + o * wt_fs + (long)j * wt_ps + (col ? i : mk - 1);
+    cx<double> *x = lds + b;
+    with_radix<E>(fz.radix[S - 1], [&](auto rc) {
+        constexpr int R = decltype(rc)::value;
+        ip_stage<double, E, R, -1, false>(
+            fz, S - 1, tw, th, [&](int, int pos) { return src[(long)pos * ld]; },
+            [&](int, int pos, cx<double> v) { x[ip_cswz(fz, pos) * W] = v; });
+    });
+    __syncthreads();
+    stage_loop<PID != 0>(1, S - 1, [&](int s) {
+        ip_stage_mem<double, E, -1, false>(x, W, fz, S - 1 - s, tw, th);
+        __syncthreads();
+    });
+    const double inv_nz = 1.0 / nz;
+    cx<double> *out = dst.p[o] + (long)j * ps + i;
+    with_radix<E>(fz.radix[0], [&](auto rc) {
+        constexpr int R = decltype(rc)::value;
+        ip_stage<double, E, R, -1, false>(
+            fz, 0, tw, th, [&](int, int pos) { return x[ip_cswz(fz, pos) * W]; },
+            [&](int, int f, cx<double> v) {
+                const int s = slot_of_freq(f, nz, nkz, tnkz);
+                if (col && s >= 0) out[(long)s * mk] = scale(v, inv_nz);
+            });
+    });
 }
 
 // Members of one transform-length group: grid.x over (column chunks, planes
@@ -297,6 +363,48 @@ void launch_zfwd_nl_ip(hipStream_t s, const Geo &g, const IpLen &fz, const cx<T>
         }))
         return;
     DGPU_DISPATCH_IPE(fz.e, (zfwd_nl_ip_e<T, EE, TOUT, 0>(s, g, fz, tw, wt, wt_fs, ld, nl, kz, jlo, jhi, nout)));
+}
+
+template <int E, int PID>
+static void zinv_src_e(hipStream_t s, const Geo &g, const IpLen &fz, const cx<double> *tw, const ZSrc &src,
+                       cx<double> *out, long out_fs, int ld, const double *kz, int j0, int nplanes)
+{
+    const int lw = z_lw(fz.t), W = 1 << lw, nchunks = (g.mk + W - 1) / W;
+    hipLaunchKernelGGL((k_zinv_src<E, PID>), dim3((unsigned)(8 * nchunks * ((nplanes + 7) / 8)), 1, src.n),
+                       dim3(W * fz.t), sizeof(cx<double>) * W * fz.n, s, fz, tw, src, g.ps, g.mk, out, out_fs,
+                       (long)g.nz * ld, ld, j0, g.nkz, g.tnkz, lw, nchunks, nplanes, kz);
+}
+
+void launch_zinv_src(hipStream_t s, const Geo &g, const IpLen &fz, const cx<double> *tw, const ZSrc &src,
+                     cx<double> *out, long out_fs, int ld, const double *kz, int j0, int nplanes)
+{
+    if (with_pid(const_plan_id(fz), ZPids<double>{}, [&](auto pc) {
+            constexpr int P = decltype(pc)::value;
+            zinv_src_e<kConstPlanSpecs[P].e, P>(s, g, fz, tw, src, out, out_fs, ld, kz, j0, nplanes);
+        }))
+        return;
+    DGPU_DISPATCH_IPE(fz.e, (zinv_src_e<EE, 0>(s, g, fz, tw, src, out, out_fs, ld, kz, j0, nplanes)));
+}
+
+template <int E, int PID>
+static void zfwd_dst_e(hipStream_t s, const Geo &g, const IpLen &fz, const cx<double> *tw, const cx<double> *wt,
+                       long wt_fs, int ld, const ZDst &dst, int j0, int nplanes)
+{
+    const int lw = z_lw(fz.t), W = 1 << lw, nchunks = (g.mk + W - 1) / W;
+    hipLaunchKernelGGL((k_zfwd_dst<E, PID>), dim3((unsigned)(8 * nchunks * ((nplanes + 7) / 8)), 1, dst.n),
+                       dim3(W * fz.t), sizeof(cx<double>) * W * fz.n, s, fz, tw, wt, wt_fs, (long)g.nz * ld, ld, g.mk,
+                       dst, g.ps, j0, g.nkz, g.tnkz, lw, nchunks, nplanes);
+}
+
+void launch_zfwd_dst(hipStream_t s, const Geo &g, const IpLen &fz, const cx<double> *tw, const cx<double> *wt,
+                     long wt_fs, int ld, const ZDst &dst, int j0, int nplanes)
+{
+    if (with_pid(const_plan_id(fz), ZPids<double>{}, [&](auto pc) {
+            constexpr int P = decltype(pc)::value;
+            zfwd_dst_e<kConstPlanSpecs[P].e, P>(s, g, fz, tw, wt, wt_fs, ld, dst, j0, nplanes);
+        }))
+        return;
+    DGPU_DISPATCH_IPE(fz.e, (zfwd_dst_e<EE, 0>(s, g, fz, tw, wt, wt_fs, ld, dst, j0, nplanes)));
 }
 
 // ---- batched (ensemble) launchers ----

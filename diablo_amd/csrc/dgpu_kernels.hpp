@@ -258,26 +258,63 @@ void launch_side_scatter(hipStream_t s, const cx<TS> *side, long side_fs, cx<TF>
 void launch_apply_bc_vel(hipStream_t s, const Geo &g, cx<double> *cu1, cx<double> *cu2, cx<double> *cu3,
                          const int *codes, const double *c1, const double *dy, const double *dyf);
 
-// les_chan's constant Smagorinsky model (dgpu_les.hip).  Planes are
-// Fortran-layout (0:NX+1, 0:NZ+1, 0:NY+1) doubles, passed by value.
-struct LesPtrs {
-    double *p[8];
+// ---- pair planes (dgpu_pairs.hip): FP64 physical fields two by two ----
+// z backward of the kept modes of n fields, each plain or times i KZ
+struct ZSrc {
+    const cx<double> *p[8];
+    int dz[8];
+    int n;
 };
+// z forward of n consecutive Wt fields into the kept modes of p[o]
+struct ZDst {
+    cx<double> *p[4];
+    int n;
+};
+// real rows A = Z_a0 + i KX Z_a1 and B likewise of each pair (-1: none)
+struct PairSrc {
+    int a0[6], a1[6], b0[6], b1[6];
+    int n;
+};
+struct PairDst {
+    cx<double> *p[6];
+};
+// Wt fields of each pair's two rows (-1: not written)
+struct PairOut {
+    int a[6], b[6];
+    int n;
+};
+void launch_zinv_src(hipStream_t s, const Geo &g, const IpLen &fz, const cx<double> *tw, const ZSrc &src,
+                     cx<double> *out, long out_fs, int ld, const double *kz, int j0, int nplanes);
+void launch_zfwd_dst(hipStream_t s, const Geo &g, const IpLen &fz, const cx<double> *tw, const cx<double> *wt,
+                     long wt_fs, int ld, const ZDst &dst, int j0, int nplanes);
+void launch_pairs_inv(hipStream_t s, const Geo &g, const IpLen &fx, const cx<double> *tw, int ld,
+                      const cx<double> *zt, long zt_fs, const PairSrc &src, const PairDst &dst, const double *kx,
+                      int j0, int nplanes);
+void launch_pairs_fwd(hipStream_t s, const Geo &g, const IpLen &fx, const cx<double> *tw, int ld, const PairDst &src,
+                      cx<double> *wt, long wt_fs, const PairOut &out, int j0, int nplanes);
+// where pair planes keep x index i of a row, and row z
+int pair_slot(const IpLen &f, int i);
+int pair_zpos(const IpLen &f, int k);
+
+// les_chan's constant Smagorinsky model (dgpu_les.hip) on pair planes.
 void launch_les_bc(hipStream_t s, const Geo &g, cx<double> *cu1, cx<double> *cu3, int u_min, int u_max, int w_min,
                    int w_max);
-void launch_les_strain(hipStream_t s, const Geo &g, const cx<double> *cu1, const cx<double> *cu2,
-                       const cx<double> *cu3, const double *kx, const double *kz, const double *dy, const double *dyf,
-                       LesPtrs out);
-void launch_les_nut(hipStream_t s, const Geo &g, LesPtrs in, LesPtrs out, const cx<double> *cu1,
-                    const cx<double> *cu3, const double *dy, const double *dyf, const double *delta_y, int jstart,
-                    int jend);
-void launch_les_cf(hipStream_t s, const Geo &g, LesPtrs t, cx<double> *cf1, cx<double> *cf2, cx<double> *cf3,
-                   const double *kx, const double *kz, const double *dyf, const double *delta_y,
-                   const double *delta_yf, int j1, int j2, bool fresh);
-void launch_les_cross_src(hipStream_t s, const Geo &g, const double *nut, const double *u, const double *dy,
-                          double *out);
-void launch_les_cross_add(hipStream_t s, const Geo &g, const double *ct, cx<double> *cf2, const double *kx,
-                          const double *kz, int use_kz);
+struct LesProd {
+    const cx<double> *pr[6];  // the pairs of dgpu_les.hip
+    const cx<double> *bc;     // wall rows after APPLY_BC_VEL_PHYS
+    double *nut;              // NU_T, rows jlo..jhi written
+    cx<double> *wt;
+    long wt_fs;
+    const double *tab;        // per-row constants [NY+2][8]
+    const cx<double> *cu1, *cu3;  // mean profiles: mode 0
+    const double *kx;
+    long ps;
+    int ny, nz, jlo, jhi, chunk, zr, force;
+};
+void launch_les_prod(hipStream_t s, const Geo &g, const IpLen &fx, const cx<double> *tw, int ld, const LesProd &a);
+void launch_les_addcf(hipStream_t s, const Geo &g, cx<double> *cf, const cx<double> *f);
+void launch_les_nut_out(hipStream_t s, const Geo &g, const double *nut, const int *zpos, const int *slot,
+                        double *fort);
 
 // z transforms as split-BF16 DFT-as-GEMM on the matrix cores (dgpu_zdft.hip):
 // weights fragment-major, hi and lo halves, nmt M tiles of 32 rows, nks
@@ -305,26 +342,21 @@ struct LesCn {
 };
 void launch_les_bc_phys(hipStream_t s, const Geo &g, cx<double> *cu1, cx<double> *cu2, cx<double> *cu3,
                         const LesBc &b, const double *dy, const double *dyf);
-void launch_les_bc_phys_planes(hipStream_t s, const Geo &g, double *u1, double *u3, const LesBc &b, const double *dy);
-void launch_les_pack(hipStream_t s, const Geo &g, const cx<double> *src, double *fort, const double *kx,
-                     const double *kz, int kmul, int j0, int j1);
-void launch_les_mul(hipStream_t s, const Geo &g, double *a, const double *nut, int j0, int j1);
-void launch_les_acc(hipStream_t s, const Geo &g, cx<double> *dst, const double *fort, const double *kx,
-                    const double *kz, int kmul, int j0, int j1);
-// Up to four independent solves (TH, U2, U1, U3), each with its right-hand
-// side, output and two scratch planes.
+void launch_les_bc_rows(hipStream_t s, const Geo &g, const cx<double> *p0, const cx<double> *p1, cx<double> *bc,
+                        const LesBc &b, const double *dy, const double *dyf);
+void launch_les_bc_put(hipStream_t s, const Geo &g, cx<double> *p0, cx<double> *p1, const cx<double> *bc);
+// The solves of the pairs (U1, U2) and (U3, TH): per pair its systems (sys < 0:
+// none), right-hand sides, fields and two scratch pairs.
 struct LesCnSet {
-    LesCn a[4];
-    const double *rhs[4];
-    double *out[4], *bm[4], *gw[4];
-    int n;
+    LesCn a[2][2];
+    const cx<double> *rhs[2];
+    cx<double> *out[2], *cw[2], *gw[2];
 };
 void launch_les_cn(hipStream_t s, const Geo &g, const LesCnSet &set, const double *nut, const double *dy,
                    const double *dyf);
-void launch_les_vmax(hipStream_t s, const Geo &g, const double *u1, const double *u2, const double *u3, double *out);
-void launch_les_add(hipStream_t s, cx<double> *dst, const cx<double> *src, long n);
-void launch_les_eps(hipStream_t s, const Geo &g, const double *u1, const double *u2, const double *u3,
-                    const double *nut, const double *dy, const double *dyf, double *out);
+void launch_les_vmax(hipStream_t s, const Geo &g, const cx<double> *p0, const cx<double> *p1, double *out);
+void launch_les_eps(hipStream_t s, const Geo &g, const cx<double> *p0, const cx<double> *p1, const double *nut,
+                    const double *dy, const double *dyf, double *out);
 struct LesCfFix {
     double nu, beta, i_ro, drhodx, drhodz;
     int jstart, jend, jstart_th, jend_th;

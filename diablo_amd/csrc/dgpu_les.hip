@@ -1,35 +1,31 @@
-// dgpu_les.hip -- les_chan's constant Smagorinsky model (for/les.f:1-331) on
-// the device, in FP64, on Fortran-layout (0:NX+1, 0:NZ+1, 0:NY+1) planes:
+// dgpu_les.hip -- les_chan's constant Smagorinsky model (for/les.f:1-331) and
+// RK_CHAN_1's LES terms on the device, in FP64, on the pair planes of
+// dgpu_pairs.hip (P[j][zp][slot], two real fields a pair):
 //
-//   k_les_bc      APPLY_BC_LES (for/les.f:805-864) on the kept modes
-//   k_les_strain  S_ij of compute_strain_chan (for/les.f:526-571) in Fourier
-//                 space, and CU1, CU3, written as Fortran-layout Fourier
-//                 planes for the standalone transforms
-//   k_les_nut     |S| on GYF and GY, |S| S_ij with the implicit parts taken
-//                 out, NU_T on GY with GHOST_LES's zero rows
-//                 (for/les.f:107-230, for/mpi.f:488-503)
-//   k_les_cf      tau_ij = DELTA |S| S_ij and its divergence into CF1-3
-//                 (for/les.f:236-301)
-//   k_les_cross   NU_T dU/dy for the explicit cross terms, and their i k
-//                 into CF2 (for/les.f:302-331)
-#include "dgpu_kernels.hpp"
+//   pair 0 (U1, U2)            pair 3 (dU1/dz + dU3/dx, dU3/dz)
+//   pair 1 (U3, TH)            pair 4 (dU2/dz, dTH/dx)
+//   pair 2 (dU1/dx, dU2/dx)    pair 5 (dTH/dz, -)
+//
+//   k_les_bc       APPLY_BC_LES (for/les.f:805-864) on the kept modes
+//   k_les_bc_rows  APPLY_BC_VEL_PHYS (for/channel.f:2495-2640) of the wall rows
+//   k_les_prod     S_ij, |S| on GYF and GY, NU_T, tau_ij (for/les.f:107-301,
+//                  526-571), the explicit cross terms (for/les.f:302-331), the
+//                  scalar's eddy flux (for/channel.f:313-375) and the eleven
+//                  products of RK_CHAN_1, summed before one x forward
+//   k_les_cn       the Crank-Nicolson solves in physical space
+//
+// tau_ij, the cross terms and the eddy flux enter CF1-3 and CFTH through the
+// same i kx, i kz and d/dy as the products they sit beside, so they are added
+// to the products in physical space and cost no transforms of their own (the
+// transforms are linear: the sum differs by round-off only).
+#include "dgpu_hot.hpp"
+
+#include <algorithm>
+#include <cmath>
 
 namespace dgpu {
 
 namespace {
-
-__device__ __forceinline__ long fidx3(int i, int k, int j, int nx, int nz)
-{
-    return (long)i + (long)(nx + 2) * ((long)k + (long)(nz + 2) * (long)j);
-}
-
-// Fourier-view slot (i, K) of plane j of a Fortran-layout field
-__device__ __forceinline__ long cidx3(int i, int K, int j, int nxp, int nz)
-{
-    return (long)i + (long)(nxp + 1) * ((long)K + (long)(nz + 2) * (long)j);
-}
-
-__device__ __forceinline__ cx<double> i_times(double k, cx<double> a) { return make_cx<double>(-k * a.im, k * a.re); }
 
 __device__ __forceinline__ double sq(double x) { return x * x; }
 
@@ -55,202 +51,6 @@ __global__ void k_les_bc(Geo g, cx<double> *__restrict__ cu1, cx<double> *__rest
     if (u_min == 1) bottom(cu1);
     if (w_min == 1) bottom(cu3);
 }
-
-// out[q]: Fortran-layout Fourier planes; q = 0..5 S_11, S_22, S_33, S_12,
-// S_13, S_23 (the reference's Sij1..Sij6), 6 CU1, 7 CU3.  Slots outside the
-// kept modes and planes outside each S_ij's rows are zero.
-__global__ void k_les_strain(Geo g, const cx<double> *__restrict__ cu1, const cx<double> *__restrict__ cu2,
-                             const cx<double> *__restrict__ cu3, const double *__restrict__ kxv,
-                             const double *__restrict__ kzv, const double *__restrict__ dy,
-                             const double *__restrict__ dyf, LesPtrs out)
-{
-    const int nxp = g.nx / 2, nz = g.nz, NY = g.ny;
-    const long plane = (long)(nxp + 1) * (nz + 2);
-    const int j = blockIdx.y;
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= plane) return;
-    const int K = (int)(e / (nxp + 1)), i = (int)(e - (long)K * (nxp + 1));
-    const bool kept = i < g.mk && K < g.mz;
-    const long ps = g.ps;
-    const cx<double> zero = make_cx<double>(0.0, 0.0);
-    cx<double> s[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) s[q] = zero;
-    if (kept) {
-        const long m = (long)K * g.mk + i;
-        const double kx = kxv[i], kz = kzv[K];
-        auto at = [&](const cx<double> *f, int jj) { return f[m + (long)jj * ps]; };
-        const cx<double> u1 = at(cu1, j), u3 = at(cu3, j), u2 = at(cu2, j);
-        if (j >= 1 && j <= NY) {
-            const cx<double> u2p = at(cu2, j + 1);
-            s[0] = i_times(kx, u1);
-            s[1] = make_cx<double>((u2p.re - u2.re) / dyf[j], (u2p.im - u2.im) / dyf[j]);
-            s[2] = i_times(kz, u3);
-            const cx<double> a = i_times(kz, u1), b = i_times(kx, u3);
-            s[4] = make_cx<double>(0.5 * (a.re + b.re), 0.5 * (a.im + b.im));
-        }
-        if (j >= 1) {
-            const cx<double> u1m = at(cu1, j - 1), u3m = at(cu3, j - 1);
-            const cx<double> a = i_times(kx, u2), b = i_times(kz, u2);
-            s[3] = make_cx<double>(0.5 * ((u1.re - u1m.re) / dy[j] + a.re), 0.5 * ((u1.im - u1m.im) / dy[j] + a.im));
-            s[5] = make_cx<double>(0.5 * (b.re + (u3.re - u3m.re) / dy[j]), 0.5 * (b.im + (u3.im - u3m.im) / dy[j]));
-        }
-        s[6] = u1;
-        s[7] = u3;
-    }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-        double *p = out.p[q] + 2 * ((long)j * plane + e);
-        p[0] = s[q].re;
-        p[1] = s[q].im;
-    }
-}
-
-// Physical planes: in[0..5] S_ij, in[6] U1, in[7] U3; out[0..4] the stress
-// parts to transform (|S| S_11, |S| S_33, TEMP (S_12 - dU1/dy / 2),
-// |S| S_13, TEMP (S_23 - dU3/dy / 2)), out[5] NU_T.  ubar, wbar: the (0,0)
-// modes of CU1, CU3.  delta_y: -2 C^2 (DX DY(j) 2 DZ)^(2/3).
-__global__ void k_les_nut(Geo g, LesPtrs in, LesPtrs out,
-                          const cx<double> *__restrict__ cu1, const cx<double> *__restrict__ cu3,
-                          const double *__restrict__ dy, const double *__restrict__ dyf,
-                          const double *__restrict__ delta_y, int jstart, int jend)
-{
-    const int nx = g.nx, nz = g.nz, NY = g.ny;
-    const long n = (long)nx * nz;
-    const int j = blockIdx.y;
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n) return;
-    const int i = (int)(e % nx), k = (int)(e / nx);
-    const long ps = g.ps;
-    const long x = fidx3(i, k, j, nx, nz);
-    const double *S11 = in.p[0], *S22 = in.p[1], *S33 = in.p[2], *S12 = in.p[3], *S13 = in.p[4], *S23 = in.p[5];
-    const double *U1 = in.p[6], *U3 = in.p[7];
-    auto ub = [&](int jj) { return cu1[(long)jj * ps].re; };
-    auto wb = [&](int jj) { return cu3[(long)jj * ps].re; };
-    double o11 = S11[x], o33 = S33[x], o13 = S13[x], o12 = S12[x], o23 = S23[x], nut = 0.0;
-    if (j >= jstart && j <= jend) {  // |S| on GYF (for/les.f:107-130)
-        const long xp = fidx3(i, k, j + 1, nx, nz);
-        const double s1 = sqrt(2.0 * sq(S11[x])
-                               + 4.0 * sq(0.5 * (S12[xp] + S12[x]) - 0.5 * (ub(j) - ub(j - 1)) / dy[j]
-                                          - 0.5 * (ub(j + 1) - ub(j)) / dy[j + 1])
-                               + 4.0 * sq(S13[x]) + 2.0 * sq(S22[x])
-                               + 4.0 * sq(0.5 * (S23[xp] + S23[x]) - 0.5 * (wb(j) - wb(j - 1)) / dy[j]
-                                          - 0.5 * (wb(j + 1) - wb(j)) / dy[j + 1])
-                               + 2.0 * sq(S33[x]));
-        o11 = s1 * S11[x];
-        o13 = s1 * S13[x];
-        o33 = s1 * S33[x];
-    }
-    if (j >= 2 && j <= NY) {  // |S| on GY (for/les.f:133-156), then NU_T
-        const long xm = fidx3(i, k, j - 1, nx, nz);
-        const double w0 = dyf[j - 1], w1 = dyf[j], d2 = 2.0 * dy[j];
-        const double temp = sqrt(2.0 * sq((S11[x] * w0 + S11[xm] * w1) / d2)
-                                 + 4.0 * sq(S12[x] - 0.5 * (ub(j) - ub(j - 1)) / dy[j])
-                                 + 4.0 * sq((S13[x] * w0 + S13[xm] * w1) / d2)
-                                 + 2.0 * sq((S22[x] * w0 + S22[xm] * w1) / d2)
-                                 + 4.0 * sq(S23[x] - 0.5 * (wb(j) - wb(j - 1)) / dy[j])
-                                 + 2.0 * sq((S33[x] * w0 + S33[xm] * w1) / d2));
-        o12 = temp * (S12[x] - 0.5 * (U1[x] - U1[xm]) / dy[j]);
-        o23 = temp * (S23[x] - 0.5 * (U3[x] - U3[xm]) / dy[j]);
-        if (j >= 3 && j <= NY - 1) nut = -0.5 * delta_y[j] * temp;  // rows 1, 2, NY, NY+1 stay 0
-    }
-    out.p[0][x] = o11;
-    out.p[1][x] = o33;
-    out.p[2][x] = o12;
-    out.p[3][x] = o13;
-    out.p[4][x] = o23;
-    out.p[5][x] = nut;
-}
-
-// CF -= div tau (for/les.f:236-301): t[0..4] the transformed parts of
-// k_les_nut (Fortran-layout Fourier), scaled here by delta_yf / delta_y.
-// fresh: cf1..cf3 start from zero and every row 0..NY+1 is written (the
-// rows outside the force's ranges with zero), so the buffers need no clear.
-__global__ void k_les_cf(Geo g, LesPtrs t, cx<double> *__restrict__ cf1,
-                         cx<double> *__restrict__ cf2, cx<double> *__restrict__ cf3, const double *__restrict__ kxv,
-                         const double *__restrict__ kzv, const double *__restrict__ dyf,
-                         const double *__restrict__ delta_y, const double *__restrict__ delta_yf, int j1, int j2,
-                         int fresh)
-{
-    const long m = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y;
-    if (m >= g.ps) return;
-    const int K = (int)(m / g.mk), i = (int)(m - (long)K * g.mk);
-    const int nxp = g.nx / 2, nz = g.nz, NY = g.ny;
-    const long ps = g.ps;
-    const double kx = kxv[i], kz = kzv[K];
-    auto T = [&](int q, int jj, double scale) {
-        const cx<double> *a = reinterpret_cast<const cx<double> *>(t.p[q]);
-        const cx<double> v = a[cidx3(i, K, jj, nxp, nz)];
-        return make_cx<double>(scale * v.re, scale * v.im);
-    };
-    const long o = m + (long)j * ps;
-    const cx<double> zero = make_cx<double>(0.0, 0.0);
-    if (j >= j1 && j <= j2) {
-        const cx<double> c11 = T(0, j, delta_yf[j]), c13 = T(3, j, delta_yf[j]), c33 = T(1, j, delta_yf[j]);
-        const double dyj = j >= 2 ? delta_y[j] : 1.0;  // rows from 2 on are scaled (for/les.f:262-270)
-        const cx<double> c12 = T(2, j, dyj), c12p = T(2, j + 1, delta_y[j + 1]);
-        const cx<double> c23 = T(4, j, dyj), c23p = T(4, j + 1, delta_y[j + 1]);
-        cx<double> f = fresh ? zero : cf1[o];
-        const cx<double> a = i_times(kx, c11), b = i_times(kz, c13);
-        f = make_cx<double>(f.re - a.re - (c12p.re - c12.re) / dyf[j] - b.re,
-                            f.im - a.im - (c12p.im - c12.im) / dyf[j] - b.im);
-        cf1[o] = f;
-        cx<double> h = fresh ? zero : cf3[o];
-        const cx<double> c = i_times(kx, c13), d = i_times(kz, c33);
-        h = make_cx<double>(h.re - c.re - (c23p.re - c23.re) / dyf[j] - d.re,
-                            h.im - c.im - (c23p.im - c23.im) / dyf[j] - d.im);
-        cf3[o] = h;
-    } else if (fresh) {
-        cf1[o] = zero;
-        cf3[o] = zero;
-    }
-    if (j >= 2 && j <= NY) {
-        const cx<double> c12 = T(2, j, delta_y[j]), c23 = T(4, j, delta_y[j]);
-        const cx<double> a = i_times(kx, c12), b = i_times(kz, c23);
-        cx<double> f = fresh ? zero : cf2[o];
-        f = make_cx<double>(f.re - a.re - b.re, f.im - a.im - b.im);
-        cf2[o] = f;
-    } else if (fresh) {
-        cf2[o] = zero;
-    }
-}
-
-// NU_T (U(j) - U(j-1)) / DY(j) on rows 2..NY (physical), for the cross terms
-__global__ void k_les_cross_src(Geo g, const double *__restrict__ nut, const double *__restrict__ u,
-                                const double *__restrict__ dy, double *__restrict__ out)
-{
-    const int nx = g.nx, nz = g.nz;
-    const long n = (long)nx * nz;
-    const int j = 2 + blockIdx.y;
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n) return;
-    const int i = (int)(e % nx), k = (int)(e / nx);
-    const long x = fidx3(i, k, j, nx, nz), xm = fidx3(i, k, j - 1, nx, nz);
-    out[x] = nut[x] * (u[x] - u[xm]) / dy[j];
-}
-
-// CF2 += i k CT on rows 2..NY (k = kx for pass 0, kz for pass 1)
-__global__ void k_les_cross_add(Geo g, const double *__restrict__ ct, cx<double> *__restrict__ cf2,
-                                const double *__restrict__ kxv, const double *__restrict__ kzv, int use_kz)
-{
-    const long m = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = 2 + blockIdx.y;
-    if (m >= g.ps) return;
-    const int K = (int)(m / g.mk), i = (int)(m - (long)K * g.mk);
-    const int nxp = g.nx / 2, nz = g.nz;
-    const double k = use_kz ? kzv[K] : kxv[i];
-    const cx<double> v = reinterpret_cast<const cx<double> *>(ct)[cidx3(i, K, j, nxp, nz)];
-    const cx<double> a = i_times(k, v);
-    const long o = m + (long)j * g.ps;
-    cx<double> f = cf2[o];
-    f = make_cx<double>(f.re + a.re, f.im + a.im);
-    cf2[o] = f;
-}
-
-// ---------------------------------------------------------------------------
-// RK_CHAN_1 with LES: the Crank-Nicolson solves in physical space
-// ---------------------------------------------------------------------------
 
 // APPLY_BC_VEL_PHYS_LOWER / _UPPER (for/channel.f:2495-2640) stated on the
 // kept modes: a value C in physical space is C on the (0,0) mode and 0 on
@@ -302,151 +102,365 @@ __global__ void k_les_bc_phys(Geo g, cx<double> *__restrict__ cu1, cx<double> *_
     }
 }
 
-// APPLY_BC_VEL_PHYS_LOWER / _UPPER's U1 and U3 rows (for/channel.f:2495-2640)
-// on physical Fortran-layout planes.
-__global__ void k_les_bc_phys_planes(Geo g, double *__restrict__ u1, double *__restrict__ u3, LesBc b,
-                                     const double *__restrict__ dy)
+// Rows 0, 1, NY, NY+1 of pairs 0 and 1 after APPLY_BC_VEL_PHYS_LOWER / _UPPER
+// (for/channel.f:2495-2640), into bc[pair][4][NZ*NX]; TH and U2(NY) unchanged.
+__global__ void k_les_bc_rows(Geo g, const cx<double> *__restrict__ p0, const cx<double> *__restrict__ p1,
+                              cx<double> *__restrict__ bc, LesBc b, const double *__restrict__ dy,
+                              const double *__restrict__ dyf)
 {
     const long n = (long)g.nx * g.nz;
     const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n) return;
-    const int i = (int)(e % g.nx), k = (int)(e / g.nx), NY = g.ny;
-    auto X = [&](int j) { return fidx3(i, k, j, g.nx, g.nz); };
-    for (int q = 0; q < 2; ++q) {
-        double *u = q == 0 ? u1 : u3;
-        const int lo = q == 0 ? b.u_lo : b.w_lo, hi = q == 0 ? b.u_hi : b.w_hi;
-        const double clo = q == 0 ? b.u_lo_c : b.w_lo_c, chi = q == 0 ? b.u_hi_c : b.w_hi_c;
-        if (lo == 0) {
-            u[X(0)] = clo;
-            u[X(1)] = clo;
-        } else {
-            u[X(1)] = u[X(2)] - dy[2] * clo;
-            u[X(0)] = u[X(1)] - dy[1] * clo;
-        }
-        if (hi == 0) {
-            u[X(NY)] = chi;
-            u[X(NY + 1)] = chi;
-        } else {
-            u[X(NY)] = u[X(NY - 1)] + dy[NY] * chi;
-            u[X(NY + 1)] = u[X(NY)] + dy[NY] * chi;
-        }
+    const int NY = g.ny;
+    auto A = [&](const cx<double> *p, int j) { return p[(long)j * n + e]; };
+    const cx<double> r0[4] = {A(p0, 0), A(p0, 1), A(p0, NY), A(p0, NY + 1)};
+    const cx<double> r1[4] = {A(p1, 0), A(p1, 1), A(p1, NY), A(p1, NY + 1)};
+    const cx<double> a2 = A(p0, 2), an = A(p0, NY - 1), b2 = A(p1, 2), bn = A(p1, NY - 1);
+    auto horiz = [&](int lo, int hi, double clo, double chi, double u2, double un, double *o) {
+        o[1] = lo == 0 ? clo : u2 - dy[2] * clo;
+        o[0] = lo == 0 ? clo : o[1] - dy[1] * clo;
+        o[2] = hi == 0 ? chi : un + dy[NY] * chi;
+        o[3] = hi == 0 ? chi : o[2] + dy[NY] * chi;
+    };
+    double u[4], w[4], v[4];
+    horiz(b.u_lo, b.u_hi, b.u_lo_c, b.u_hi_c, a2.re, an.re, u);
+    horiz(b.w_lo, b.w_hi, b.w_lo_c, b.w_hi_c, b2.re, bn.re, w);
+    v[1] = b.v_lo == 0 ? 2.0 * b.v_lo_c - a2.im : a2.im - dyf[1] * b.v_lo_c;
+    v[0] = b.v_lo == 0 ? v[1] : v[1] - dyf[1] * b.v_lo_c;
+    v[2] = r0[2].im;
+    v[3] = b.v_hi == 0 ? 2.0 * b.v_hi_c - v[2] : v[2] + dy[NY] * b.v_hi_c;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        bc[r * n + e] = make_cx(u[r], v[r]);
+        bc[(4 + r) * n + e] = make_cx(w[r], r1[r].im);
     }
 }
 
-void launch_les_bc_phys_planes(hipStream_t s, const Geo &g, double *u1, double *u3, const LesBc &b, const double *dy)
+// The rows of k_les_bc_rows back into the pairs (the fields the solves take).
+__global__ void k_les_bc_put(Geo g, cx<double> *__restrict__ p0, cx<double> *__restrict__ p1,
+                             const cx<double> *__restrict__ bc)
 {
     const long n = (long)g.nx * g.nz;
-    hipLaunchKernelGGL(k_les_bc_phys_planes, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, g, u1, u3, b, dy);
-}
-
-// Kept modes (plane stride ps) -> Fortran-layout Fourier planes, times i kx
-// (kmul 1) or i kz (kmul 2); planes outside j0..j1 and slots outside the
-// kept modes are zero.
-__global__ void k_les_pack(Geo g, const cx<double> *__restrict__ src, double *__restrict__ fort,
-                           const double *__restrict__ kxv, const double *__restrict__ kzv, int kmul, int j0, int j1)
-{
-    const int nxp = g.nx / 2, nz = g.nz;
-    const long plane = (long)(nxp + 1) * (nz + 2);
-    const int j = blockIdx.y;
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= plane) return;
-    const int K = (int)(e / (nxp + 1)), i = (int)(e - (long)K * (nxp + 1));
-    cx<double> v = make_cx<double>(0.0, 0.0);
-    if (i < g.mk && K < g.mz && j >= j0 && j <= j1) {
-        v = src[(long)K * g.mk + i + (long)j * g.ps];
-        if (kmul == 1) v = i_times(kxv[i], v);
-        else if (kmul == 2) v = i_times(kzv[K], v);
-    }
-    double *p = fort + 2 * ((long)j * plane + e);
-    p[0] = v.re;
-    p[1] = v.im;
-}
-
-// Physical planes j0..j1: a *= nut
-__global__ void k_les_mul(Geo g, double *__restrict__ a, const double *__restrict__ nut, int j0)
-{
-    const long n = (long)g.nx * g.nz;
-    const int j = j0 + blockIdx.y;
     const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n) return;
-    const int i = (int)(e % g.nx), k = (int)(e / g.nx);
-    const long x = fidx3(i, k, j, g.nx, g.nz);
-    a[x] = nut[x] * a[x];
+    const int r = blockIdx.y & 3, j = r < 2 ? r : g.ny - 2 + r;
+    cx<double> *p = blockIdx.y < 4 ? p0 : p1;
+    p[(long)j * n + e] = bc[(long)blockIdx.y * n + e];
 }
 
-// dst (kept modes) += (i kx | i kz | 1) * Fortran-layout Fourier planes, j0..j1
-__global__ void k_les_acc(Geo g, cx<double> *__restrict__ dst, const double *__restrict__ fort,
-                          const double *__restrict__ kxv, const double *__restrict__ kzv, int kmul, int j0)
+// -------------------------------------------------------------------------
+// k_les_prod: zr z rows per block, planes ja..jb (a chunk of the sweep).  A
+// thread owns NP positions of the rows for the whole sweep and keeps what the
+// stencils need of the plane before in registers, so every pair value is read
+// from HBM once; the products of plane j = m - 1 (m the newest plane) go to
+// LDS and NPO rows of T threads run their x forward while the next plane's
+// values are on their way.  tab[j*8 + {0..6}]: 1/DYF, 1/DY, 1/(2 DYF),
+// DYF(j-1)/(2 DY), DYF(j)/(2 DY), -2 C^2 DELTA^2 on GYF, on GY.
+// force: the SGS force alone (dgpu_les_chan), no products and no scalar.
+// 384x257x384: 2.29 ms (5.6 GB: six pairs in, NU_T and eight row fields out),
+// bound by its registers (256, two waves per SIMD) rather than HBM; it replaces
+// the x kernel (1.30 ms), nine plane transforms (2.9 ms) and seven pointwise
+// kernels (2.9 ms) of the Fortran-layout form.  Substep 18.1 -> 10.0 ms.
+// -------------------------------------------------------------------------
+template <int E, int NTH, int PID, bool WIDE>
+__global__ void __launch_bounds__(WIDE ? 768 : 256) __attribute__((amdgpu_waves_per_eu(2))) k_les_prod(IpLen frt, const cx<double> *__restrict__ twg, int mk, int ld,
+                                                  LesProd a)
+{
+    constexpr int npo = XCount<NTH>::npo, NP = (E + npo - 1) / npo;
+    const IpLen &fx = plan_ref<PID>(frt);
+    extern __shared__ unsigned char smem_raw[];
+    cx<double> *const fb = reinterpret_cast<cx<double> *>(smem_raw);
+    const int nx = fx.n, TT = fx.t, S = fx.nstages, NY = a.ny;
+    const int tid = threadIdx.x, nthr = blockDim.x, zr = a.zr;
+    const int pg = tid / TT, zs = pg / npo, p = pg - zs * npo;
+    int th = tid - pg * TT;
+    cx<double> *tw = fb + (long)zr * npo * nx;
+    double *kxs = reinterpret_cast<double *>(tw + fx.twn);
+    for (int e = tid; e < fx.twn; e += nthr) tw[e] = twg[e];
+    for (int e = tid; e < mk; e += nthr) kxs[e] = a.kx[e];
+    const int zi = blockIdx.x * zr + zs;
+    const bool zvalid = zi < a.nz;
+    const int ja = a.jlo + blockIdx.y * a.chunk, jb = min(a.jhi, ja + a.chunk - 1);
+    const long pp = (long)a.nz * nx;
+    // this thread's positions: offset in a pair plane, LDS slot of product row 0
+    int off[NP], ls[NP];
+    bool on[NP];
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+        const int e0 = tid + nthr * k;
+        const bool in = e0 < zr * nx;
+        const int e = in ? e0 : 0, zq = e / nx, slot = e - zq * nx, zp = blockIdx.x * zr + zq;
+        on[k] = in && zp < a.nz;
+        off[k] = min(zp, a.nz - 1) * nx + slot;
+        const int R = fx.radix[S - 1], idx = slot / TT, u = idx / R;
+        const int pos = (slot - idx * TT + TT * u) * R + (idx - u * R);
+        ls[k] = in ? zq * npo * nx + ip_swz(fx, pos) : -1;
+    }
+    struct Keep {
+        double pu, pv, pw, pt, su, sw, s11, s13, s33, s22, s12, s23, dxt, dzt, nut, t12, t23, f1, f3, ft, q, p3, p4;
+    } K[NP];
+    cx<double> c0[NP], c1[NP], c2[NP], c3[NP], c4[NP], c5[NP], n0[NP];
+    auto load = [&](int plane) {
+#pragma unroll
+        for (int k = 0; k < NP; ++k) {
+            const long o = plane * pp + off[k];
+            c1[k] = a.pr[1][o];
+            c2[k] = a.pr[2][o];
+            c3[k] = a.pr[3][o];
+            c4[k] = a.pr[4][o];
+            if constexpr (NTH > 0) c5[k] = a.pr[5][o];
+        }
+    };
+    auto load0 = [&](int plane) {
+#pragma unroll
+        for (int k = 0; k < NP; ++k) n0[k] = a.pr[0][min(plane, NY + 1) * pp + off[k]];
+    };
+    load0(ja - 1);
+    load(ja - 1);
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+        c0[k] = n0[k];
+        K[k] = Keep{};
+        K[k].su = c0[k].re;
+        K[k].sw = c1[k].re;
+    }
+    load0(ja);
+    auto ub = [&](int j) { return a.cu1[(long)j * a.ps].re; };
+    auto wb = [&](int j) { return a.cu3[(long)j * a.ps].re; };
+    const bool wave_rows = (64 % TT) == 0;
+    auto row_sync = [&]() {
+        if (wave_rows) wave_lds_sync();
+        else __syncthreads();
+    };
+    double dub_j = 0.0, dwb_j = 0.0;
+    if (ja >= 2) {
+        dub_j = 0.5 * (ub(ja - 1) - ub(ja - 2)) * a.tab[(ja - 1) * 8 + 1];
+        dwb_j = 0.5 * (wb(ja - 1) - wb(ja - 2)) * a.tab[(ja - 1) * 8 + 1];
+    }
+    for (int m = ja - 1; m <= jb + 1; ++m) {
+        const int j = m - 1;
+        const bool out = j >= ja;
+        const double *T = a.tab + m * 8, *Tj = a.tab + max(j, 0) * 8;
+        const double rdy = T[1], w0 = T[3], w1 = T[4], dG = T[6];
+        const bool gy = m >= 2 && m <= NY, has_nut = m >= 3 && m <= NY - 1;
+        const bool stress = j >= 2 && j <= NY - 1;
+        const int br = m <= 1 ? m : (m >= NY ? m - NY + 2 : -1);
+        double dub = dub_j, dwb = dwb_j;  // m = ja - 1: kept above
+        if (m >= ja && m >= 1) {
+            dub = 0.5 * (ub(m) - ub(m - 1)) * rdy;
+            dwb = 0.5 * (wb(m) - wb(m - 1)) * rdy;
+        }
+#pragma unroll
+        for (int k = 0; k < NP; ++k) {
+            Keep &P = K[k];
+            const double Us = c0[k].re, Vs = c0[k].im, Ws = c1[k].re, th0 = c1[k].im;
+            double u = Us, v = Vs, w = Ws, t = th0;
+            if (br >= 0) {
+                const cx<double> x = a.bc[br * pp + off[k]], y = a.bc[(4 + br) * pp + off[k]];
+                u = x.re;
+                v = x.im;
+                w = y.re;
+            }
+            if (a.force) u = v = w = t = 0.0;
+            const double s11 = c2[k].re, s33 = c3[k].im, s13 = 0.5 * c3[k].re;
+            const double s22 = (n0[k].im - Vs) * T[0];
+            const double dU = (Us - P.su) * rdy, dW = (Ws - P.sw) * rdy;
+            const double s12 = 0.5 * (dU + c2[k].im), s23 = 0.5 * (c4[k].re + dW);
+            double t12 = 0.0, t23 = 0.0, nut = 0.0;
+            if (gy) {
+                const double S = sqrt(2.0 * sq(s11 * w0 + P.s11 * w1) + 4.0 * sq(s12 - dub) +
+                                      4.0 * sq(s13 * w0 + P.s13 * w1) + 2.0 * sq(s22 * w0 + P.s22 * w1) +
+                                      4.0 * sq(s23 - dwb) + 2.0 * sq(s33 * w0 + P.s33 * w1));
+                t12 = dG * (S * (s12 - 0.5 * dU));
+                t23 = dG * (S * (s23 - 0.5 * dW));
+                if (has_nut) nut = -0.5 * dG * S;
+            }
+            // at GY row m
+            const double p3 = (w1 * u + w0 * P.pu) * v + t12 - nut * dU;
+            const double p4 = (w1 * w + w0 * P.pw) * v + t23 - nut * dW;
+            const double f1 = (u + P.pu) * v, f3 = (w + P.pw) * v, ft = (t + P.pt) * v;
+            const double q = 0.25 * sq(v + P.pv);
+            if (out) {  // the products of plane j
+                double x1 = P.pu * P.pu, x0 = P.pw * P.pu, x2 = P.pw * P.pw;
+                double x5 = (f1 - P.f1) * Tj[2], x6 = (f3 - P.f3) * Tj[2];
+                if (stress) {
+                    const double S = sqrt(2.0 * sq(P.s11) + 4.0 * sq(0.5 * (s12 + P.s12) - dub_j - dub) +
+                                          4.0 * sq(P.s13) + 2.0 * sq(P.s22) +
+                                          4.0 * sq(0.5 * (s23 + P.s23) - dwb_j - dwb) + 2.0 * sq(P.s33));
+                    const double A = Tj[5] * S;
+                    x1 += A * P.s11;
+                    x0 += A * P.s13;
+                    x2 += A * P.s33;
+                    x5 += (t12 - P.t12) * Tj[0];
+                    x6 += (t23 - P.t23) * Tj[0];
+                }
+                if (ls[k] >= 0) {
+                    cx<double> *f = fb + ls[k];
+                    f[0 * nx] = make_cx(x1, x5);
+                    f[1 * nx] = make_cx(P.p3, (q - P.q) * Tj[1]);
+                    f[2 * nx] = make_cx(x0, x6);
+                    f[3 * nx] = make_cx(P.p4, x2);
+                    if constexpr (NTH > 0) {
+                        f[4 * nx] = make_cx(P.pt * P.pu - P.nut * P.dxt, (ft - P.ft) * Tj[2]);
+                        f[5 * nx] = make_cx(P.pt * P.pw - P.nut * P.dzt, 0.0);
+                    }
+                    if (on[k]) a.nut[j * pp + off[k]] = P.nut;
+                }
+            }
+            P.pu = u; P.pv = v; P.pw = w; P.pt = t;
+            P.su = Us; P.sw = Ws;
+            P.s11 = s11; P.s13 = s13; P.s33 = s33; P.s22 = s22; P.s12 = s12; P.s23 = s23;
+            if constexpr (NTH > 0) {
+                P.dxt = c4[k].im;
+                P.dzt = c5[k].re;
+            }
+            P.nut = nut; P.t12 = t12; P.t23 = t23;
+            P.f1 = f1; P.f3 = f3; P.ft = ft; P.q = q; P.p3 = p3; P.p4 = p4;
+        }
+        dub_j = dub;
+        dwb_j = dwb;
+        __syncthreads();
+        if (m <= jb) {
+#pragma unroll
+            for (int k = 0; k < NP; ++k) c0[k] = n0[k];
+            load0(m + 2);
+            load(m + 1);
+        }
+        if (out) {
+            asm volatile("" : "+v"(th));  // keeps the stages' index arithmetic out of the sweep's registers
+            cx<double> *row = fb + ((long)zs * npo + p) * nx;
+            stage_loop<PID != 0>(0, S - 1, [&](int s) {
+                ip_stage_row<double, E, -1, false>(row, fx, S - 1 - s, tw, th);
+                row_sync();
+            });
+            cx<double> *o0 = a.wt + ((long)j * a.nz + min(zi, a.nz - 1)) * ld;
+            const long wf = a.wt_fs;
+            const double h = 0.5 / nx;
+            x_split<double, E>(fx, row, tw, th, mk, [&](int kp, cx<double> Zk, cx<double> Zn) {
+                if (!zvalid) return;
+                const cx<double> Xa = make_cx((Zk.re + Zn.re) * h, (Zk.im - Zn.im) * h);
+                const cx<double> Xb = make_cx((Zk.im + Zn.im) * h, -(Zk.re - Zn.re) * h);
+                const double kx = kxs[kp];
+                const cx<double> G = make_cx(kx * Xa.im - Xb.re, -kx * Xa.re - Xb.im);  // -(i kx Xa + Xb)
+                const cx<double> nXa = make_cx(-Xa.re, -Xa.im), nXb = make_cx(-Xb.re, -Xb.im);
+                switch (p) {  // the outputs of k_xfused_ip's product rows
+                case 0: o0[0 * wf + kp] = G; break;
+                case 1: o0[2 * wf + kp] = G; break;
+                case 2: o0[4 * wf + kp] = G; o0[1 * wf + kp] = nXa; break;
+                case 3: o0[3 * wf + kp] = nXa; o0[5 * wf + kp] = nXb; break;
+                case 4: o0[6 * wf + kp] = G; break;
+                default: o0[7 * wf + kp] = nXa; break;
+                }
+            });
+        }
+        __syncthreads();
+    }
+}
+
+// WIDE: rows of more than 256 threads (NX above 512 or so)
+template <int E, int NTH, int PID, bool WIDE = false>
+static void les_prod_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<double> *tw, int ld, LesProd a)
+{
+    constexpr int npo = XCount<NTH>::npo;
+    if constexpr (!WIDE && PID == 0)
+        if (npo * fx.t > 256) return les_prod_e<E, NTH, PID, true>(s, g, fx, tw, ld, a);
+    // short rows are packed as in the fused x kernel
+    const size_t row = sizeof(cx<double>) * (size_t)fx.n * npo;
+    const size_t fixed = sizeof(cx<double>) * fx.twn + sizeof(double) * g.mk;
+    a.zr = 1;
+    while (2 * a.zr * npo * fx.t <= 256 && 2 * a.zr <= g.nz && fixed + 2 * a.zr * row <= 64 * 1024) a.zr *= 2;
+    const int threads = a.zr * npo * fx.t;
+    const size_t lds = fixed + a.zr * row;
+    if (lds > 64 * 1024)
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_les_prod<E, NTH, PID, WIDE>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    const long rows = (g.nz + a.zr - 1) / a.zr;
+    a.chunk = sweep_rule(rows, a.jhi - a.jlo + 1, kernel_slots(&k_les_prod<E, NTH, PID, WIDE>, threads, lds));
+    const int nchunks = (a.jhi - a.jlo + a.chunk) / a.chunk;
+    hipLaunchKernelGGL((k_les_prod<E, NTH, PID, WIDE>), dim3((unsigned)rows, nchunks), dim3(threads), lds, s, fx, tw, g.mk,
+                       ld, a);
+}
+
+void launch_les_prod(hipStream_t s, const Geo &g, const IpLen &fx, const cx<double> *tw, int ld, const LesProd &a)
+{
+    if (g.nth == 1 && with_pid(const_plan_id(fx), XPids64{}, [&](auto pc) {
+            constexpr int P = decltype(pc)::value;
+            les_prod_e<kConstPlanSpecs[P].e, 1, P>(s, g, fx, tw, ld, a);
+        }))
+        return;
+    if (g.nth == 0) {
+        DGPU_DISPATCH_XE64(fx.e, (les_prod_e<EE, 0, 0>(s, g, fx, tw, ld, a)));
+    } else {
+        DGPU_DISPATCH_XE64(fx.e, (les_prod_e<EE, 1, 0>(s, g, fx, tw, ld, a)));
+    }
+}
+
+// CF1-3 (rows 2..NY) += the SGS force in the nonlinear-term slots x, y, z.
+__global__ void k_les_addcf(Geo g, cx<double> *__restrict__ cf, const cx<double> *__restrict__ f)
 {
     const long m = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = j0 + blockIdx.y;
     if (m >= g.ps) return;
-    const int K = (int)(m / g.mk), i = (int)(m - (long)K * g.mk);
-    cx<double> v = reinterpret_cast<const cx<double> *>(fort)[cidx3(i, K, j, g.nx / 2, g.nz)];
-    if (kmul == 1) v = i_times(kxv[i], v);
-    else if (kmul == 2) v = i_times(kzv[K], v);
-    const long o = m + (long)j * g.ps;
-    cx<double> f = dst[o];
-    f = make_cx<double>(f.re + v.re, f.im + v.im);
-    dst[o] = f;
+    const long o = m + (long)(2 + blockIdx.y) * g.ps;
+    const cx<double> a = cf[o], b = f[o];
+    cf[o] = make_cx(a.re + b.re, a.im + b.im);
 }
 
-// One implicit Crank-Nicolson solve in physical space per (x, z) column
-// (for/channel.f:762-1029 with the LES terms): rows jlo..jhi from the
-// molecular and eddy parts, the boundary rows of APPLY_BC_*_LOWER/UPPER
-// (for/channel.f:1660-2282), THOMAS_REAL at NPROCY = 1 (for/mpi.f:630-809),
-// and rows clo..chi written to out.  bm, gw: per-column scratch planes.
-// With EXPL the right-hand side of rows jlo..jhi also takes the explicit
-// eddy-viscosity (diffusivity) half, temp2 d/dy(nut du/dy)
-// (for/channel.f:628-659, 748-760), from the field u at rows j-1..j+1: on
-// GYF rows with NU_T on the faces (U1, U3, TH), or on GY rows with NU_T
-// averaged onto the GYF faces (U2).
-template <bool EXPL>
-__device__ __forceinline__ void les_row(const LesCn &a, const double *__restrict__ nut, const double *u, long x,
-                                        long xp, long xm, const double *__restrict__ dy,
-                                        const double *__restrict__ dyf, const double *__restrict__ rhs, int j,
-                                        double &L, double &D, double &U, double &V)
+void launch_les_addcf(hipStream_t s, const Geo &g, cx<double> *cf, const cx<double> *f)
+{
+    hipLaunchKernelGGL(k_les_addcf, dim3((unsigned)((g.ps + 255) / 256), g.ny - 1), dim3(256), 0, s, g, cf, f);
+}
+
+// NU_T of pair planes as a Fortran-layout field, pads and rows outside 0..NX-1,
+// 0..NZ-1 zero.  zpos, slot: pair_zpos and pair_slot of every z and x.
+__global__ void k_les_nut_out(Geo g, const double *__restrict__ nut, const int *__restrict__ zpos,
+                              const int *__restrict__ slot, double *__restrict__ fort)
+{
+    const long plane = (long)(g.nx + 2) * (g.nz + 2);
+    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= plane) return;
+    const int k = (int)(e / (g.nx + 2)), i = (int)(e - (long)k * (g.nx + 2)), j = blockIdx.y;
+    fort[j * plane + e] =
+        (k < g.nz && i < g.nx) ? nut[((long)j * g.nz + zpos[k]) * g.nx + slot[i]] : 0.0;
+}
+
+void launch_les_nut_out(hipStream_t s, const Geo &g, const double *nut, const int *zpos, const int *slot, double *fort)
+{
+    const long plane = (long)(g.nx + 2) * (g.nz + 2);
+    hipLaunchKernelGGL(k_les_nut_out, dim3((unsigned)((plane + 255) / 256), g.ny + 2), dim3(256), 0, s, g, nut, zpos,
+                       slot, fort);
+}
+
+// One Crank-Nicolson row of one system (for/channel.f:762-1029 with the LES
+// terms): rows jlo..jhi from the molecular and eddy parts, the boundary rows
+// of APPLY_BC_*_LOWER/UPPER (for/channel.f:1660-2282).  n0, np, nm: NU_T at
+// rows j, j+1, j-1; u0, up, um the field, whose explicit eddy-viscosity half
+// temp2 d/dy(nut du/dy) (for/channel.f:628-659, 748-760) joins the right-hand
+// side r: on GYF rows with NU_T on the faces (U1, U3, TH), or on GY rows with
+// NU_T averaged onto the GYF faces (U2).
+__device__ __forceinline__ void les_row(const LesCn &a, int j, const double *__restrict__ dy,
+                                        const double *__restrict__ dyf, double n0, double np, double nm, double u0,
+                                        double up, double um, double r, double &L, double &D, double &U, double &V)
 {
     const int NY = a.ny;
     L = 0.0; D = 1.0; U = 0.0; V = 0.0;
     if (j >= a.jlo && j <= a.jhi) {
-        const double c = a.cmol;
-        if (a.sys == LES_SYS_TH) {
-            L = -c / (dy[j] * dyf[j]);
-            D = 1. + c / (dy[j + 1] * dyf[j]) + c / (dy[j] * dyf[j]);
-            U = -c / (dy[j + 1] * dyf[j]);
-        } else if (a.sys == LES_SYS_U2) {
-            L = -c / (dyf[j - 1] * dy[j]);
-            D = 1. + c / (dyf[j] * dy[j]) + c / (dyf[j - 1] * dy[j]);
-            U = -c / (dyf[j] * dy[j]);
-        } else {
-            L = -c / (dy[j] * dyf[j]);
-            D = 1. - c * (-1. / (dy[j + 1] * dyf[j]) - 1. / (dy[j] * dyf[j]));
-            U = -c / (dy[j + 1] * dyf[j]);
-        }
-        V = rhs[x];
-        const double t2 = a.temp2;
-        if constexpr (EXPL) {
-            double t;
-            if (a.sys == LES_SYS_U2)
-                t = (0.5 * (nut[x] + nut[xp]) * (u[xp] - u[x]) / dyf[j] -
-                     0.5 * (nut[x] + nut[xm]) * (u[x] - u[xm]) / dyf[j - 1]) /
-                    dy[j];
-            else
-                t = (nut[xp] * (u[xp] - u[x]) / dy[j + 1] - nut[x] * (u[x] - u[xm]) / dy[j]) / dyf[j];
-            V = V + t2 * t;
-        }
+        const double c = a.cmol, t2 = a.temp2;
+        double wm, wp, em, ep;  // molecular and eddy weights of rows j-1 and j+1
         if (a.sys == LES_SYS_U2) {
-            const double nm = nut[x] + nut[xm], np = nut[x] + nut[xp];
-            L = L - t2 * 0.5 * nm / (dyf[j - 1] * dy[j]);
-            D = D + t2 * 0.5 * np / (dyf[j] * dy[j]) + t2 * 0.5 * nm / (dyf[j - 1] * dy[j]);
-            U = U - t2 * 0.5 * np / (dyf[j] * dy[j]);
+            wm = 1.0 / (dyf[j - 1] * dy[j]);
+            wp = 1.0 / (dyf[j] * dy[j]);
+            em = t2 * 0.5 * (n0 + nm) * wm;
+            ep = t2 * 0.5 * (n0 + np) * wp;
         } else {
-            const double n0 = nut[x], n1 = nut[xp];
-            L = L - t2 * n0 / (dy[j] * dyf[j]);
-            D = D + t2 * n1 / (dy[j + 1] * dyf[j]) + t2 * n0 / (dy[j] * dyf[j]);
-            U = U - t2 * n1 / (dy[j + 1] * dyf[j]);
+            wm = 1.0 / (dy[j] * dyf[j]);
+            wp = 1.0 / (dy[j + 1] * dyf[j]);
+            em = t2 * n0 * wm;
+            ep = t2 * np * wp;
         }
+        L = -(c * wm + em);
+        U = -(c * wp + ep);
+        D = 1.0 + (c * wp + ep) + (c * wm + em);
+        V = r + (ep * (up - u0) - em * (u0 - um));
     }
     auto set = [&](double l, double d, double u, double v) { L = l; D = d; U = u; V = v; };
     if (a.sys == LES_SYS_U2) {
@@ -475,71 +489,79 @@ __device__ __forceinline__ void les_row(const LesCn &a, const double *__restrict
     }
 }
 
-// grid (column blocks, systems): every system of the substep in one launch
-// (they are independent), so the sweeps of all four fill the machine.  The
-// system's field is read (the explicit half, forward sweep) and overwritten
-// (back substitution) through out: a column is read and written by its own
-// thread only, every read before the first write.
-__global__ void k_les_cn(Geo g, LesCnSet set, const double *__restrict__ nut, const double *__restrict__ dy,
-                         const double *__restrict__ dyf)
+// THOMAS_REAL (for/mpi.f:630-809) down the columns of a pair plane, one thread
+// a real column of one of the pair's two systems (grid.y: the pair).  The
+// forward sweep leaves U/B and G/B of every row in the scratch planes; the
+// back substitution reads only those.  Rows clo..chi of the field are
+// overwritten.  A column is read and written by its own thread only, every
+// read of the field before the first write.
+__global__ void __launch_bounds__(256) k_les_cn(Geo g, LesCnSet set, const double *__restrict__ nut,
+                                                const double *__restrict__ dy, const double *__restrict__ dyf)
 {
-    const long n = (long)g.nx * g.nz;
+    const long n = 2L * g.nx * g.nz;  // doubles a pair plane
     const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n) return;
-    const int sy = blockIdx.y;
-    const LesCn &a = set.a[sy];
-    const double *__restrict__ rhs = set.rhs[sy];
-    double *__restrict__ bm = set.bm[sy];
-    double *__restrict__ gw = set.gw[sy];
-    double *__restrict__ out = set.out[sy];
-    const int i = (int)(e % g.nx), k = (int)(e / g.nx);
+    const LesCn a = set.a[blockIdx.y][e & 1];
+    if (a.sys < 0) return;
+    const double *__restrict__ rhs = reinterpret_cast<const double *>(set.rhs[blockIdx.y]) + e;
+    double *__restrict__ cw = reinterpret_cast<double *>(set.cw[blockIdx.y]) + e;
+    double *__restrict__ gw = reinterpret_cast<double *>(set.gw[blockIdx.y]) + e;
+    double *__restrict__ out = reinterpret_cast<double *>(set.out[blockIdx.y]) + e;
+    const double *__restrict__ nt = nut + (e >> 1);
+    const long nn = n >> 1;
     const int NY = g.ny;
-    auto X = [&](int j) { return fidx3(i, k, j, g.nx, g.nz); };
-    // forward elimination, rows 1..NY+1 (THOMAS_FORWARD_REAL_MPI)
-    double L, D, U, V;
-    les_row<true>(a, nut, out, X(0), X(1), X(0), dy, dyf, rhs, 0, L, D, U, V);
-    double bprev = D, cprev = U, gprev = V;
-    bm[X(0)] = D;
-    gw[X(0)] = V;
-    for (int j = 1; j <= NY + 1; ++j) {
-        const long x = X(j);
-        les_row<true>(a, nut, out, x, X(j <= NY ? j + 1 : j), X(j - 1), dy, dyf, rhs, j, L, D, U, V);
-        const double m = -L / bprev;
-        D = D + m * cprev;
-        V = V + m * gprev;
-        bm[x] = D;
-        gw[x] = V;
+    double um = 0.0, u0 = out[0], up = out[n], nm = 0.0, n0 = nt[0], np = nt[nn];
+    double bprev = 1.0, cprev = 0.0, gprev = 0.0;
+    for (int j = 0; j <= NY + 1; ++j) {
+        double L, D, U, V;
+        les_row(a, j, dy, dyf, n0, np, nm, u0, up, um, rhs[j * n], L, D, U, V);
+        if (j > 0) {
+            const double m = -L / bprev;
+            D = D + m * cprev;
+            V = V + m * gprev;
+        }
+        const double rb = D != 0.0 ? 1.0 / D : 0.0;  // zero-pivot guard of the back substitution
+        cw[j * n] = U * rb;
+        gw[j * n] = V * rb;
         bprev = D;
         cprev = U;
         gprev = V;
+        um = u0;
+        u0 = up;
+        nm = n0;
+        n0 = np;
+        const int jn = j + 2 <= NY + 1 ? j + 2 : NY + 1;
+        up = out[jn * n];
+        np = nt[jn * nn];
     }
-    // back substitution with the zero-pivot guard (THOMAS_BACKWARD_REAL_MPI)
-    double xn = gprev / bprev;
-    if (NY + 1 >= a.clo && NY + 1 <= a.chi) out[X(NY + 1)] = xn;
-    for (int j = NY; j >= 0; --j) {
-        const long x = X(j);
-        les_row<false>(a, nut, out, x, X(j + 1), X(j > 0 ? j - 1 : 0), dy, dyf, rhs, j, L, D, U, V);
-        const double b = bm[x];
-        xn = (b != 0.0) ? (gw[x] - U * xn) / b : 0.0;
-        if (j >= a.clo && j <= a.chi) out[x] = xn;
+    double xn = 0.0;
+    for (int j = NY + 1; j >= 0; --j) {
+        xn = gw[j * n] - cw[j * n] * xn;
+        if (j >= a.clo && j <= a.chi) out[j * n] = xn;
     }
+}
+
+void launch_les_cn(hipStream_t s, const Geo &g, const LesCnSet &set, const double *nut, const double *dy,
+                   const double *dyf)
+{
+    const long n = 2L * g.nx * g.nz;
+    hipLaunchKernelGGL(k_les_cn, dim3((unsigned)((n + 255) / 256), 2), dim3(256), 0, s, g, set, nut, dy, dyf);
 }
 
 // Per-plane maxima of |U1|, |U2|, |U3| on physical planes 1..NY into
 // out[q * NY + j - 1] (COURANT's input, for/courant.f:25-45)
-__global__ void __launch_bounds__(256) k_les_vmax(Geo g, const double *__restrict__ u1, const double *__restrict__ u2,
-                                                  const double *__restrict__ u3, double *__restrict__ out)
+__global__ void __launch_bounds__(256) k_les_vmax(Geo g, const cx<double> *__restrict__ p0,
+                                                  const cx<double> *__restrict__ p1, double *__restrict__ out)
 {
     __shared__ double red[3][256];
     const int j = 1 + blockIdx.x, tid = threadIdx.x;
     const long n = (long)g.nx * g.nz;
     double m[3] = {0.0, 0.0, 0.0};
     for (long e = tid; e < n; e += 256) {
-        const int i = (int)(e % g.nx), k = (int)(e / g.nx);
-        const long x = fidx3(i, k, j, g.nx, g.nz);
-        m[0] = fmax(m[0], fabs(u1[x]));
-        m[1] = fmax(m[1], fabs(u2[x]));
-        m[2] = fmax(m[2], fabs(u3[x]));
+        const cx<double> a = p0[j * n + e], b = p1[j * n + e];
+        m[0] = fmax(m[0], fabs(a.re));
+        m[1] = fmax(m[1], fabs(a.im));
+        m[2] = fmax(m[2], fabs(b.re));
     }
     for (int q = 0; q < 3; ++q) red[q][tid] = m[q];
     __syncthreads();
@@ -549,6 +571,11 @@ __global__ void __launch_bounds__(256) k_les_vmax(Geo g, const double *__restric
         __syncthreads();
     }
     if (tid < 3) out[(long)tid * g.ny + (j - 1)] = red[tid][0];
+}
+
+void launch_les_vmax(hipStream_t s, const Geo &g, const cx<double> *p0, const cx<double> *p1, double *out)
+{
+    hipLaunchKernelGGL(k_les_vmax, dim3(g.ny), dim3(256), 0, s, g, p0, p1, out);
 }
 
 // The reference forms CF from the velocity before les_chan resets its
@@ -600,8 +627,8 @@ void launch_les_cf_rows(hipStream_t s, const Geo &g, const cx<double> *pre, cons
 // tkebudget_chan_les (for/save_stats.f:887-960): per plane j = 1..NY the sum
 // over the physical points of u_i times its implicit eddy-viscosity term;
 // out[j - 1].  Fixed-order reduction.
-__global__ void __launch_bounds__(256) k_les_eps(Geo g, const double *__restrict__ u1, const double *__restrict__ u2,
-                                                 const double *__restrict__ u3, const double *__restrict__ nut,
+__global__ void __launch_bounds__(256) k_les_eps(Geo g, const cx<double> *__restrict__ p0,
+                                                 const cx<double> *__restrict__ p1, const double *__restrict__ nut,
                                                  const double *__restrict__ dy, const double *__restrict__ dyf,
                                                  double *__restrict__ out)
 {
@@ -610,15 +637,13 @@ __global__ void __launch_bounds__(256) k_les_eps(Geo g, const double *__restrict
     const long n = (long)g.nx * g.nz;
     double acc = 0.0;
     for (long e = tid; e < n; e += 256) {
-        const int i = (int)(e % g.nx), k = (int)(e / g.nx);
-        const long x = fidx3(i, k, j, g.nx, g.nz), xp = fidx3(i, k, j + 1, g.nx, g.nz),
-                   xm = fidx3(i, k, j - 1, g.nx, g.nz);
-        const double t = u1[x] * ((nut[xp] * (u1[xp] - u1[x]) / dy[j + 1] - nut[x] * (u1[x] - u1[xm]) / dy[j]) / dyf[j]) +
-                         u3[x] * ((nut[xp] * (u3[xp] - u3[x]) / dy[j + 1] - nut[x] * (u3[x] - u3[xm]) / dy[j]) / dyf[j]) +
-                         u2[x] * ((0.5 * (nut[x] + nut[xp]) * (u2[xp] - u2[x]) / dyf[j] -
-                                   0.5 * (nut[x] + nut[xm]) * (u2[x] - u2[xm]) / dyf[j - 1]) /
-                                  dy[j]);
-        acc += t;
+        const long x = j * n + e, xp = x + n, xm = x - n;
+        const cx<double> a = p0[x], ap = p0[xp], am = p0[xm];
+        const double w = p1[x].re, wp = p1[xp].re, wm = p1[xm].re, n0 = nut[x], np = nut[xp], nm = nut[xm];
+        acc += a.re * ((np * (ap.re - a.re) / dy[j + 1] - n0 * (a.re - am.re) / dy[j]) / dyf[j]) +
+               w * ((np * (wp - w) / dy[j + 1] - n0 * (w - wm) / dy[j]) / dyf[j]) +
+               a.im * ((0.5 * (n0 + np) * (ap.im - a.im) / dyf[j] - 0.5 * (n0 + nm) * (a.im - am.im) / dyf[j - 1]) /
+                       dy[j]);
     }
     red[tid] = acc;
     __syncthreads();
@@ -629,63 +654,10 @@ __global__ void __launch_bounds__(256) k_les_eps(Geo g, const double *__restrict
     if (tid == 0) out[j - 1] = red[0];
 }
 
-void launch_les_eps(hipStream_t s, const Geo &g, const double *u1, const double *u2, const double *u3,
-                    const double *nut, const double *dy, const double *dyf, double *out)
+void launch_les_eps(hipStream_t s, const Geo &g, const cx<double> *p0, const cx<double> *p1, const double *nut,
+                    const double *dy, const double *dyf, double *out)
 {
-    hipLaunchKernelGGL(k_les_eps, dim3(g.ny), dim3(256), 0, s, g, u1, u2, u3, nut, dy, dyf, out);
-}
-
-__global__ void k_les_add(cx<double> *__restrict__ dst, const cx<double> *__restrict__ src, long n)
-{
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n) return;
-    const cx<double> a = dst[e], b = src[e];
-    dst[e] = make_cx<double>(a.re + b.re, a.im + b.im);
-}
-
-void launch_les_add(hipStream_t s, cx<double> *dst, const cx<double> *src, long n)
-{
-    hipLaunchKernelGGL(k_les_add, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, dst, src, n);
-}
-
-void launch_les_bc_phys(hipStream_t s, const Geo &g, cx<double> *cu1, cx<double> *cu2, cx<double> *cu3,
-                        const LesBc &b, const double *dy, const double *dyf)
-{
-    hipLaunchKernelGGL(k_les_bc_phys, dim3((unsigned)((g.ps + 255) / 256)), dim3(256), 0, s, g, cu1, cu2, cu3, b, dy,
-                       dyf);
-}
-
-void launch_les_pack(hipStream_t s, const Geo &g, const cx<double> *src, double *fort, const double *kx,
-                     const double *kz, int kmul, int j0, int j1)
-{
-    const long plane = (long)(g.nx / 2 + 1) * (g.nz + 2);
-    hipLaunchKernelGGL(k_les_pack, dim3((unsigned)((plane + 255) / 256), g.ny + 2), dim3(256), 0, s, g, src, fort,
-                       kx, kz, kmul, j0, j1);
-}
-
-void launch_les_mul(hipStream_t s, const Geo &g, double *a, const double *nut, int j0, int j1)
-{
-    const long n = (long)g.nx * g.nz;
-    hipLaunchKernelGGL(k_les_mul, dim3((unsigned)((n + 255) / 256), j1 - j0 + 1), dim3(256), 0, s, g, a, nut, j0);
-}
-
-void launch_les_acc(hipStream_t s, const Geo &g, cx<double> *dst, const double *fort, const double *kx,
-                    const double *kz, int kmul, int j0, int j1)
-{
-    hipLaunchKernelGGL(k_les_acc, dim3((unsigned)((g.ps + 255) / 256), j1 - j0 + 1), dim3(256), 0, s, g, dst, fort,
-                       kx, kz, kmul, j0);
-}
-
-void launch_les_cn(hipStream_t s, const Geo &g, const LesCnSet &set, const double *nut, const double *dy,
-                   const double *dyf)
-{
-    const long n = (long)g.nx * g.nz;
-    hipLaunchKernelGGL(k_les_cn, dim3((unsigned)((n + 255) / 256), set.n), dim3(256), 0, s, g, set, nut, dy, dyf);
-}
-
-void launch_les_vmax(hipStream_t s, const Geo &g, const double *u1, const double *u2, const double *u3, double *out)
-{
-    hipLaunchKernelGGL(k_les_vmax, dim3(g.ny), dim3(256), 0, s, g, u1, u2, u3, out);
+    hipLaunchKernelGGL(k_les_eps, dim3(g.ny), dim3(256), 0, s, g, p0, p1, nut, dy, dyf, out);
 }
 
 void launch_les_bc(hipStream_t s, const Geo &g, cx<double> *cu1, cx<double> *cu3, int u_min, int u_max, int w_min,
@@ -695,45 +667,24 @@ void launch_les_bc(hipStream_t s, const Geo &g, cx<double> *cu1, cx<double> *cu3
                        w_min, w_max);
 }
 
-void launch_les_strain(hipStream_t s, const Geo &g, const cx<double> *cu1, const cx<double> *cu2,
-                       const cx<double> *cu3, const double *kx, const double *kz, const double *dy, const double *dyf,
-                       LesPtrs out)
+void launch_les_bc_phys(hipStream_t s, const Geo &g, cx<double> *cu1, cx<double> *cu2, cx<double> *cu3,
+                        const LesBc &b, const double *dy, const double *dyf)
 {
-    const long plane = (long)(g.nx / 2 + 1) * (g.nz + 2);
-    hipLaunchKernelGGL(k_les_strain, dim3((unsigned)((plane + 255) / 256), g.ny + 2), dim3(256), 0, s, g, cu1, cu2,
-                       cu3, kx, kz, dy, dyf, out);
+    hipLaunchKernelGGL(k_les_bc_phys, dim3((unsigned)((g.ps + 255) / 256)), dim3(256), 0, s, g, cu1, cu2, cu3, b, dy,
+                       dyf);
 }
 
-void launch_les_nut(hipStream_t s, const Geo &g, LesPtrs in, LesPtrs out,
-                    const cx<double> *cu1, const cx<double> *cu3, const double *dy, const double *dyf,
-                    const double *delta_y, int jstart, int jend)
+void launch_les_bc_rows(hipStream_t s, const Geo &g, const cx<double> *p0, const cx<double> *p1, cx<double> *bc,
+                        const LesBc &b, const double *dy, const double *dyf)
 {
     const long n = (long)g.nx * g.nz;
-    hipLaunchKernelGGL(k_les_nut, dim3((unsigned)((n + 255) / 256), g.ny + 2), dim3(256), 0, s, g, in, out, cu1, cu3,
-                       dy, dyf, delta_y, jstart, jend);
+    hipLaunchKernelGGL(k_les_bc_rows, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, g, p0, p1, bc, b, dy, dyf);
 }
 
-void launch_les_cf(hipStream_t s, const Geo &g, LesPtrs t, cx<double> *cf1, cx<double> *cf2,
-                   cx<double> *cf3, const double *kx, const double *kz, const double *dyf, const double *delta_y,
-                   const double *delta_yf, int j1, int j2, bool fresh)
-{
-    hipLaunchKernelGGL(k_les_cf, dim3((unsigned)((g.ps + 255) / 256), g.ny + (fresh ? 2 : 1)), dim3(256), 0, s, g,
-                       t, cf1, cf2, cf3, kx, kz, dyf, delta_y, delta_yf, j1, j2, fresh ? 1 : 0);
-}
-
-void launch_les_cross_src(hipStream_t s, const Geo &g, const double *nut, const double *u, const double *dy,
-                          double *out)
+void launch_les_bc_put(hipStream_t s, const Geo &g, cx<double> *p0, cx<double> *p1, const cx<double> *bc)
 {
     const long n = (long)g.nx * g.nz;
-    hipLaunchKernelGGL(k_les_cross_src, dim3((unsigned)((n + 255) / 256), g.ny - 1), dim3(256), 0, s, g, nut, u, dy,
-                       out);
-}
-
-void launch_les_cross_add(hipStream_t s, const Geo &g, const double *ct, cx<double> *cf2, const double *kx,
-                          const double *kz, int use_kz)
-{
-    hipLaunchKernelGGL(k_les_cross_add, dim3((unsigned)((g.ps + 255) / 256), g.ny - 1), dim3(256), 0, s, g, ct, cf2,
-                       kx, kz, use_kz);
+    hipLaunchKernelGGL(k_les_bc_put, dim3((unsigned)((n + 255) / 256), 8), dim3(256), 0, s, g, p0, p1, bc);
 }
 
 }  // namespace dgpu
