@@ -85,7 +85,6 @@ struct dgpu_ctx {
     cx<double> *d_zt = nullptr, *d_wt = nullptr;
     long zfs = 0;  // complex elements per intermediate field: (NY+2)*NZ*ld
     double *d_fort = nullptr;  // Fortran-layout staging for host entry points
-    double *d_fa = nullptr, *d_fb = nullptr;  // POISSON_P_CHAN work planes
     double *d_gyf = nullptr;    // GYF (0:NY+1), part of d_vec
     double *d_stats = nullptr;  // dgpu_stats_chan output
     double *d_noalloc = nullptr;  // this GPU's fixed array of dgpu_stats_chan_noalloc
@@ -742,7 +741,7 @@ int32_t dgpu_destroy(dgpu_ctx *c)
         if (ge) (void)hipGraphExecDestroy(ge);
     for (auto e : c->event_pool) (void)hipEventDestroy(e);
     void *bufs[] = {c->d_vec, c->d_tw, c->d_state, c->d_pmult, c->d_pinv, c->d_rd, c->d_nlptr, c->d_zt, c->d_wt,
-                    c->d_fa, c->d_fb, c->d_iptw, c->d_iptwf, c->d_ztf, c->d_wtf, c->d_nlf, c->d_nlptrf,
+                    c->d_iptw, c->d_iptwf, c->d_ztf, c->d_wtf, c->d_nlf, c->d_nlptrf,
                     c->d_fort, c->d_cn, c->d_codes, c->d_c1, c->d_state32, c->d_side, c->d_map,
                     c->d_pmultf, c->d_pinvf, c->d_gs32, c->d_stats, c->d_vmax_part, c->d_vmax, c->d_file, c->d_les, c->d_zdft,
                     c->d_pairtw, c->d_perm, c->d_pairs};
@@ -2077,7 +2076,7 @@ int32_t dgpu_fft_xz_to_physical(dgpu_ctx *c, double *vv, int32_t jmin, int32_t j
     return DGPU_OK;
 }
 
-// Device-side Fortran-layout plane transforms used by POISSON_P_CHAN.
+// Device-side Fortran-layout plane transforms used by the restart files.
 static int fort_to_physical(dgpu_ctx *c, double *buf, int j0, int j1)
 {
     const dgpu::Geo &g = c->g;
@@ -2106,36 +2105,35 @@ int32_t dgpu_poisson_p_chan(dgpu_ctx *c)
     if (int rc = to_master(c)) return rc;
     c->master_dirty = true;
     const dgpu::Geo &g = c->g;
-    if (int rc = ensure_fort(c)) return rc;
-    const size_t n = (size_t)(g.nx + 2) * (g.nz + 2) * (g.ny + 2);
-    if (!c->d_fa) HIPCHK(c, hipMalloc(&c->d_fa, n * sizeof(double)));
-    if (!c->d_fb) HIPCHK(c, hipMalloc(&c->d_fb, n * sizeof(double)));
-    double *fa = c->d_fa, *fb = c->d_fb, *fc = c->d_fort;
+    if (int rc = ensure_pairs(c, 6)) return rc;
+    const cx<double> *twz = c->d_iptw + c->ipx.twn;
     cx<double> *cs = c->nl[1], *scr = c->nl[0];
-    const int j0 = 2, j1 = g.ny;
-    for (int group = 0; group < 4; ++group) {
-        dgpu::launch_pp_spec(c->stream, group, g, c->cu[0], c->cu[1], c->cu[2], c->d_dyf, c->d_kx, c->d_kz, fa, fb,
-                             group == 0 ? fc : nullptr);
-        if (int rc = check_launch(c, "pp_spec")) return rc;
-        if (int rc = fort_to_physical(c, fa, j0, j1)) return rc;
-        if (int rc = fort_to_physical(c, fb, j0, j1)) return rc;
-        if (group == 0) {
-            if (int rc = fort_to_physical(c, fc, j0, j1)) return rc;
-            dgpu::launch_pp_phys(c->stream, 0, g, fa, fb, fb, fc);
-        } else {
-            dgpu::launch_pp_phys(c->stream, 1, g, fa, fb, fb, nullptr);
-        }
-        if (int rc = check_launch(c, "pp_phys")) return rc;
-        if (int rc = fort_to_fourier(c, fa, j0, j1)) return rc;
-        if (group == 0) {
-            if (int rc = fort_to_fourier(c, fb, j0, j1)) return rc;
-            if (int rc = fort_to_fourier(c, fc, j0, j1)) return rc;
-            dgpu::launch_pp_accum(c->stream, g, cs, fa, fb, fc, 1);
-        } else {
-            dgpu::launch_pp_accum(c->stream, g, cs, fa, nullptr, nullptr, 0);
-        }
-        if (int rc = check_launch(c, "pp_accum")) return rc;
+    // CU1-3 and their z derivatives (Wt fields 0-2, 3-5), with the x
+    // derivatives on five pair planes
+    dgpu::ZSrc z{};
+    z.n = 6;
+    for (int q = 0; q < 6; ++q) {
+        z.p[q] = c->cu[q % 3];
+        z.dz[q] = q >= 3;
     }
+    dgpu::launch_zinv_src(c->stream, g, c->ipz, twz, z, c->d_wt, c->zfs, c->ld, c->d_kz, 0, g.ny + 2);
+    if (int rc = check_launch(c, "zinv(poisson)")) return rc;
+    const dgpu::PairSrc src{{0, 2, -1, 3, 5}, {-1, -1, 1, -1, -1}, {1, -1, -1, 4, -1}, {-1, 0, 2, -1, -1}, 5};
+    if (int rc = pairs_x(c, src, c->d_wt, 0)) return rc;
+    dgpu::PairDst pr{};
+    for (int q = 0; q < 5; ++q) pr.p[q] = pair_buf(c, q);
+    dgpu::launch_pp_rhs(c->stream, g, pr, pair_buf(c, 5), c->d_dyf);
+    if (int rc = check_launch(c, "pp_rhs")) return rc;
+    // rows 2 + 2q and 3 + 2q: the two rows of pair plane q, Wt fields 0 and 1
+    const dgpu::PairDst sum{{pair_buf(c, 5)}};
+    dgpu::launch_pairs_fwd(c->stream, g, c->ipx64, c->d_pairtw, c->ld, sum, c->d_wt, c->zfs,
+                           dgpu::PairOut{{0}, {1}, 1}, 0, g.ny / 2);
+    if (int rc = check_launch(c, "x forward(poisson)")) return rc;
+    dgpu::Geo g2 = g;
+    g2.ps = 2 * g.ps;
+    dgpu::launch_zfwd_dst(c->stream, g2, c->ipz, twz, c->d_wt, c->zfs, c->ld,
+                          dgpu::ZDst{{cs + 2 * g.ps, cs + 3 * g.ps}, 2}, 0, g.ny / 2);
+    if (int rc = check_launch(c, "zfwd(poisson)")) return rc;
     dgpu::launch_pp_solve(c->stream, g, cs, g.nth ? c->cth[0] : nullptr, g.nth ? c->p.ri[0] : 0.0, c->d_gyf,
                           c->d_pmult, c->d_pinv, c->d_rd, scr, c->cp);
     if (int rc = check_launch(c, "pp_solve")) return rc;

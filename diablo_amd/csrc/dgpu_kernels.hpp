@@ -218,13 +218,7 @@ void launch_zfwd_pack(hipStream_t s, const Geo &g, const Fft<T> &fz, const cx<T>
 template <typename T>
 void launch_x_c2r(hipStream_t s, const Geo &g, const Fft<T> &fx, const cx<T> *zt, int mkin, double *fort, int j0,
                   int nplanes);
-// POISSON_P_CHAN pieces (dgpu_poisson.hip)
-void launch_pp_spec(hipStream_t s, int group, const Geo &g, const cx<double> *cu1, const cx<double> *cu2,
-                    const cx<double> *cu3, const double *dyf, const double *kx, const double *kz, double *fa,
-                    double *fb, double *fc);
-void launch_pp_phys(hipStream_t s, int op, const Geo &g, double *fa, const double *fb, double *fbw, double *fc);
-void launch_pp_accum(hipStream_t s, const Geo &g, cx<double> *cs, const double *fa, const double *fb,
-                     const double *fc, int first);
+// POISSON_P_CHAN's solve (dgpu_poisson.hip)
 void launch_pp_solve(hipStream_t s, const Geo &g, const cx<double> *cs, const cx<double> *cth, double ri,
                      const double *gyf, const double *pmult, const double *pinv, const double *rd, cx<double> *scr,
                      cx<double> *cp);
@@ -292,6 +286,8 @@ void launch_pairs_inv(hipStream_t s, const Geo &g, const IpLen &fx, const cx<dou
                       int j0, int nplanes);
 void launch_pairs_fwd(hipStream_t s, const Geo &g, const IpLen &fx, const cx<double> *tw, int ld, const PairDst &src,
                       cx<double> *wt, long wt_fs, const PairOut &out, int j0, int nplanes);
+// POISSON_P_CHAN's right-hand sides, rows 2.. two by two (dgpu_poisson.hip)
+void launch_pp_rhs(hipStream_t s, const Geo &g, const PairDst &pr, cx<double> *out, const double *dyf);
 // where pair planes keep x index i of a row, and row z
 int pair_slot(const IpLen &f, int i);
 int pair_zpos(const IpLen &f, int k);

@@ -1,179 +1,158 @@
 // dgpu_poisson.hip -- POISSON_P_CHAN (for/channel.f:1217-1453) on the device.
 //
 // CP from CU1-3 (and CTH): the right-hand side sum_ij (du_i/dx_j)(du_j/dx_i)
-// is assembled with the reference's four groups of terms (nine transforms to
-// physical space and six back), then one tridiagonal solve per (kx,kz) mode.
+// in physical space from the velocity and its x and z gradients on pair planes
+// (dgpu_pairs.hip; the y differences of the reference's spectral inputs are
+// taken on the physical planes, which is the same by linearity), then one
+// tridiagonal solve per (kx,kz) mode.  The reference transforms each of its
+// six products back; here they are summed first and two planes' sums share one
+// complex x transform: nine inverse real transforms and one forward a plane.
+// 192x129x192: 1031 -> 500 us for the whole call, of which the solve 179 -> 48.
 // The solve rows that are read (1..NY) carry the same matrix as REM_DIV_CHAN's
 // (for/channel.f:1126-1143 vs 1399-1440, boundary rows for/mpi.f:1293-1369),
 // so the context's precomputed Poisson factorisation is reused.
-//
-// Work arrays are Fortran-layout planes (the layout the standalone transform
-// kernels take); this routine runs once per restart, not per time step.
 #include "dgpu_kernels.hpp"
 
 namespace dgpu {
 
-// Spectral inputs of one group of terms into Fortran-layout complex planes.
-// group 0: (i kx CU1, (CU2(j+1)-CU2(j))/DYF(j), i kz CU3)
-// group 1: ((CU1(j+1)-CU1(j-1))/(2 DYF(j)), i kx 0.5 (CU2(j)+CU2(j+1)))
-// group 2: ((CU3(j+1)-CU3(j-1))/(2 DYF(j)), i kz 0.5 (CU2(j)+CU2(j+1)))
-// group 3: (i kz CU1, i kx CU3)
-// Planes 2..NY get the values on the kept slots; every other slot is zero.
-__global__ void k_pp_spec(int group, Geo g, const cx<double> *__restrict__ cu1, const cx<double> *__restrict__ cu2,
-                          const cx<double> *__restrict__ cu3, const double *__restrict__ dyf,
-                          const double *__restrict__ kxv, const double *__restrict__ kzv, double *fa, double *fb,
-                          double *fc)
+// pairs: 0 (U1, U2), 1 (U3, dU1/dx), 2 (dU2/dx, dU3/dx), 3 (dU1/dz, dU2/dz),
+// 4 (dU3/dz, -).  out plane q: the right-hand sides of rows 2 + 2q and 3 + 2q
+// (0 beyond NY).  A thread owns one position and a chunk of plane pairs; the
+// planes it has read roll through its registers.
+__global__ void __launch_bounds__(256) k_pp_rhs(Geo g, PairDst pr, cx<double> *__restrict__ out,
+                                                const double *__restrict__ dyf, int chunk)
 {
-    const int j = blockIdx.y;
-    const int nxp = g.nx / 2;
-    const long plane = (long)(nxp + 1) * (g.nz + 2);
-    const long ps = g.ps;
-    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < plane; e += (long)gridDim.x * blockDim.x) {
-        const int K = (int)(e / (nxp + 1)), i = (int)(e - (long)K * (nxp + 1));
-        cx<double> a = make_cx<double>(0, 0), b = a, c = a;
-        if (i < g.mk && K < g.mz && j >= 2 && j <= g.ny) {
-            const long o = (long)j * ps + (long)K * g.mk + i;
-            const double kx = kxv[i], kz = kzv[K];
-            if (group == 0) {
-                const cx<double> u1 = cu1[o], u3 = cu3[o], d = cu2[o + ps] - cu2[o];
-                a = make_cx<double>(-kx * u1.im, kx * u1.re);
-                b = make_cx<double>(d.re / dyf[j], d.im / dyf[j]);
-                c = make_cx<double>(-kz * u3.im, kz * u3.re);
-            } else if (group == 1 || group == 2) {
-                const cx<double> *u = (group == 1) ? cu1 : cu3;
-                const double k = (group == 1) ? kx : kz;
-                const cx<double> d = u[o + ps] - u[o - ps];
-                a = make_cx<double>(d.re / (2. * dyf[j]), d.im / (2. * dyf[j]));
-                const cx<double> s = cu2[o] + cu2[o + ps];
-                b = make_cx<double>(-(k * 0.5) * s.im, (k * 0.5) * s.re);
-            } else {
-                const cx<double> u1 = cu1[o], u3 = cu3[o];
-                a = make_cx<double>(-kz * u1.im, kz * u1.re);
-                b = make_cx<double>(-kx * u3.im, kx * u3.re);
-            }
+    const long n = (long)g.nx * g.nz;
+    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= n) return;
+    const int NY = g.ny, q0 = blockIdx.y * chunk, q1 = min(q0 + chunk, NY / 2);
+    auto at = [&](int q, int j) { return pr.p[q][(long)min(j, NY + 1) * n + e]; };
+    const int j0 = 2 + 2 * q0;
+    double um = at(0, j0 - 1).re, wm = at(1, j0 - 1).re;
+    cx<double> a = at(0, j0), b = at(1, j0), c = at(2, j0), d = at(3, j0), f = at(4, j0);
+    for (int q = q0; q < q1; ++q) {
+        double r[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int j = 2 + 2 * q + h;
+            const cx<double> ap = at(0, j + 1), bp = at(1, j + 1), cp = at(2, j + 1), dp = at(3, j + 1),
+                             fp = at(4, j + 1);
+            const double i1 = 1.0 / dyf[min(j, NY + 1)], i2 = 0.5 * i1;
+            const double vy = (ap.im - a.im) * i1, uy = (ap.re - um) * i2, wy = (bp.re - wm) * i2;
+            const double vx = 0.5 * (c.re + cp.re), vz = 0.5 * (d.im + dp.im);
+            r[h] = j <= NY ? b.im * b.im + vy * vy + f.re * f.re + 2.0 * uy * vx + 2.0 * wy * vz + 2.0 * d.re * c.im
+                           : 0.0;
+            um = a.re;
+            wm = b.re;
+            a = ap; b = bp; c = cp; d = dp; f = fp;
         }
-        const long idx = ((long)j * plane + e) * 2;
-        fa[idx] = a.re; fa[idx + 1] = a.im;
-        fb[idx] = b.re; fb[idx + 1] = b.im;
-        if (fc) { fc[idx] = c.re; fc[idx + 1] = c.im; }
+        out[(long)q * n + e] = make_cx(r[0], r[1]);
     }
 }
 
-// Physical-space products on planes 2..NY: op 0 squares a, b, c in place
-// (for/channel.f:1246-1254); op 1 sets a = 2*a*b (for/channel.f:1283-1289).
-__global__ void k_pp_phys(int op, Geo g, double *fa, const double *fb, double *fbw, double *fc)
+void launch_pp_rhs(hipStream_t s, const Geo &g, const PairDst &pr, cx<double> *out, const double *dyf)
 {
-    const int j = 2 + blockIdx.y;
-    const long rowlen = g.nx + 2;
-    const long plane = rowlen * (g.nz + 2);
-    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < (long)g.nz * g.nx;
-         e += (long)gridDim.x * blockDim.x) {
-        const int z = (int)(e / g.nx), x = (int)(e - (long)z * g.nx);
-        const long idx = (long)j * plane + (long)z * rowlen + x;
-        if (op == 0) {
-            fa[idx] = fa[idx] * fa[idx];
-            fbw[idx] = fbw[idx] * fbw[idx];
-            fc[idx] = fc[idx] * fc[idx];
-        } else {
-            fa[idx] = 2. * fa[idx] * fb[idx];
-        }
-    }
+    const long n = (long)g.nx * g.nz;
+    const int chunk = 8;  // 16 planes: one in nine read twice
+    hipLaunchKernelGGL(k_pp_rhs, dim3((unsigned)((n + 255) / 256), (g.ny / 2 + chunk - 1) / chunk), dim3(256), 0, s, g,
+                       pr, out, dyf, chunk);
 }
 
-// cs (kept layout, planes 2..NY) = [cs +] a (+ b + c) from Fortran-layout
-// Fourier planes (for/channel.f:1261-1367).
-__global__ void k_pp_accum(Geo g, cx<double> *cs, const double *fa, const double *fb, const double *fc, int first)
+// Buoyancy term, the tridiagonal solve and CP (for/channel.f:1373-1449).  The
+// elimination is two linear recurrences over the rows, g(j) = r(j) + m(j)
+// g(j-1) and phi(j) = (g(j) - U(j) phi(j+1)) / B(j); a column is cut into 16
+// segments run side by side from zero and then again from their carries, which
+// pass from segment to segment through LDS (one thread a column took 179 us at
+// 192x129x192: 131 waves, 258 dependent rows).  16 modes (256 B of a row) x 16
+// segments a block.
+__global__ void __launch_bounds__(256) k_pp_solve(Geo g, const cx<double> *__restrict__ cs,
+                                                  const cx<double> *__restrict__ cth, double ri,
+                                                  const double *__restrict__ gyf, const double *__restrict__ pmult,
+                                                  const double *__restrict__ pinv, const double *__restrict__ rd,
+                                                  cx<double> *__restrict__ scr, cx<double> *__restrict__ cp)
 {
-    const int j = 2 + blockIdx.y;
-    const int nxp = g.nx / 2;
-    const long plane = (long)(nxp + 1) * (g.nz + 2);
-    for (long m = (long)blockIdx.x * blockDim.x + threadIdx.x; m < g.ps; m += (long)gridDim.x * blockDim.x) {
-        const int K = (int)(m / g.mk), i = (int)(m - (long)K * g.mk);
-        const long idx = ((long)j * plane + (long)K * (nxp + 1) + i) * 2;
-        cx<double> v = make_cx<double>(fa[idx], fa[idx + 1]);
-        if (fb) v = v + make_cx<double>(fb[idx], fb[idx + 1]);
-        if (fc) v = v + make_cx<double>(fc[idx], fc[idx + 1]);
-        cx<double> &o = cs[(long)j * g.ps + m];
-        o = first ? v : o + v;
-    }
-}
-
-// Buoyancy term, the tridiagonal solve and CP (for/channel.f:1373-1449).
-__global__ void k_pp_solve(Geo g, const cx<double> *__restrict__ cs, const cx<double> *__restrict__ cth,
-                           double ri, const double *__restrict__ gyf, const double *__restrict__ pmult,
-                           const double *__restrict__ pinv, const double *__restrict__ rd, cx<double> *scr,
-                           cx<double> *cp)
-{
-    const long m = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= g.ps) return;
-    const bool is00 = (m == 0);
-    const int NY = g.ny;
+    __shared__ cx<double> end[16][16];
+    __shared__ double prod[16][16];
+    const int lm = threadIdx.x & 15, seg = threadIdx.x >> 4;
+    const long mode = (long)blockIdx.x * 16 + lm;
+    const bool on = mode < g.ps;
+    const long m = on ? mode : g.ps - 1;
+    const bool is00 = m == 0;
+    const int NY = g.ny, len = (NY + 15) / 16, a = 1 + seg * len, b = min(NY, a + len - 1);
     const long ps = g.ps;
-    cx<double> gprev = make_cx<double>(0, 0);
-    scr[m + ps] = gprev;
-    for (int j = 2; j <= NY; ++j) {
+    const cx<double> zero = make_cx(0.0, 0.0);
+    auto row = [&](int j, cx<double> gp) {  // forward recurrence
         const long o = m + (long)j * ps;
-        cx<double> vec = make_cx<double>(0, 0);
+        if (j == 1) return zero;
+        cx<double> v = zero;
         if (j < NY) {
             cx<double> s = cs[o];
             if (cth && !is00) {
                 const cx<double> d = cth[o + ps] - cth[o - ps];
                 const double den = gyf[j + 1] - gyf[j - 1];
-                s = s + make_cx<double>((ri * d.re) / den, (ri * d.im) / den);
+                s = s + make_cx((ri * d.re) / den, (ri * d.im) / den);
             }
-            vec = make_cx<double>(-1. * s.re, -1. * s.im);
+            v = make_cx(-s.re, -s.im);
         }
         const double mu = pmult[o];
-        const cx<double> gj = make_cx<double>(vec.re + mu * gprev.re, vec.im + mu * gprev.im);
-        scr[o] = gj;
-        gprev = gj;
+        return make_cx(v.re + mu * gp.re, v.im + mu * gp.im);
+    };
+    cx<double> x = zero;
+    double pr = 1.0;
+    for (int j = a; j <= b; ++j) {
+        x = row(j, x);
+        pr = j == 1 ? 0.0 : pr * pmult[m + (long)j * ps];
     }
-    cx<double> phip = make_cx<double>(0, 0);
-    const double u1row = is00 ? 0.0 : -1.0;
-    for (int j = NY; j >= 1; --j) {
+    end[seg][lm] = x;
+    prod[seg][lm] = pr;
+    __syncthreads();
+    x = zero;
+    for (int s = 0; s < seg; ++s) {
+        const cx<double> t = end[s][lm];
+        const double p = prod[s][lm];
+        x = make_cx(t.re + p * x.re, t.im + p * x.im);
+    }
+    for (int j = a; j <= b; ++j) {
+        x = row(j, x);
+        if (on) scr[m + (long)j * ps] = x;
+    }
+    __syncthreads();
+    // back substitution; the last row takes no row above
+    auto back = [&](int j, cx<double> xp, double &w) {
         const long o = m + (long)j * ps;
         const cx<double> gj = scr[o];
-        const double ip = pinv[o];
-        cx<double> phi;
-        if (j == NY) {
-            phi = make_cx<double>(gj.re * ip, gj.im * ip);
-        } else {
-            const double U = (j == 1) ? u1row : rd[(long)j * 4 + 0];
-            phi = make_cx<double>((gj.re - U * phip.re) * ip, (gj.im - U * phip.im) * ip);
-        }
-        cp[o] = phi;
-        phip = phi;
+        const double ip = pinv[o], U = j == NY ? 0.0 : (j == 1 ? (is00 ? 0.0 : -1.0) : rd[(long)j * 4]);
+        w = -U * ip;
+        return make_cx((gj.re - U * xp.re) * ip, (gj.im - U * xp.im) * ip);
+    };
+    x = zero;
+    pr = 1.0;
+    for (int j = b; j >= a; --j) {
+        double w;
+        x = back(j, x, w);
+        pr *= w;
     }
-}
-
-void launch_pp_spec(hipStream_t s, int group, const Geo &g, const cx<double> *cu1, const cx<double> *cu2,
-                    const cx<double> *cu3, const double *dyf, const double *kx, const double *kz, double *fa,
-                    double *fb, double *fc)
-{
-    const long plane = (long)(g.nx / 2 + 1) * (g.nz + 2);
-    hipLaunchKernelGGL(k_pp_spec, dim3((unsigned)((plane + 255) / 256), g.ny + 2), dim3(256), 0, s, group, g, cu1,
-                       cu2, cu3, dyf, kx, kz, fa, fb, fc);
-}
-
-void launch_pp_phys(hipStream_t s, int op, const Geo &g, double *fa, const double *fb, double *fbw, double *fc)
-{
-    const long n = (long)g.nz * g.nx;
-    hipLaunchKernelGGL(k_pp_phys, dim3((unsigned)((n + 255) / 256), g.ny - 1), dim3(256), 0, s, op, g, fa, fb, fbw,
-                       fc);
-}
-
-void launch_pp_accum(hipStream_t s, const Geo &g, cx<double> *cs, const double *fa, const double *fb,
-                     const double *fc, int first)
-{
-    hipLaunchKernelGGL(k_pp_accum, dim3((unsigned)((g.ps + 255) / 256), g.ny - 1), dim3(256), 0, s, g, cs, fa, fb,
-                       fc, first);
+    end[seg][lm] = x;
+    prod[seg][lm] = pr;
+    __syncthreads();
+    x = zero;
+    for (int s = 15; s > seg; --s) {
+        const cx<double> t = end[s][lm];
+        const double p = prod[s][lm];
+        x = make_cx(t.re + p * x.re, t.im + p * x.im);
+    }
+    for (int j = b; j >= a; --j) {
+        double w;
+        x = back(j, x, w);
+        if (on) cp[m + (long)j * ps] = x;
+    }
 }
 
 void launch_pp_solve(hipStream_t s, const Geo &g, const cx<double> *cs, const cx<double> *cth, double ri,
                      const double *gyf, const double *pmult, const double *pinv, const double *rd, cx<double> *scr,
                      cx<double> *cp)
 {
-    hipLaunchKernelGGL(k_pp_solve, dim3((unsigned)((g.ps + 63) / 64)), dim3(64), 0, s, g, cs, cth, ri, gyf, pmult,
+    hipLaunchKernelGGL(k_pp_solve, dim3((unsigned)((g.ps + 15) / 16)), dim3(256), 0, s, g, cs, cth, ri, gyf, pmult,
                        pinv, rd, scr, cp);
 }
 

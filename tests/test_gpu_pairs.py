@@ -71,3 +71,20 @@ def test_les_sizes(oracle_mod, size, deck):
 def test_les_chan_mixed_only_lengths(oracle_mod, nx):
     say("les_chan mixed", nx)
     _les_chan(oracle_mod, case.channel_case(nx, 6, 8, kick=0.3, streak=0.1), "mixed")
+
+
+@pytest.mark.parametrize("size", SIZES)
+@pytest.mark.parametrize("deck", ["channel", "kh"])
+def test_poisson_sizes(oracle_mod, size, deck):
+    """Odd and even NY (the last pair of rows half empty or full), more and
+    fewer rows than the solve's 16 segments; 1e-11 as the same call's other test."""
+    nx, ny, nz = size
+    cfg = (case.channel_case(nx, ny, nz, kick=0.3, streak=0.1) if deck == "channel"
+           else case.kh_case(nx, ny, nz, kick=0.05))
+    say("poisson", deck, size)
+    o, g = _pair(oracle_mod, cfg, "fp64")
+    g.poisson_p_chan()
+    o.poisson_p_chan()
+    errs, bad = compare_states(cfg, g.state(), o.state(), 1e-11, fields=("CP",))
+    say(errs)
+    assert not bad, bad
