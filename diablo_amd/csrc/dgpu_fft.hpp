@@ -302,7 +302,7 @@ constexpr ConstPlanSpec kConstPlanSpecs[] = {
     {0, 0, 0, 0u, 0},
     // x plans (rows of the fused nonlinear kernel); row swizzle mask, shift
     {384, 12, 6, 15u, 0, 2},  // 1: (6,4,4,4), FP64
-    {192, 12, 6, 15u, 0, 2},  // 2: (6,4,4,2), FP32
+    {192, 12, 6, 15u, 0, 2},  // 2: (6,4,4,2), FP32 and FP64
     {96, 12, 6, 14u, 0, 1},   // 3: (6,4,4), FP32
     {128, 8, 4, 15u, 0, 3},   // 4: (4,8,4), FP64
     {64, 16, 8, 12u, 0, 1},   // 5: (8,8), FP32
@@ -322,6 +322,9 @@ constexpr ConstPlanSpec kConstPlanSpecs[] = {
     {192, 12, 0, 0u, 0},           // 15: (6,4,4,2)
     {256, 8, 0, 0u, 2},            // 16: (8,8,4)
     {384, 12, 6, 31u, 0, 2},       // 17: (6,4,4,4), FP32 x plan
+    // FP64 x plans of the short rows
+    {96, 12, 6, 7u, 0, 2},         // 18: (6,4,4), FP64
+    {64, 8, 4, 7u, 0, 3},          // 19: (4,8,2), FP64
 };
 constexpr int kNumConstPlans = (int)(sizeof(kConstPlanSpecs) / sizeof(kConstPlanSpecs[0]));
 

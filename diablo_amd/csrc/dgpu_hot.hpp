@@ -39,7 +39,7 @@ __device__ constexpr IpLen kDevConstPlans[] = {const_plan(0),  const_plan(1),  c
                                                const_plan(4),  const_plan(5),  const_plan(6),  const_plan(7),
                                                const_plan(8),  const_plan(9),  const_plan(10), const_plan(11),
                                                const_plan(12), const_plan(13), const_plan(14), const_plan(15),
-                                               const_plan(16), const_plan(17)};
+                                               const_plan(16), const_plan(17), const_plan(18), const_plan(19)};
 static_assert(sizeof(kDevConstPlans) / sizeof(IpLen) == (size_t)kNumConstPlans, "one entry per compile-time plan");
 
 template <int PID>
@@ -80,18 +80,17 @@ static inline int z_lw(int t)
 }
 
 // Compile-time plans each kernel family is built for, per precision (ids of
-// kConstPlanSpecs): x, the 384 and 256 cases in both precisions and the
-// ensemble lengths of the FP32 path; z, every length with a plan, both
-// precisions.
+// kConstPlanSpecs): the x and z plans of 64, 96, 128, 192, 256 and 384 in both
+// precisions.  On a run-time plan the stage loops do not unroll and every index
+// is computed with run-time divisors: one RK3 step at 128x129x128 FP64 726 ->
+// 667 us, 192x129x192 FP64 1833 -> 1713 and mixed 1055 -> 949 us with the x
+// kernel on the compile-time plan.
 template <int... P>
 struct PidList {};
 template <typename T>
-using XPids = std::conditional_t<sizeof(T) == 4, PidList<2, 3, 5, 13, 14, 17>, PidList<1, 12>>;
-// the single-context x kernel: the 384 and 256 plans
-template <typename T>
-using XPidsSingle = std::conditional_t<sizeof(T) == 4, PidList<13, 17>, PidList<1, 12>>;
+using XPids = std::conditional_t<sizeof(T) == 4, PidList<2, 3, 5, 13, 14, 17>, PidList<1, 2, 4, 12, 18, 19>>;
 // the FP64 pair transforms (dgpu_pairs.hip) and the LES products
-using XPids64 = PidList<1, 12>;
+using XPids64 = XPids<double>;
 template <typename T>
 using ZPids = PidList<6, 8, 9, 10, 15, 16>;
 

@@ -517,14 +517,14 @@ static void xfused_ip_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T
 }
 
 
-// The single-run x kernel is built for the 384 and 256 plans (the ensembles
-// use the batched kernel) with one scalar; other shapes run on runtime plans.
+// The x kernels are built for the compile-time plans with one scalar; other
+// shapes run on run-time plans.
 template <typename T>
 static void xfused_ip_any(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, int ld, const cx<T> *zt,
                           long zt_fs, cx<T> *wt, long wt_fs, const double *dy, const double *dyf, const double *kx,
                           int jlo, int jhi, int chunk, int *pick)
 {
-    if (g.nth == 1 && with_pid(const_plan_id(fx), XPidsSingle<T>{}, [&](auto pc) {
+    if (g.nth == 1 && with_pid(const_plan_id(fx), XPids<T>{}, [&](auto pc) {
             constexpr int P = decltype(pc)::value;
             xfused_ip_e<T, kConstPlanSpecs[P].e, 1, P>(s, g, fx, tw, ld, zt, zt_fs, wt, wt_fs, dy, dyf, kx, jlo, jhi,
                                                        chunk, pick);
