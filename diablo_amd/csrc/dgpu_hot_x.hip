@@ -28,7 +28,7 @@ namespace dgpu {
 // position by position in the same permutation for every row.
 // -------------------------------------------------------------------------
 template <typename T, int E, int NTH, bool CP, bool MZ>
-__device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__restrict__ twg, int mk, int ld,
+__device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__restrict__ twg, int mk_rt, int ld,
                                             const cx<T> *__restrict__ zt, long zt_fs, long zt_ps,
                                             cx<T> *__restrict__ wt, long wt_fs, long wt_ps,
                                             const double *__restrict__ dy, const double *__restrict__ dyf,
@@ -46,6 +46,10 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
     const int nx = fx.n;
     const int zsz = (3 * npi + npo) * nx;  // a z row's window and product rows
     const int TT = fx.t, S = fx.nstages, L0 = fx.span[0];
+    // with a compile-time plan the kept modes are constant too, and which of a
+    // thread's inputs and outputs lie in the dealiasing gap is known: their
+    // loads, selects and stores go
+    const int mk = CP ? nx / 3 + 1 : mk_rt;
     const int tid = threadIdx.x, nthr = blockDim.x;
     const int pg = tid / TT, zs = MZ ? pg / nrow : 0;
     const int p = pg - zs * nrow;
@@ -247,6 +251,7 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
         // every stage out of the sweep, which would hold it in registers
         // across the whole loop: recomputing it is cheaper than the spills.
         asm volatile("" : "+v"(th));
+        __builtin_assume(th >= 0 && th < TT);
         const bool inv = j <= jb && dif_row;  // backward of plane j+1
         const bool fwd = j > ja && dit_row;   // forward of the products of plane j-1
         cx<T> *drow = inv ? slot_row(j + 1, p) : win;
@@ -254,7 +259,10 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
         stage_loop<CP>(0, S - 1, [&](int s) {
             // FP32: once more per stage (its 128 VGPRs spill less: 0.645 ->
             // 0.622 ms at 384; FP64 measured no better)
-            if constexpr (sizeof(T) == 4) asm volatile("" : "+v"(th));
+            if constexpr (sizeof(T) == 4) {
+                asm volatile("" : "+v"(th));
+                __builtin_assume(th >= 0 && th < TT);
+            }
             if (inv) ip_stage_row<T, E, +1, true>(drow, fx, s + 1, tw, th);
             if (fwd) ip_stage_row<T, E, -1, false>(frow, fx, S - 1 - s, tw, th);
             row_sync();
