@@ -1155,8 +1155,8 @@ static int ensure_pairs(dgpu_ctx *c, int n)
     return DGPU_OK;
 }
 
-// Kept modes of CU1-3, CTH (and, with grads, their z derivatives) to the rows
-// Wt, fields 0..nin-1 (nin..2 nin-1).
+// Kept modes of CU1-3, CTH to the rows Wt, fields 0..nin-1; with grads also
+// dU1/dz + dU3/dx, dU2/dz, dU3/dz and dTH/dz, fields nin..2 nin-1.
 static int pairs_z(dgpu_ctx *c, bool grads)
 {
     const int nin = 3 + c->g.nth;
@@ -1166,8 +1166,9 @@ static int pairs_z(dgpu_ctx *c, bool grads)
         z.p[q] = q % nin < 3 ? c->cu[q % nin] : c->cth[0];
         z.dz[q] = q >= nin;
     }
-    dgpu::launch_zinv_src(c->stream, c->g, c->ipz, c->d_iptw + c->ipx.twn, z, c->d_wt, c->zfs, c->ld, c->d_kz, 0,
-                          c->g.ny + 2);
+    if (grads) z.x[nin] = c->cu[2];
+    dgpu::launch_zinv_src(c->stream, c->g, c->ipz, c->d_iptw + c->ipx.twn, z, c->d_wt, c->zfs, c->ld, c->d_kx,
+                          c->d_kz, 0, c->g.ny + 2);
     return check_launch(c, "zinv(pairs)");
 }
 
@@ -1183,14 +1184,14 @@ static int pairs_x(dgpu_ctx *c, const dgpu::PairSrc &src, const cx<double> *zt, 
 // (U1, U2), (U3, TH) of Wt's first fields
 static dgpu::PairSrc pairs_of_fields(const dgpu_ctx *c)
 {
-    return dgpu::PairSrc{{0, 2}, {-1, -1}, {1, c->g.nth ? 3 : -1}, {-1, -1}, 2};
+    return dgpu::PairSrc{{0, 2}, {1, c->g.nth ? 3 : -1}, {0, 0}, {0, 0}, 2};
 }
 
 struct LesMem {
     double *nut;         // NU_T
     cx<double> *bc;      // [2][4][NZ*NX]
     cx<double> *pre;     // [4][ps]
-    double *tab;         // [NY+2][8]
+    double *tab, *w;     // [NY+2][8], [NY+2][4]
     size_t bytes;
 };
 static LesMem les_mem(const dgpu_ctx *c)
@@ -1207,6 +1208,7 @@ static LesMem les_mem(const dgpu_ctx *c)
     m.bc = reinterpret_cast<cx<double> *>(take(sizeof(cx<double>) * 8 * pair_plane(c)));
     m.pre = reinterpret_cast<cx<double> *>(take(sizeof(cx<double>) * 4 * c->g.ps));
     m.tab = reinterpret_cast<double *>(take(sizeof(double) * 8 * (c->g.ny + 2)));
+    m.w = reinterpret_cast<double *>(take(sizeof(double) * 4 * (c->g.ny + 2)));
     m.bytes = at;
     return m;
 }
@@ -1240,7 +1242,14 @@ static int ensure_les(dgpu_ctx *c)
         r[5] = -2.0 * std::pow(C_SMAG, 2.0) * std::pow(dx * beta_sgs * DYF[j] * 2.0 * dz * beta_sgs, 2.0 / 3.0);
         r[6] = -2.0 * std::pow(C_SMAG, 2.0) * std::pow(dx * beta_sgs * DY[j] * 2.0 * dz * beta_sgs, 2.0 / 3.0);
     }
+    std::vector<double> w(4 * (size_t)(NY + 2), 0.0);
+    for (int j = 1; j <= NY; ++j) {
+        if (j > 1) w[4 * (size_t)j] = 1.0 / (DYF[j - 1] * DY[j]);
+        w[4 * (size_t)j + 1] = 1.0 / (DY[j] * DYF[j]);
+        w[4 * (size_t)j + 2] = 1.0 / (DY[j + 1] * DYF[j]);
+    }
     HIPCHK(c, hipMemcpyAsync(les_mem(c).tab, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(les_mem(c).w, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return DGPU_OK;
 }
@@ -1262,13 +1271,13 @@ static int les_terms(dgpu_ctx *c, int jlo, bool force)
                         c->p.w_bc_ymax);
     if (int rc = check_launch(c, "les_bc")) return rc;
     if (int rc = pairs_z(c, true)) return rc;
-    const int th = g.nth ? 3 : -1, dth = g.nth ? nin + 3 : -1;
-    // pairs 0-5 (dgpu_les.hip): plain rows, x derivatives, z derivatives
-    dgpu::PairSrc src{{0, 2, -1, nin, nin + 1, dth},
-                      {-1, -1, 0, 2, -1, -1},
-                      {1, th, -1, nin + 2, -1, -1},
-                      {-1, -1, 1, -1, th, -1},
-                      g.nth ? 6 : 5};
+    const int th = g.nth ? 3 : -1;
+    // pairs 0-5 (dgpu_les.hip)
+    const dgpu::PairSrc src{{0, 2, 0, nin, nin + 1, nin + 3},
+                            {1, th, 1, nin + 2, th, -1},
+                            {0, 0, 1, 0, 0, 0},
+                            {0, 0, 1, 0, 1, 0},
+                            g.nth ? 6 : 5};
     if (int rc = pairs_x(c, src, c->d_wt, 0)) return rc;
     dgpu::LesBc b;
     b.u_lo = c->p.u_bc_ymin; b.u_hi = c->p.u_bc_ymax; b.w_lo = c->p.w_bc_ymin; b.w_hi = c->p.w_bc_ymax;
@@ -1772,14 +1781,13 @@ static int les_substep(dgpu_ctx *c, int rk_step, double time, double temp1, doub
         if (int rc = check_launch(c, "zfwd_nl")) return rc;
         if (int rc = pairs_x(c, pairs_of_fields(c), c->d_zt, 0)) return rc;
     }
-    // new CF and the right-hand sides (sweep A of the column kernel)
+    // new CF and the right-hand sides
     dgpu::CnArgs A;
     make_cn_args(c, rk_step, time, temp3, temp4, temp5, A);
-    A.rhs_only = 1;
     dgpu::CnPtrs<double, double> P;
     fill_ptrs<double>(c, P, c->nl);
-    dgpu::launch_cn<double, double>(c->stream, A, P);
-    if (int rc = check_launch(c, "cn(rhs)")) return rc;
+    dgpu::launch_cn_rhs(c->stream, A, P);
+    if (int rc = check_launch(c, "cn_rhs")) return rc;
     if (c->les_model) {
         dgpu::LesCfFix f;
         f.nu = c->p.nu; f.beta = c->p.beta; f.i_ro = c->p.i_ro;
@@ -1794,7 +1802,7 @@ static int les_substep(dgpu_ctx *c, int rk_step, double time, double temp1, doub
     dgpu::ZSrc z{};
     z.n = nin;
     for (int q = 0; q < nin; ++q) z.p[q] = c->nl[q];
-    dgpu::launch_zinv_src(c->stream, g, c->ipz, twz, z, c->d_zt, c->zfs, c->ld, c->d_kz, 0, NY + 2);
+    dgpu::launch_zinv_src(c->stream, g, c->ipz, twz, z, c->d_zt, c->zfs, c->ld, c->d_kx, c->d_kz, 0, NY + 2);
     if (int rc = check_launch(c, "zinv(rhs)")) return rc;
     if (int rc = pairs_x(c, pairs_of_fields(c), c->d_zt, 6)) return rc;
     // implicit solves: TH, U2, U1, U3 (for/channel.f:762-1029), independent,
@@ -1824,7 +1832,7 @@ static int les_substep(dgpu_ctx *c, int rk_step, double time, double temp1, doub
         set.cw[q] = pair_buf(c, 2 + 2 * q);
         set.gw[q] = pair_buf(c, 3 + 2 * q);
     }
-    dgpu::launch_les_cn(c->stream, g, set, m.nut, c->d_dy, c->d_dyf);
+    dgpu::launch_les_cn(c->stream, g, set, m.nut, m.w, c->d_dy, c->d_dyf);
     if (int rc = check_launch(c, "les_cn")) return rc;
     // COURANT on the physical velocity after the solves (for/channel.f:1037-1040)
     if (courant) {
@@ -1842,7 +1850,15 @@ static int les_substep(dgpu_ctx *c, int rk_step, double time, double temp1, doub
     if (int rc = check_launch(c, "zfwd(pairs)")) return rc;
     dgpu::RdArgs R;
     fill_rdargs(c, R, 1, temp4);
-    dgpu::launch_remdiv<double, double>(c->stream, R, P);
+    if (const int nw = seg_waves(c, NY, false)) {
+        // the segmented kernel in place: the solutions are in the state already
+        P.gs[dgpu::SYS_U1] = c->cu[0];
+        P.gs[dgpu::SYS_U2] = c->cu[1];
+        P.gs[dgpu::SYS_U3] = c->cu[2];
+        dgpu::launch_remdiv_seg<double, double>(c->stream, nw, R, P);
+    } else {
+        dgpu::launch_remdiv<double, double>(c->stream, R, P);
+    }
     return check_launch(c, "remdiv");
 }
 
@@ -2116,9 +2132,9 @@ int32_t dgpu_poisson_p_chan(dgpu_ctx *c)
         z.p[q] = c->cu[q % 3];
         z.dz[q] = q >= 3;
     }
-    dgpu::launch_zinv_src(c->stream, g, c->ipz, twz, z, c->d_wt, c->zfs, c->ld, c->d_kz, 0, g.ny + 2);
+    dgpu::launch_zinv_src(c->stream, g, c->ipz, twz, z, c->d_wt, c->zfs, c->ld, c->d_kx, c->d_kz, 0, g.ny + 2);
     if (int rc = check_launch(c, "zinv(poisson)")) return rc;
-    const dgpu::PairSrc src{{0, 2, -1, 3, 5}, {-1, -1, 1, -1, -1}, {1, -1, -1, 4, -1}, {-1, 0, 2, -1, -1}, 5};
+    const dgpu::PairSrc src{{0, 2, 1, 3, 5}, {1, 0, 2, 4, -1}, {0, 0, 1, 0, 0}, {0, 1, 1, 0, 0}, 5};
     if (int rc = pairs_x(c, src, c->d_wt, 0)) return rc;
     dgpu::PairDst pr{};
     for (int q = 0; q < 5; ++q) pr.p[q] = pair_buf(c, q);

@@ -72,10 +72,12 @@ __device__ __forceinline__ void piped_sweep(int j0, int dir, int n, Ld &&ld, Bod
 // DA, DB: planes in flight in sweeps A and B.  SIDE: the few low-mode
 // columns of the mixed path (one block): deeper prefetch.  TPF: the table
 // rows are fetched with the rest of a plane's inputs, DA/DB planes ahead,
-// instead of read (scalar loads) when the plane is processed.
+// instead of read (scalar loads) when the plane is processed.  RHS: rows
+// ja..ja+jn-1 of sweep A with no elimination (P.gs receives the right-hand
+// sides), no sweep B.
 template <typename T, int NTH, typename NLT, typename AT, typename PT, int DA = (sizeof(T) == 4 ? 6 : 3),
-          int DB = (sizeof(T) == 4 ? 16 : 8), bool SIDE = false, bool TPF = SIDE>
-__device__ __forceinline__ void cn_body(AT A, PT P, int bx)
+          int DB = (sizeof(T) == 4 ? 16 : 8), bool SIDE = false, bool TPF = SIDE, bool RHS = false>
+__device__ __forceinline__ void cn_body(AT A, PT P, int bx, int ja = 0, int jn = 0)
 {
     const Geo &g = A.g;
     const int q = wave_uniform(threadIdx.x >> 6);  // system of this wavefront
@@ -111,7 +113,10 @@ __device__ __forceinline__ void cn_body(AT A, PT P, int bx)
     const cx<T> *const p_cu1 = P.cu1;
     const cx<T> *const p_cu3 = P.cu3;
     const cx<T> *const p_cth = P.cth;
-    const bool rhs_only = A.rhs_only != 0;
+    if constexpr (!RHS) {
+        ja = 0;
+        jn = NY + 2;
+    }
 
     // ---------------- sweep A ----------------
     // Inputs of plane j are loaded four planes ahead (piped_sweep); every
@@ -121,7 +126,7 @@ __device__ __forceinline__ void cn_body(AT A, PT P, int bx)
             cx<T> fp, nl, cf, aux1, aux2, cp;
             double tr[10];  // TPF: this row's table entries, fetched ahead
         };
-        cx<T> fm = zero, f0 = fld[m];  // this system's field at j-1, j (j+1 comes in)
+        cx<T> fm = zero, f0 = fld[m + (long)ja * ps];  // this system's field at j-1, j (j+1 comes in)
         cx<T> thm = zero;              // CTH at j-1 (U2 buoyancy)
         cx<T> cpm = zero;              // CP at j-1 (U2 pressure)
         cx<T> gprev = zero;
@@ -130,8 +135,14 @@ __device__ __forceinline__ void cn_body(AT A, PT P, int bx)
         const bool has1 = (q != SYS_U2);
         const bool has2 = (q == SYS_TH0) || NTH;
         const bool hascp = (q != SYS_TH0);
+        if (RHS && ja > 0) {
+            const long o = m + (long)(ja - 1) * ps;
+            fm = fld[o];
+            if (has2) thm = a2p[o];
+            if (hascp) cpm = p_cp[o];
+        }
         piped_sweep<DA>(
-            0, +1, NY + 2,
+            ja, +1, jn,
             [&](int j) {
                 const long o = m + (long)j * ps;
                 InA in;
@@ -217,7 +228,7 @@ __device__ __forceinline__ void cn_body(AT A, PT P, int bx)
                     vec = make_cx<T>(cr.re + (wp * fp.re + w0 * f0.re + wm * fm.re),
                                      cr.im + (wp * fp.im + w0 * f0.im + wm * fm.im));
                 }
-                const cx<T> gj = (j == 0 || rhs_only) ? vec : fma_c(mult, gprev, vec);
+                const cx<T> gj = (j == 0 || RHS) ? vec : fma_c(mult, gprev, vec);
                 if (cfr) cf[o] = cfn;
                 gs[o] = gj;
                 gprev = gj;
@@ -227,9 +238,10 @@ __device__ __forceinline__ void cn_body(AT A, PT P, int bx)
                 cpm = cp0;
             });
     }
+    if constexpr (RHS) return;
     __syncthreads();
     // ---------------- sweep B ----------------
-    if (live && !rhs_only) {
+    if (live) {
         struct InB {
             cx<T> g;
             double ip, u, cpy;  // TPF: fetched ahead
@@ -273,6 +285,28 @@ __global__ void __launch_bounds__(256, 3) k_cn(CnArgs A, CnPtrs<T, NLT> P)
 {
     cn_body<T, NTH, NLT, const CnArgs, const CnPtrs<T, NLT>, (sizeof(T) == 4 ? 6 : 3), (sizeof(T) == 4 ? 16 : 8),
             false, sizeof(T) == 4>(A, P, xcd_contiguous(blockIdx.x, gridDim.x));
+}
+
+// Right-hand sides alone.  They need no recurrence, so the rows are cut into
+// runs of kRhsRows (one row in eight read twice, mostly from cache): one thread
+// a column took 100 us at 96x81x108, where it fills 38 CUs, and 0.85 ms at
+// 384x257x384; the runs take 26 us and 0.66 ms.
+constexpr int kRhsRows = 16;
+template <int NTH>
+__global__ void __launch_bounds__(256, 3) k_cn_rhs(CnArgs A, CnPtrs<double, double> P)
+{
+    const int ja = blockIdx.y * kRhsRows, jn = min(kRhsRows, A.g.ny + 2 - ja);
+    cn_body<double, NTH, double, const CnArgs, const CnPtrs<double, double>, 3, 8, false, false, true>(
+        A, P, xcd_contiguous(blockIdx.x, gridDim.x), ja, jn);
+}
+
+void launch_cn_rhs(hipStream_t s, const CnArgs &a, const CnPtrs<double, double> &p)
+{
+    const dim3 grid((unsigned)(((a.g.ps + 63) / 64 + 7) / 8 * 8), (a.g.ny + 2 + kRhsRows - 1) / kRhsRows);
+    if (a.g.nth == 0)
+        hipLaunchKernelGGL((k_cn_rhs<0>), grid, dim3(256), 0, s, a, p);
+    else
+        hipLaunchKernelGGL((k_cn_rhs<1>), grid, dim3(256), 0, s, a, p);
 }
 
 // The mixed path's low-mode columns: a block or two, so registers are free.

@@ -25,13 +25,14 @@ namespace dgpu {
 // kept slots straight from the state, the last stage writes Zt rows.
 // grid (column chunks, planes, fields), block W*T, LDS W*NZ values.
 // -------------------------------------------------------------------------
-// kzv (DZ only): null, or the input is multiplied by i KZ.
+// DZ only: with kzv the input is multiplied by i KZ, with inx i KX inx joins it.
 template <typename T, int E, typename TIN, bool CP, bool DZ = false>
 __device__ __forceinline__ void zinv_body(const IpLen &fz, const cx<T> *__restrict__ tw,
                                           const cx<TIN> *__restrict__ in, long in_fs, long in_ps, int mk,
                                           cx<T> *__restrict__ out, long out_fs, long out_ps, int ld, int j0, int nkz,
                                           int tnkz, int lw, int bx, int by, int bz,
-                                          const double *__restrict__ kzv = nullptr)
+                                          const double *__restrict__ kzv = nullptr,
+                                          const cx<TIN> *__restrict__ inx = nullptr, double kx = 0.0)
 {
     extern __shared__ unsigned char smem_raw[];
     cx<T> *lds = reinterpret_cast<cx<T> *>(smem_raw);
@@ -58,6 +59,10 @@ __device__ __forceinline__ void zinv_body(const IpLen &fz, const cx<T> *__restri
                     if (kzv) {
                         const TIN kz = TIN(kzv[max(s, 0)]);
                         v = make_cx<TIN>(-kz * v.im, kz * v.re);
+                    }
+                    if (inx) {
+                        const cx<TIN> y = inx[(long)j * in_ps + (long)max(s, 0) * mk + (col ? i : mk - 1)];
+                        v = make_cx<TIN>(v.re - TIN(kx) * y.im, v.im + TIN(kx) * y.re);
                     }
                 }
                 return (col && s >= 0) ? cvt_<T>(v) : make_cx<T>(0, 0);
@@ -103,14 +108,16 @@ template <int E, int PID>
 __global__ void __launch_bounds__(256) k_zinv_src(IpLen fz, const cx<double> *__restrict__ tw, ZSrc src, long in_ps,
                                                    int mk, cx<double> *__restrict__ out, long out_fs, long out_ps,
                                                    int ld, int j0, int nkz, int tnkz, int lw, int nchunks,
-                                                   int nplanes, const double *__restrict__ kzv)
+                                                   int nplanes, const double *__restrict__ kxv,
+                                                   const double *__restrict__ kzv)
 {
     int chunk, plane;
     if (!plane_chunk(blockIdx.x, nchunks, nplanes, chunk, plane)) return;
     const int f = blockIdx.z;
     zinv_body<double, E, double, PID != 0, true>(plan_ref<PID>(fz), tw, src.p[f], 0, in_ps, mk, out + f * out_fs, 0,
                                                  out_ps, ld, j0, nkz, tnkz, lw, chunk, plane, 0,
-                                                 src.dz[f] ? kzv : nullptr);
+                                                 src.dz[f] ? kzv : nullptr, src.x[f],
+                                                 kxv[min((chunk << lw) + (int)(threadIdx.x & ((1 << lw) - 1)), mk - 1)]);
 }
 
 // z forward (DIT) of one Wt field per output, no derivative: the kept slots
@@ -367,23 +374,23 @@ void launch_zfwd_nl_ip(hipStream_t s, const Geo &g, const IpLen &fz, const cx<T>
 
 template <int E, int PID>
 static void zinv_src_e(hipStream_t s, const Geo &g, const IpLen &fz, const cx<double> *tw, const ZSrc &src,
-                       cx<double> *out, long out_fs, int ld, const double *kz, int j0, int nplanes)
+                       cx<double> *out, long out_fs, int ld, const double *kx, const double *kz, int j0, int nplanes)
 {
     const int lw = z_lw(fz.t), W = 1 << lw, nchunks = (g.mk + W - 1) / W;
     hipLaunchKernelGGL((k_zinv_src<E, PID>), dim3((unsigned)(8 * nchunks * ((nplanes + 7) / 8)), 1, src.n),
                        dim3(W * fz.t), sizeof(cx<double>) * W * fz.n, s, fz, tw, src, g.ps, g.mk, out, out_fs,
-                       (long)g.nz * ld, ld, j0, g.nkz, g.tnkz, lw, nchunks, nplanes, kz);
+                       (long)g.nz * ld, ld, j0, g.nkz, g.tnkz, lw, nchunks, nplanes, kx, kz);
 }
 
 void launch_zinv_src(hipStream_t s, const Geo &g, const IpLen &fz, const cx<double> *tw, const ZSrc &src,
-                     cx<double> *out, long out_fs, int ld, const double *kz, int j0, int nplanes)
+                     cx<double> *out, long out_fs, int ld, const double *kx, const double *kz, int j0, int nplanes)
 {
     if (with_pid(const_plan_id(fz), ZPids<double>{}, [&](auto pc) {
             constexpr int P = decltype(pc)::value;
-            zinv_src_e<kConstPlanSpecs[P].e, P>(s, g, fz, tw, src, out, out_fs, ld, kz, j0, nplanes);
+            zinv_src_e<kConstPlanSpecs[P].e, P>(s, g, fz, tw, src, out, out_fs, ld, kx, kz, j0, nplanes);
         }))
         return;
-    DGPU_DISPATCH_IPE(fz.e, (zinv_src_e<EE, 0>(s, g, fz, tw, src, out, out_fs, ld, kz, j0, nplanes)));
+    DGPU_DISPATCH_IPE(fz.e, (zinv_src_e<EE, 0>(s, g, fz, tw, src, out, out_fs, ld, kx, kz, j0, nplanes)));
 }
 
 template <int E, int PID>

@@ -51,10 +51,6 @@ struct CnArgs {
     // stride nl_ps.  The mixed path runs its FP64 low-|k| columns this way.
     const int *map;
     long nl_ps;
-    // 1: sweep A only, with no elimination: the solve scratch receives each
-    // row's right-hand side and the field is left as it was (the LES path
-    // solves in physical space)
-    int rhs_only;
 };
 
 template <typename T, typename NLT = T>
@@ -198,6 +194,9 @@ size_t zip_lds_bytes(const IpLen &fz, size_t elem);
 
 template <typename T, typename NLT>
 void launch_cn(hipStream_t s, const CnArgs &a, const CnPtrs<T, NLT> &p);
+// The new CF and the right-hand sides alone: P.gs receives each row's, the
+// fields stay as they are (the LES path solves in physical space).
+void launch_cn_rhs(hipStream_t s, const CnArgs &a, const CnPtrs<double, double> &p);
 // The mixed path's low-mode columns (few lanes): deeper prefetch variants.
 template <typename T, typename NLT>
 void launch_cn_side(hipStream_t s, const CnArgs &a, const CnPtrs<T, NLT> &p);
@@ -253,9 +252,10 @@ void launch_apply_bc_vel(hipStream_t s, const Geo &g, cx<double> *cu1, cx<double
                          const int *codes, const double *c1, const double *dy, const double *dyf);
 
 // ---- pair planes (dgpu_pairs.hip): FP64 physical fields two by two ----
-// z backward of the kept modes of n fields, each plain or times i KZ
+// z backward of the kept modes of n fields, each p (dz: times i KZ), plus i KX x
+// where x is given
 struct ZSrc {
-    const cx<double> *p[8];
+    const cx<double> *p[8], *x[8];
     int dz[8];
     int n;
 };
@@ -264,9 +264,10 @@ struct ZDst {
     cx<double> *p[4];
     int n;
 };
-// real rows A = Z_a0 + i KX Z_a1 and B likewise of each pair (-1: none)
+// the real rows A and B of each pair: Zt fields a and b (b < 0: none), times
+// i KX with da, db
 struct PairSrc {
-    int a0[6], a1[6], b0[6], b1[6];
+    int a[6], b[6], da[6], db[6];
     int n;
 };
 struct PairDst {
@@ -278,7 +279,7 @@ struct PairOut {
     int n;
 };
 void launch_zinv_src(hipStream_t s, const Geo &g, const IpLen &fz, const cx<double> *tw, const ZSrc &src,
-                     cx<double> *out, long out_fs, int ld, const double *kz, int j0, int nplanes);
+                     cx<double> *out, long out_fs, int ld, const double *kx, const double *kz, int j0, int nplanes);
 void launch_zfwd_dst(hipStream_t s, const Geo &g, const IpLen &fz, const cx<double> *tw, const cx<double> *wt,
                      long wt_fs, int ld, const ZDst &dst, int j0, int nplanes);
 void launch_pairs_inv(hipStream_t s, const Geo &g, const IpLen &fx, const cx<double> *tw, int ld,
@@ -348,8 +349,9 @@ struct LesCnSet {
     const cx<double> *rhs[2];
     cx<double> *out[2], *cw[2], *gw[2];
 };
-void launch_les_cn(hipStream_t s, const Geo &g, const LesCnSet &set, const double *nut, const double *dy,
-                   const double *dyf);
+// w: per row [NY+2][4]: 1/(DYF(j-1) DY(j)), 1/(DY(j) DYF(j)), 1/(DY(j+1) DYF(j)), -
+void launch_les_cn(hipStream_t s, const Geo &g, const LesCnSet &set, const double *nut, const double *w,
+                   const double *dy, const double *dyf);
 void launch_les_vmax(hipStream_t s, const Geo &g, const cx<double> *p0, const cx<double> *p1, double *out);
 void launch_les_eps(hipStream_t s, const Geo &g, const cx<double> *p0, const cx<double> *p1, const double *nut,
                     const double *dy, const double *dyf, double *out);

@@ -157,25 +157,33 @@ __global__ void k_les_bc_put(Geo g, cx<double> *__restrict__ p0, cx<double> *__r
 // values are on their way.  tab[j*8 + {0..6}]: 1/DYF, 1/DY, 1/(2 DYF),
 // DYF(j-1)/(2 DY), DYF(j)/(2 DY), -2 C^2 DELTA^2 on GYF, on GY.
 // force: the SGS force alone (dgpu_les_chan), no products and no scalar.
-// 384x257x384: 2.29 ms (5.6 GB: six pairs in, NU_T and eight row fields out),
-// bound by its registers (256, two waves per SIMD) rather than HBM; it replaces
-// the x kernel (1.30 ms), nine plane transforms (2.9 ms) and seven pointwise
+// 384x257x384: 1.92 ms (5.6 GB: six pairs in, NU_T and eight row fields out, 2.9
+// TB/s; three waves per SIMD; 2.29 ms with two positions a thread, 256 registers
+// and 44 of them spilled); it replaces the x kernel (1.30 ms), nine plane transforms (2.9 ms) and seven pointwise
 // kernels (2.9 ms) of the Fortran-layout form.  Substep 18.1 -> 10.0 ms.
 // -------------------------------------------------------------------------
-template <int E, int NTH, int PID, bool WIDE>
-__global__ void __launch_bounds__(WIDE ? 768 : 256) __attribute__((amdgpu_waves_per_eu(2))) k_les_prod(IpLen frt, const cx<double> *__restrict__ twg, int mk, int ld,
+constexpr int kStash = 8;
+template <int E, int NTH, int PID, int LM, bool WIDE>
+__global__ void __launch_bounds__(WIDE ? 768 : 384) __attribute__((amdgpu_waves_per_eu(3))) k_les_prod(IpLen frt, const cx<double> *__restrict__ twg, int mk_rt, int ld,
                                                   LesProd a)
 {
-    constexpr int npo = XCount<NTH>::npo, NP = (E + npo - 1) / npo;
+    constexpr int npo = XCount<NTH>::npo, NP = (E + LM * npo - 1) / (LM * npo);
     const IpLen &fx = plan_ref<PID>(frt);
     extern __shared__ unsigned char smem_raw[];
     cx<double> *const fb = reinterpret_cast<cx<double> *>(smem_raw);
     const int nx = fx.n, TT = fx.t, S = fx.nstages, NY = a.ny;
+    const int mk = PID != 0 ? nx / 3 + 1 : mk_rt;
     const int tid = threadIdx.x, nthr = blockDim.x, zr = a.zr;
+    // the first zr * npo * T threads run the transforms
     const int pg = tid / TT, zs = pg / npo, p = pg - zs * npo;
+    const bool tr = zs < zr;
     int th = tid - pg * TT;
     cx<double> *tw = fb + (long)zr * npo * nx;
     double *kxs = reinterpret_cast<double *>(tw + fx.twn);
+    // row m's products and fluxes wait here for the next plane (kStash values a
+    // position, each lane its own): in registers they spilled, 2.2 GB of scratch
+    // traffic a launch
+    double *stash = kxs + mk + tid;
     for (int e = tid; e < fx.twn; e += nthr) tw[e] = twg[e];
     for (int e = tid; e < mk; e += nthr) kxs[e] = a.kx[e];
     const int zi = blockIdx.x * zr + zs;
@@ -197,8 +205,14 @@ __global__ void __launch_bounds__(WIDE ? 768 : 256) __attribute__((amdgpu_waves_
         ls[k] = in ? zq * npo * nx + ip_swz(fx, pos) : -1;
     }
     struct Keep {
-        double pu, pv, pw, pt, su, sw, s11, s13, s33, s22, s12, s23, dxt, dzt, nut, t12, t23, f1, f3, ft, q, p3, p4;
+        double pu, pv, pw, pt, su, sw, s11, s13, s33, s22, s12, s23, t12, t23;
     } K[NP];
+    enum { Q_P3, Q_P4, Q_F1, Q_F3, Q_FT, Q_Q, Q_X8, Q_X9 };
+    double own[WIDE ? NP : 1][kStash];  // rows of more than 384 threads have no LDS left for it
+    auto Q = [&](int k, int q) -> double & {
+        if constexpr (WIDE) return own[k][q];
+        else return stash[(k * kStash + q) * nthr];
+    };
     cx<double> c0[NP], c1[NP], c2[NP], c3[NP], c4[NP], c5[NP], n0[NP];
     auto load = [&](int plane) {
 #pragma unroll
@@ -282,7 +296,7 @@ __global__ void __launch_bounds__(WIDE ? 768 : 256) __attribute__((amdgpu_waves_
             const double q = 0.25 * sq(v + P.pv);
             if (out) {  // the products of plane j
                 double x1 = P.pu * P.pu, x0 = P.pw * P.pu, x2 = P.pw * P.pw;
-                double x5 = (f1 - P.f1) * Tj[2], x6 = (f3 - P.f3) * Tj[2];
+                double x5 = (f1 - Q(k, Q_F1)) * Tj[2], x6 = (f3 - Q(k, Q_F3)) * Tj[2];
                 if (stress) {
                     const double S = sqrt(2.0 * sq(P.s11) + 4.0 * sq(0.5 * (s12 + P.s12) - dub_j - dub) +
                                           4.0 * sq(P.s13) + 2.0 * sq(P.s22) +
@@ -297,25 +311,30 @@ __global__ void __launch_bounds__(WIDE ? 768 : 256) __attribute__((amdgpu_waves_
                 if (ls[k] >= 0) {
                     cx<double> *f = fb + ls[k];
                     f[0 * nx] = make_cx(x1, x5);
-                    f[1 * nx] = make_cx(P.p3, (q - P.q) * Tj[1]);
+                    f[1 * nx] = make_cx(Q(k, Q_P3), (q - Q(k, Q_Q)) * Tj[1]);
                     f[2 * nx] = make_cx(x0, x6);
-                    f[3 * nx] = make_cx(P.p4, x2);
+                    f[3 * nx] = make_cx(Q(k, Q_P4), x2);
                     if constexpr (NTH > 0) {
-                        f[4 * nx] = make_cx(P.pt * P.pu - P.nut * P.dxt, (ft - P.ft) * Tj[2]);
-                        f[5 * nx] = make_cx(P.pt * P.pw - P.nut * P.dzt, 0.0);
+                        f[4 * nx] = make_cx(Q(k, Q_X8), (ft - Q(k, Q_FT)) * Tj[2]);
+                        f[5 * nx] = make_cx(Q(k, Q_X9), 0.0);
                     }
-                    if (on[k]) a.nut[j * pp + off[k]] = P.nut;
                 }
             }
             P.pu = u; P.pv = v; P.pw = w; P.pt = t;
             P.su = Us; P.sw = Ws;
             P.s11 = s11; P.s13 = s13; P.s33 = s33; P.s22 = s22; P.s12 = s12; P.s23 = s23;
+            P.t12 = t12; P.t23 = t23;
+            if (on[k] && m >= ja && m <= jb) a.nut[m * pp + off[k]] = nut;
+            Q(k, Q_P3) = p3;
+            Q(k, Q_P4) = p4;
+            Q(k, Q_F1) = f1;
+            Q(k, Q_F3) = f3;
+            Q(k, Q_Q) = q;
             if constexpr (NTH > 0) {
-                P.dxt = c4[k].im;
-                P.dzt = c5[k].re;
+                Q(k, Q_FT) = ft;
+                Q(k, Q_X8) = t * u - nut * c4[k].im;
+                Q(k, Q_X9) = t * w - nut * c5[k].re;
             }
-            P.nut = nut; P.t12 = t12; P.t23 = t23;
-            P.f1 = f1; P.f3 = f3; P.ft = ft; P.q = q; P.p3 = p3; P.p4 = p4;
         }
         dub_j = dub;
         dwb_j = dwb;
@@ -328,16 +347,16 @@ __global__ void __launch_bounds__(WIDE ? 768 : 256) __attribute__((amdgpu_waves_
         }
         if (out) {
             asm volatile("" : "+v"(th));  // keeps the stages' index arithmetic out of the sweep's registers
-            cx<double> *row = fb + ((long)zs * npo + p) * nx;
+            __builtin_assume(th >= 0 && th < TT);
+            cx<double> *row = fb + (tr ? (long)zs * npo + p : 0) * nx;
             stage_loop<PID != 0>(0, S - 1, [&](int s) {
-                ip_stage_row<double, E, -1, false>(row, fx, S - 1 - s, tw, th);
+                if (tr) ip_stage_row<double, E, -1, false>(row, fx, S - 1 - s, tw, th);
                 row_sync();
             });
             cx<double> *o0 = a.wt + ((long)j * a.nz + min(zi, a.nz - 1)) * ld;
             const long wf = a.wt_fs;
             const double h = 0.5 / nx;
-            x_split<double, E>(fx, row, tw, th, mk, [&](int kp, cx<double> Zk, cx<double> Zn) {
-                if (!zvalid) return;
+            if (tr && zvalid) x_split<double, E>(fx, row, tw, th, mk, [&](int kp, cx<double> Zk, cx<double> Zn) {
                 const cx<double> Xa = make_cx((Zk.re + Zn.re) * h, (Zk.im - Zn.im) * h);
                 const cx<double> Xb = make_cx((Zk.im + Zn.im) * h, -(Zk.re - Zn.re) * h);
                 const double kx = kxs[kp];
@@ -357,27 +376,31 @@ __global__ void __launch_bounds__(WIDE ? 768 : 256) __attribute__((amdgpu_waves_
     }
 }
 
-// WIDE: rows of more than 256 threads (NX above 512 or so)
-template <int E, int NTH, int PID, bool WIDE = false>
+// LM: threads a position is shared out over, in units of the transforms' own
+// (2: one position a thread up to 12 values a transform thread).  WIDE: rows of
+// more than 384 threads (NX above 512 or so), one unit.
+template <int E, int NTH, int PID, int LM = (E > XCount<NTH>::npo ? 2 : 1), bool WIDE = false>
 static void les_prod_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<double> *tw, int ld, LesProd a)
 {
     constexpr int npo = XCount<NTH>::npo;
     if constexpr (!WIDE && PID == 0)
-        if (npo * fx.t > 256) return les_prod_e<E, NTH, PID, true>(s, g, fx, tw, ld, a);
+        if (LM * npo * fx.t > 384) return les_prod_e<E, NTH, PID, 1, true>(s, g, fx, tw, ld, a);
     // short rows are packed as in the fused x kernel
-    const size_t row = sizeof(cx<double>) * (size_t)fx.n * npo;
+    const size_t stash =  // a z row's
+        WIDE ? 0 : sizeof(double) * kStash * ((E + LM * npo - 1) / (LM * npo)) * LM * npo * fx.t;
+    const size_t row = sizeof(cx<double>) * (size_t)fx.n * npo + stash;
     const size_t fixed = sizeof(cx<double>) * fx.twn + sizeof(double) * g.mk;
     a.zr = 1;
-    while (2 * a.zr * npo * fx.t <= 256 && 2 * a.zr <= g.nz && fixed + 2 * a.zr * row <= 64 * 1024) a.zr *= 2;
-    const int threads = a.zr * npo * fx.t;
+    while (2 * a.zr * LM * npo * fx.t <= 384 && 2 * a.zr <= g.nz && fixed + 2 * a.zr * row <= 64 * 1024) a.zr *= 2;
+    const int threads = a.zr * LM * npo * fx.t;
     const size_t lds = fixed + a.zr * row;
     if (lds > 64 * 1024)
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_les_prod<E, NTH, PID, WIDE>),
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_les_prod<E, NTH, PID, LM, WIDE>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     const long rows = (g.nz + a.zr - 1) / a.zr;
-    a.chunk = sweep_rule(rows, a.jhi - a.jlo + 1, kernel_slots(&k_les_prod<E, NTH, PID, WIDE>, threads, lds));
+    a.chunk = sweep_rule(rows, a.jhi - a.jlo + 1, kernel_slots(&k_les_prod<E, NTH, PID, LM, WIDE>, threads, lds));
     const int nchunks = (a.jhi - a.jlo + a.chunk) / a.chunk;
-    hipLaunchKernelGGL((k_les_prod<E, NTH, PID, WIDE>), dim3((unsigned)rows, nchunks), dim3(threads), lds, s, fx, tw, g.mk,
+    hipLaunchKernelGGL((k_les_prod<E, NTH, PID, LM, WIDE>), dim3((unsigned)rows, nchunks), dim3(threads), lds, s, fx, tw, g.mk,
                        ld, a);
 }
 
@@ -437,26 +460,19 @@ void launch_les_nut_out(hipStream_t s, const Geo &g, const double *nut, const in
 // temp2 d/dy(nut du/dy) (for/channel.f:628-659, 748-760) joins the right-hand
 // side r: on GYF rows with NU_T on the faces (U1, U3, TH), or on GY rows with
 // NU_T averaged onto the GYF faces (U2).
-__device__ __forceinline__ void les_row(const LesCn &a, int j, const double *__restrict__ dy,
-                                        const double *__restrict__ dyf, double n0, double np, double nm, double u0,
+// w: the row's metric weights (launch_les_cn).
+__device__ __forceinline__ void les_row(const LesCn &a, int j, const double *__restrict__ w,
+                                        const double *__restrict__ dy, const double *__restrict__ dyf, double n0, double np, double nm, double u0,
                                         double up, double um, double r, double &L, double &D, double &U, double &V)
 {
     const int NY = a.ny;
     L = 0.0; D = 1.0; U = 0.0; V = 0.0;
     if (j >= a.jlo && j <= a.jhi) {
         const double c = a.cmol, t2 = a.temp2;
-        double wm, wp, em, ep;  // molecular and eddy weights of rows j-1 and j+1
-        if (a.sys == LES_SYS_U2) {
-            wm = 1.0 / (dyf[j - 1] * dy[j]);
-            wp = 1.0 / (dyf[j] * dy[j]);
-            em = t2 * 0.5 * (n0 + nm) * wm;
-            ep = t2 * 0.5 * (n0 + np) * wp;
-        } else {
-            wm = 1.0 / (dy[j] * dyf[j]);
-            wp = 1.0 / (dy[j + 1] * dyf[j]);
-            em = t2 * n0 * wm;
-            ep = t2 * np * wp;
-        }
+        const bool v = a.sys == LES_SYS_U2;
+        // metric weights, and the eddy weights of rows j-1 and j+1
+        const double wm = v ? w[4 * j] : w[4 * j + 1], wp = v ? w[4 * j + 1] : w[4 * j + 2];
+        const double em = t2 * (v ? 0.5 * (n0 + nm) : n0) * wm, ep = t2 * (v ? 0.5 * (n0 + np) : np) * wp;
         L = -(c * wm + em);
         U = -(c * wp + ep);
         D = 1.0 + (c * wp + ep) + (c * wm + em);
@@ -489,14 +505,139 @@ __device__ __forceinline__ void les_row(const LesCn &a, int j, const double *__r
     }
 }
 
-// THOMAS_REAL (for/mpi.f:630-809) down the columns of a pair plane, one thread
-// a real column of one of the pair's two systems (grid.y: the pair).  The
+// The solves in segments: a real column (a double column of a pair plane) is
+// cut into 32 segments of RM rows or fewer.  A lane eliminates its segment's
+// rows [a, b] downwards,
+//   x(j) = g(j) - c(j) x(j+1) - f(j) x(a-1),
+// and folds them upwards to the same form for x(a) in x(b+1) and x(a-1); the
+// two equations of every segment form a block-tridiagonal system that one lane
+// a column solves through LDS, and each lane back-substitutes its rows.  The
+// matrix differs from column to column (NU_T), so nothing is precomputed; rows
+// stay in registers: each value is read once and written once (56 B a point and
+// pair against 120 B of the sweeps below, whose scratch makes a round trip).
+// 16 columns (128 B of a row) x 32 segments a block.
+// 384x257x384: 1.98 -> 1.46 ms; 96x81x108, where one thread a column filled
+// 162 CUs: 89 -> 40 us.
+template <int RM>
+__global__ void __launch_bounds__(512) k_les_cn_seg(Geo g, LesCnSet set, const double *__restrict__ nut,
+                                                    const double *__restrict__ w, const double *__restrict__ dy,
+                                                    const double *__restrict__ dyf)
+{
+    constexpr int NS = 32, NC = 16;
+    __shared__ double eq[NS][6][NC];  // x(a): G, C, F; x(b): g, c, f -- then x(b+1), x(a-1)
+    const int col = threadIdx.x & (NC - 1), seg = threadIdx.x / NC;
+    const long n = 2L * g.nx * g.nz;  // doubles a pair plane (a multiple of 16: NX, NZ are even and NX*NZ*2 >= 32)
+    const long e0 = (long)blockIdx.x * NC + col;
+    const bool on = e0 < n;
+    const long e = on ? e0 : n - 1;
+    const LesCn a = set.a[blockIdx.y][e & 1];
+    const bool live = on && a.sys >= 0;
+    const double *__restrict__ rhs = reinterpret_cast<const double *>(set.rhs[blockIdx.y]) + e;
+    double *__restrict__ out = reinterpret_cast<double *>(set.out[blockIdx.y]) + e;
+    const double *__restrict__ nt = nut + (e >> 1);
+    const long nn = n >> 1;
+    const int NY = g.ny, R = (NY + 2 + NS - 1) / NS, ja = seg * R, jb = min(ja + R - 1, NY + 1);
+    double G[RM], C[RM], F[RM];
+    double ga = 0.0, ca = -1.0, fa = 0.0, gb = 0.0, cb = 0.0, fb = -1.0;  // a segment without rows passes both through
+    if (live && ja <= jb) {
+        double um = ja > 0 ? out[(ja - 1) * n] : 0.0, u0 = out[ja * n];
+        double nm = ja > 0 ? nt[(ja - 1) * nn] : 0.0, n0 = nt[ja * nn];
+#pragma unroll
+        for (int r = 0; r < RM; ++r) {
+            const int j = ja + r;
+            if (j <= jb) {
+                const int jn = min(j + 1, NY + 1);
+                const double up = out[jn * n], np = nt[jn * nn];
+                double L, D, U, V;
+                les_row(a, j, w, dy, dyf, n0, np, nm, u0, up, um, rhs[j * n], L, D, U, V);
+                if (r > 0) {
+                    D = D - L * C[r - 1];
+                    V = V - L * G[r - 1];
+                }
+                const double rd = D != 0.0 ? 1.0 / D : 0.0;
+                C[r] = U * rd;
+                G[r] = V * rd;
+                F[r] = r > 0 ? -L * F[r - 1] * rd : L * rd;
+                um = u0;
+                u0 = up;
+                nm = n0;
+                n0 = np;
+            }
+        }
+        bool first = true;
+#pragma unroll
+        for (int r = RM - 1; r >= 0; --r) {
+            if (ja + r <= jb) {
+                if (first) {
+                    ga = gb = G[r];
+                    ca = cb = C[r];
+                    fa = fb = F[r];
+                    first = false;
+                } else {
+                    ga = G[r] - C[r] * ga;
+                    fa = F[r] - C[r] * fa;
+                    ca = -C[r] * ca;
+                }
+            }
+        }
+    }
+    eq[seg][0][col] = ga;
+    eq[seg][1][col] = ca;
+    eq[seg][2][col] = fa;
+    eq[seg][3][col] = gb;
+    eq[seg][4][col] = cb;
+    eq[seg][5][col] = fb;
+    __syncthreads();
+    if (seg == 0) {
+        // x(b) of the segment before = al - be x(a) of this one
+        double al = 0.0, be = 0.0;
+        for (int s = 0; s < NS; ++s) {
+            const double Ga = eq[s][0][col], Ca = eq[s][1][col], Fa = eq[s][2][col];
+            const double Gb = eq[s][3][col], Cb = eq[s][4][col], Fb = eq[s][5][col];
+            const double rw = 1.0 / (1.0 - Fa * be);
+            const double ga_ = (Ga - Fa * al) * rw, de = Ca * rw;  // x(a) = ga_ - de x(b+1)
+            eq[s][0][col] = ga_;
+            eq[s][1][col] = de;
+            eq[s][2][col] = al;
+            eq[s][3][col] = be;
+            const double t = Fb * be;
+            al = Gb - Fb * al + t * ga_;
+            be = Cb + t * de;
+        }
+        double X = 0.0;
+        for (int s = NS - 1; s >= 0; --s) {
+            const double xa = eq[s][0][col] - eq[s][1][col] * X;
+            const double Y = eq[s][2][col] - eq[s][3][col] * xa;
+            eq[s][4][col] = X;
+            eq[s][5][col] = Y;
+            X = xa;
+        }
+    }
+    __syncthreads();
+    if (live && ja <= jb) {
+        double x = eq[seg][4][col];
+        const double y = eq[seg][5][col];
+#pragma unroll
+        for (int r = RM - 1; r >= 0; --r) {
+            const int j = ja + r;
+            if (j <= jb) {
+                x = G[r] - C[r] * x - F[r] * y;
+                if (j >= a.clo && j <= a.chi) out[j * n] = x;
+            }
+        }
+    }
+}
+
+// Columns of more than 542 rows: THOMAS_REAL (for/mpi.f:630-809) down the
+// columns of a pair plane, one thread a real column of one of the pair's two
+// systems (grid.y: the pair).  The
 // forward sweep leaves U/B and G/B of every row in the scratch planes; the
 // back substitution reads only those.  Rows clo..chi of the field are
 // overwritten.  A column is read and written by its own thread only, every
 // read of the field before the first write.
 __global__ void __launch_bounds__(256) k_les_cn(Geo g, LesCnSet set, const double *__restrict__ nut,
-                                                const double *__restrict__ dy, const double *__restrict__ dyf)
+                                                const double *__restrict__ w, const double *__restrict__ dy,
+                                                const double *__restrict__ dyf)
 {
     const long n = 2L * g.nx * g.nz;  // doubles a pair plane
     const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -514,7 +655,7 @@ __global__ void __launch_bounds__(256) k_les_cn(Geo g, LesCnSet set, const doubl
     double bprev = 1.0, cprev = 0.0, gprev = 0.0;
     for (int j = 0; j <= NY + 1; ++j) {
         double L, D, U, V;
-        les_row(a, j, dy, dyf, n0, np, nm, u0, up, um, rhs[j * n], L, D, U, V);
+        les_row(a, j, w, dy, dyf, n0, np, nm, u0, up, um, rhs[j * n], L, D, U, V);
         if (j > 0) {
             const double m = -L / bprev;
             D = D + m * cprev;
@@ -541,11 +682,23 @@ __global__ void __launch_bounds__(256) k_les_cn(Geo g, LesCnSet set, const doubl
     }
 }
 
-void launch_les_cn(hipStream_t s, const Geo &g, const LesCnSet &set, const double *nut, const double *dy,
-                   const double *dyf)
+// Rows a segment: the fewest registers that hold a 32nd of the column.
+void launch_les_cn(hipStream_t s, const Geo &g, const LesCnSet &set, const double *nut, const double *w,
+                   const double *dy, const double *dyf)
 {
     const long n = 2L * g.nx * g.nz;
-    hipLaunchKernelGGL(k_les_cn, dim3((unsigned)((n + 255) / 256), 2), dim3(256), 0, s, g, set, nut, dy, dyf);
+    const int rows = (g.ny + 2 + 31) / 32;
+    const dim3 grid((unsigned)((n + 15) / 16), 2);
+    if (rows <= 3)
+        hipLaunchKernelGGL((k_les_cn_seg<3>), grid, dim3(512), 0, s, g, set, nut, w, dy, dyf);
+    else if (rows <= 5)
+        hipLaunchKernelGGL((k_les_cn_seg<5>), grid, dim3(512), 0, s, g, set, nut, w, dy, dyf);
+    else if (rows <= 9)
+        hipLaunchKernelGGL((k_les_cn_seg<9>), grid, dim3(512), 0, s, g, set, nut, w, dy, dyf);
+    else if (rows <= 17)
+        hipLaunchKernelGGL((k_les_cn_seg<17>), grid, dim3(512), 0, s, g, set, nut, w, dy, dyf);
+    else
+        hipLaunchKernelGGL(k_les_cn, dim3((unsigned)((n + 255) / 256), 2), dim3(256), 0, s, g, set, nut, w, dy, dyf);
 }
 
 // Per-plane maxima of |U1|, |U2|, |U3| on physical planes 1..NY into
