@@ -29,16 +29,41 @@ __device__ __forceinline__ cx<double> ik(double k, cx<double> a) { return make_c
 
 }  // namespace
 
-__global__ void __launch_bounds__(256) k_stats(Geo g, const cx<double> *__restrict__ cu1,
+// A plane has one block of 16 waves.  Blocks go to the eight XCDs in turn; each
+// XCD gets a run of planes, so the rows j-1 and j+1 a block reads are found in
+// its L2, where its neighbours are reading them too (256x193x256: 52 us; 77 with planes
+// dealt out in turn, 85 with four waves a block as well).
+constexpr int kStatThreads = 1024, kStatWaves = kStatThreads / 64;
+__device__ __forceinline__ int stat_plane(int b, int ny) { return (b & 7) * ((ny + 7) >> 3) + (b >> 3); }
+
+// red[q][0] = the block's sum of acc[q]
+template <int N>
+__device__ __forceinline__ void block_sums(double (&acc)[N], double (&red)[N][kStatWaves])
+{
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        for (int h = 32; h > 0; h >>= 1) acc[q] += __shfl_down(acc[q], h);
+        if ((threadIdx.x & 63) == 0) red[q][threadIdx.x >> 6] = acc[q];
+    }
+    __syncthreads();
+    if (threadIdx.x < N) {
+        double v = red[threadIdx.x][0];
+        for (int wv = 1; wv < kStatWaves; ++wv) v += red[threadIdx.x][wv];
+        red[threadIdx.x][0] = v;
+    }
+    __syncthreads();
+}
+
+__global__ void __launch_bounds__(kStatThreads) k_stats(Geo g, const cx<double> *__restrict__ cu1,
                                                const cx<double> *__restrict__ cu2, const cx<double> *__restrict__ cu3,
                                                const cx<double> *__restrict__ cp, const cx<double> *__restrict__ cth,
                                                const double *__restrict__ dy, const double *__restrict__ dyf,
                                                const double *__restrict__ gyf, const double *__restrict__ kxv,
                                                const double *__restrict__ kzv, double *__restrict__ out)
 {
-    __shared__ double red[kSums][256];
-    const int j = 1 + blockIdx.x;
-    const int NY = g.ny;
+    __shared__ double red[kSums][kStatWaves];
+    const int NY = g.ny, j = 1 + stat_plane(blockIdx.x, NY);
+    if (j > NY) return;
     const long ps = g.ps;
     double acc[kSums];
 #pragma unroll
@@ -46,8 +71,8 @@ __global__ void __launch_bounds__(256) k_stats(Geo g, const cx<double> *__restri
     const double ayj = dyf[j - 1] / (2.0 * dy[j]), bmj = dyf[j] / (2.0 * dy[j]);
     const double i2f = 1.0 / (2.0 * dyf[j]);
     const double igt = 1.0 / (gyf[j + 1] - gyf[j - 1]);
-    for (long m = threadIdx.x; m < ps; m += blockDim.x) {
-        const int K = (int)(m / g.mk), i = (int)(m - (long)K * g.mk);
+    for (int m = threadIdx.x; m < (int)ps; m += kStatThreads) {
+        const int K = m / g.mk, i = m - K * g.mk;
         const bool mean = (m == 0);
         const double w = (i == 0) ? 1.0 : 2.0;
         const double kx = kxv[i], kz = kzv[K];
@@ -82,16 +107,7 @@ __global__ void __launch_bounds__(256) k_stats(Geo g, const cx<double> *__restri
             acc[S_PE] += w * (abs2(ik(kx, t0)) + abs2(ax(igt, tp - tm)) + abs2(ik(kz, t0)));
         }
     }
-#pragma unroll
-    for (int q = 0; q < kSums; ++q) red[q][threadIdx.x] = acc[q];
-    __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) {
-#pragma unroll
-            for (int q = 0; q < kSums; ++q) red[q][threadIdx.x] += red[q][threadIdx.x + h];
-        }
-        __syncthreads();
-    }
+    block_sums<kSums>(acc, red);
     if (threadIdx.x == 0) {
         auto put = [&](int q, double v) { out[(long)q * NY + (j - 1)] = v; };
         const double ume = cu1[(long)j * ps].re, umem = cu1[(long)(j - 1) * ps].re;
@@ -135,22 +151,22 @@ __global__ void __launch_bounds__(256) k_stats(Geo g, const cx<double> *__restri
 //   q = 8     sum over fluctuating modes of w |CU2(j+1) - CU2(j-1)|^2,
 //             j = 2..NY-1 (dv/dy), 0 elsewhere
 //   q = 9     Re CU2(0,0,j) (vme)
-__global__ void __launch_bounds__(256) k_tke(Geo g, const cx<double> *__restrict__ cu1,
+__global__ void __launch_bounds__(kStatThreads) k_tke(Geo g, const cx<double> *__restrict__ cu1,
                                              const cx<double> *__restrict__ cu2, const cx<double> *__restrict__ cu3,
                                              const double *__restrict__ kxv, const double *__restrict__ kzv,
                                              double *__restrict__ out)
 {
     constexpr int kT = 9;
-    __shared__ double red[kT][256];
-    const int j = 1 + blockIdx.x;
-    const int NY = g.ny;
+    __shared__ double red[kT][kStatWaves];
+    const int NY = g.ny, j = 1 + stat_plane(blockIdx.x, NY);
+    if (j > NY) return;
     const long ps = g.ps;
     double acc[kT];
 #pragma unroll
     for (int q = 0; q < kT; ++q) acc[q] = 0.0;
     const bool dv = (j >= 2 && j <= NY - 1);
-    for (long m = threadIdx.x; m < ps; m += blockDim.x) {
-        const int K = (int)(m / g.mk), i = (int)(m - (long)K * g.mk);
+    for (int m = threadIdx.x; m < (int)ps; m += kStatThreads) {
+        const int K = m / g.mk, i = m - K * g.mk;
         const bool mean = (m == 0);
         const double w = (i == 0) ? 1.0 : 2.0;
         const double kx2 = kxv[i] * kxv[i], kz2 = kzv[K] * kzv[K];
@@ -170,16 +186,7 @@ __global__ void __launch_bounds__(256) k_tke(Geo g, const cx<double> *__restrict
             if (dv) acc[8] += w * abs2(cu2[m + (long)(j + 1) * ps] - cu2[m + (long)(j - 1) * ps]);
         }
     }
-#pragma unroll
-    for (int q = 0; q < kT; ++q) red[q][threadIdx.x] = acc[q];
-    __syncthreads();
-    for (int h = 128; h > 0; h >>= 1) {
-        if ((int)threadIdx.x < h) {
-#pragma unroll
-            for (int q = 0; q < kT; ++q) red[q][threadIdx.x] += red[q][threadIdx.x + h];
-        }
-        __syncthreads();
-    }
+    block_sums<kT>(acc, red);
     if (threadIdx.x == 0) {
 #pragma unroll
         for (int q = 0; q < kT; ++q) out[(long)q * NY + (j - 1)] = red[q][0];
@@ -190,14 +197,14 @@ __global__ void __launch_bounds__(256) k_tke(Geo g, const cx<double> *__restrict
 void launch_tke(hipStream_t s, const Geo &g, const cx<double> *cu1, const cx<double> *cu2, const cx<double> *cu3,
                 const double *kx, const double *kz, double *out)
 {
-    hipLaunchKernelGGL(k_tke, dim3(g.ny), dim3(256), 0, s, g, cu1, cu2, cu3, kx, kz, out);
+    hipLaunchKernelGGL(k_tke, dim3(8 * ((g.ny + 7) / 8)), dim3(kStatThreads), 0, s, g, cu1, cu2, cu3, kx, kz, out);
 }
 
 void launch_stats(hipStream_t s, const Geo &g, const cx<double> *cu1, const cx<double> *cu2, const cx<double> *cu3,
                   const cx<double> *cp, const cx<double> *cth, const double *dy, const double *dyf,
                   const double *gyf, const double *kx, const double *kz, double *out)
 {
-    hipLaunchKernelGGL(k_stats, dim3(g.ny), dim3(256), 0, s, g, cu1, cu2, cu3, cp, cth, dy, dyf, gyf, kx, kz, out);
+    hipLaunchKernelGGL(k_stats, dim3(8 * ((g.ny + 7) / 8)), dim3(kStatThreads), 0, s, g, cu1, cu2, cu3, cp, cth, dy, dyf, gyf, kx, kz, out);
 }
 
 // The per-plane statistics of dgpu_stats_chan_noalloc: DGPU_NSTAT rows of
