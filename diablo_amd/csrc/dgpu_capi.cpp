@@ -1569,8 +1569,15 @@ static int fused_waves(const dgpu_ctx *c, int ny)
     if (!c->colnw) return 0;
     // tall columns; with the FP32 state also the short ones the fused kernel
     // cuts into 16 segments (NY <= 142): the 64-member ensemble 17.13k ->
-    // 17.65k Mpts*substeps/s against the two kernels
-    const bool auto_on = (ny >= 160 && (c->f32state || c->colnw == 8)) || (c->f32state && ny + 2 <= 144);
+    // 17.65k Mpts*substeps/s against the two kernels.  Any column where the
+    // modes alone give a block or more per CU (one block is 32 of them): the
+    // barriers of one block then hide behind another's loads (8 waves, a step
+    // of 256x97x256 in FP64 1826 -> 1637 us, 384x129x384 5165 -> 4772,
+    // 384x150x384 with the FP32 state 3200 -> 2936; even at 192x97x192, and
+    // 474 -> 478 and 230 -> 301 at 128 and 64).
+    const bool many = c->g.ps >= 8192 && c->colnw == 8;
+    const bool auto_on =
+        many || (ny >= 160 && (c->f32state || c->colnw == 8)) || (c->f32state && ny + 2 <= 144);
     const bool want = c->colfuse == 1 || (c->colfuse < 0 && auto_on);
     return (want && fused_fits(c, ny, c->colnw)) ? c->colnw : 0;
 }

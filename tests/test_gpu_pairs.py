@@ -88,3 +88,42 @@ def test_poisson_sizes(oracle_mod, size, deck):
     errs, bad = compare_states(cfg, g.state(), o.state(), 1e-11, fields=("CP",))
     say(errs)
     assert not bad, bad
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_many_mode_column_default(precision):
+    """From 8192 modes up the default column stage is the fused kernel at any
+    NY it fits, below that not (NY = 150: the case that neither rule of short
+    and tall columns covers).  FP64: within 1e-11 of the two kernels.  FP32
+    state: no further from the FP64 run than 1.5 times the two kernels,
+    plus 1e-7."""
+    from diablo_amd import gpu
+
+    def run(n, precision, shape=None):
+        cfg = case.channel_case(n, 150, n, kick=0.05, dt=1e-4)
+        say(n, precision, shape)
+        g = gpu.GpuChannel(cfg, precision=precision)
+        if shape is not None:
+            g.set_column_shape(*shape)
+        fused = g.column_fused()
+        g.initialize(*case.initial_physical(cfg))
+        g.step(1)
+        g.synchronize()
+        s = g.state()
+        g.close()
+        return cfg, fused, s
+
+    assert not run(162, precision)[1]
+    cfg, fused, one = run(192, precision)
+    assert fused
+    _, fused, two = run(192, precision, (8, 0))
+    assert not fused
+    if precision == "fp64":
+        errs, bad = compare_states(cfg, one, two, 1e-11, ["CU1", "CU2", "CU3", "CP"])
+        assert not bad, errs
+        return
+    ref = run(192, "fp64", (8, 0))[2]
+    e1 = compare_states(cfg, one, ref, 1.0, ["CU1", "CU2", "CU3", "CP"])[0]
+    e2 = compare_states(cfg, two, ref, 1.0, ["CU1", "CU2", "CU3", "CP"])[0]
+    say("fused", e1, "two", e2)
+    assert all(e1[k] <= 1.5 * e2[k] + 1e-7 for k in e1)
