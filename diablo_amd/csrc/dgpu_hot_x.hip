@@ -89,7 +89,9 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
     };
     // Backward stage 0 from the registers: spectrum of A + iB with the
     // Hermitian halves of both rows (C2R ignores Im of the DC term).
+    const bool lin = CP && ip_bits_apart<E, R0>(fx, 0);
     auto dif0 = [&](cx<T> *row) {
+        const int s0 = ip_swz(fx, th);
         ip_stage<T, E, R0, +1, true>(
             fx, 0, tw, th,
             [&](int idx, int f) {
@@ -104,17 +106,20 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
                 }
                 return make_cx<T>(A.re - B.im, A.im + B.re);
             },
-            [&](int, int pos, cx<T> v) { row[ip_swz(fx, pos)] = v; });
+            [&](int idx, int pos, cx<T> v) {
+                row[lin ? ip_slot(fx, s0, TT * (idx / R0) + L0 * (idx % R0)) : ip_swz(fx, pos)] = v;
+            });
     };
     // Forward stage 0 of product pair row r (plane j): groups th and L0 - th
     // (0 and L0/2 for th == 0) hold Z(k') and Z(NX - k') of their frequencies.
     auto dit_out = [&](const cx<T> *row, int r, int j) {
         const int ga = th, gb = th == 0 ? TT : L0 - th;
         cx<T> va[R0], vb[R0];
+        const int sa = ip_swz(fx, ga), sb = ip_swz(fx, gb);
 #pragma unroll
         for (int q = 0; q < R0; ++q) {
-            va[q] = row[ip_swz(fx, ga + q * L0)];
-            vb[q] = row[ip_swz(fx, gb + q * L0)];
+            va[q] = row[lin ? ip_slot(fx, sa, q * L0) : ip_swz(fx, ga + q * L0)];
+            vb[q] = row[lin ? ip_slot(fx, sb, q * L0) : ip_swz(fx, gb + q * L0)];
         }
         ip_group<T, R0, -1, false>(va, tw + fx.twoff[0], ga);
         ip_group<T, R0, -1, false>(vb, tw + fx.twoff[0], gb);
@@ -219,7 +224,7 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
     if (pro) dif0(slot_row(pro_plane, pro_pair));
     __syncthreads();
     stage_loop<CP>(1, S, [&](int s) {
-        if (pro) ip_stage_row<T, E, +1, true>(slot_row(pro_plane, pro_pair), fx, s, tw, th);
+        if (pro) ip_stage_row<T, E, +1, true, CP>(slot_row(pro_plane, pro_pair), fx, s, tw, th);
         __syncthreads();
     });
     if (dif_row) {
@@ -263,8 +268,8 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
                 asm volatile("" : "+v"(th));
                 __builtin_assume(th >= 0 && th < TT);
             }
-            if (inv) ip_stage_row<T, E, +1, true>(drow, fx, s + 1, tw, th);
-            if (fwd) ip_stage_row<T, E, -1, false>(frow, fx, S - 1 - s, tw, th);
+            if (inv) ip_stage_row<T, E, +1, true, CP>(drow, fx, s + 1, tw, th);
+            if (fwd) ip_stage_row<T, E, -1, false, CP>(frow, fx, S - 1 - s, tw, th);
             row_sync();
         });
         if (fwd) dit_out(frow, p - npi, j - 1);

@@ -350,7 +350,7 @@ __global__ void __launch_bounds__(WIDE ? 768 : 384) __attribute__((amdgpu_waves_
             __builtin_assume(th >= 0 && th < TT);
             cx<double> *row = fb + (tr ? (long)zs * npo + p : 0) * nx;
             stage_loop<PID != 0>(0, S - 1, [&](int s) {
-                if (tr) ip_stage_row<double, E, -1, false>(row, fx, S - 1 - s, tw, th);
+                if (tr) ip_stage_row<double, E, -1, false, PID != 0>(row, fx, S - 1 - s, tw, th);
                 row_sync();
             });
             cx<double> *o0 = a.wt + ((long)j * a.nz + min(zi, a.nz - 1)) * ld;

@@ -101,7 +101,7 @@ __global__ void __launch_bounds__(128) k_pairs_inv(IpLen frt, const cx<double> *
             [&](int, int pos, cx<double> v) { row[ip_swz(fx, pos)] = v; });
         row_sync();
         stage_loop<PID != 0>(1, S - 1, [&](int s) {
-            ip_stage_row<double, E, +1, true>(row, fx, s, tw, th);
+            ip_stage_row<double, E, +1, true, PID != 0>(row, fx, s, tw, th);
             row_sync();
         });
         cx<double> *out = dst.p[o.pair] + ((long)(j0 + o.plane) * nz + o.zp) * nx + th;
@@ -149,7 +149,7 @@ __global__ void __launch_bounds__(128) k_pairs_fwd(IpLen frt, const cx<double> *
         });
         row_sync();
         stage_loop<PID != 0>(1, S - 1, [&](int s) {
-            ip_stage_row<double, E, -1, false>(row, fx, S - 1 - s, tw, th);
+            ip_stage_row<double, E, -1, false, PID != 0>(row, fx, S - 1 - s, tw, th);
             row_sync();
         });
         cx<double> *o0 = wt + ((long)(j0 + o.plane) * nz + o.zp) * ld;
