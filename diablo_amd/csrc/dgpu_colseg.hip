@@ -162,7 +162,7 @@ __device__ __forceinline__ void cn_rhs(int q, const CnMode<T> &K, TB &&tb, cx<T>
     }
     cfn = cfn + nlv;
     if (tb(L_ISBC) != T(0)) {
-        vec = K.is00 ? make_cx<T>(tb(L_BC00), 0) : zero;
+        vec = K.is00 ? make_cx<T>(tb(L_BC00), 0) : cx<T>{};
     } else {
         cx<T> cr = f0;
         if (K.rk_gt1) cr = cfma(K.temp3, cfo, cr);
@@ -246,16 +246,16 @@ __device__ __forceinline__ void cn_seg_solve(AT A, PT P, int bx, int q, cx<T> (&
             in.fp = fld[o + (j <= NY ? ps : 0)];
             const cx<NLT> nv = nl[gm + (long)j * nps];
             in.nl = make_cx<T>(T(nv.re), T(nv.im));
-            in.cf = rk_gt1 ? cf[o] : zero;
-            in.aux1 = has1 ? a1p[o] : zero;
-            in.aux2 = has2 ? a2p[o] : zero;
-            in.cp = hascp ? P.cp[o] : zero;
+            in.cf = rk_gt1 ? cf[o] : cx<T>{};
+            in.aux1 = has1 ? a1p[o] : cx<T>{};
+            in.aux2 = has2 ? a2p[o] : cx<T>{};
+            in.cp = hascp ? P.cp[o] : cx<T>{};
             return in;
         };
         const long oa = m + (long)a * ps;
-        cx<T> fm = a >= 1 ? fld[oa - ps] : zero, f0 = fld[oa];
-        cx<T> thm = (a >= 1 && has2) ? a2p[oa - ps] : zero;
-        cx<T> cpm = (a >= 1 && hascp) ? P.cp[oa - ps] : zero;
+        cx<T> fm = a >= 1 ? fld[oa - ps] : cx<T>{}, f0 = fld[oa];
+        cx<T> thm = (a >= 1 && has2) ? a2p[oa - ps] : cx<T>{};
+        cx<T> cpm = (a >= 1 && hascp) ? P.cp[oa - ps] : cx<T>{};
         cx<T> gl = zero;
         T cprod = T(1);
         In cur = load(a);
@@ -268,10 +268,10 @@ __device__ __forceinline__ void cn_seg_solve(AT A, PT P, int bx, int q, cx<T> (&
                 const T mult = t[L_MULT];
                 const bool isbc = t[L_ISBC] != T(0);
                 const bool cfr = t[L_CFR] != T(0);
-                const cx<T> fp = (j <= NY) ? cur.fp : zero;
+                const cx<T> fp = (j <= NY) ? cur.fp : cx<T>{};
                 const bool use = cfr || !isbc;
-                const cx<T> nlv = use ? cur.nl : zero;
-                const cx<T> cfo = use ? cur.cf : zero;
+                const cx<T> nlv = use ? cur.nl : cx<T>{};
+                const cx<T> cfo = use ? cur.cf : cx<T>{};
                 const cx<T> aux2 = cur.aux2, cp0 = cur.cp;
                 cx<T> cfn, vec;
                 cn_rhs<T, NTH>(q, K, [&](int k) { return t[k]; }, f0, fm, fp, cur.aux1, aux2, thm, cp0, cpm, nlv, cfo,
@@ -641,6 +641,9 @@ __device__ __forceinline__ void cn3_solve(const CnArgs &A, const CnPtrs<T, NLT> 
 
     // ---- forward, local ----
     if (rows) {
+        // "cond ? array[i] : cx<T>{}" selects values; with a named zero it
+        // selects between two addresses, one of them on the stack, and the
+        // load becomes a flat one in two halves (FP64 1.20 -> 1.17 ms)
         struct In3 {
             cx<T> fp[3], nl[3], cf[3], th, cp;
         };
@@ -652,9 +655,9 @@ __device__ __forceinline__ void cn3_solve(const CnArgs &A, const CnPtrs<T, NLT> 
                 in.fp[q] = fldp[q][o + (j <= NY ? ps : 0)];
                 const cx<NLT> nv = P.nl[q][gm + (long)j * nps];
                 in.nl[q] = make_cx<T>(T(nv.re), T(nv.im));
-                in.cf[q] = K.rk_gt1 ? cfp[q][o] : zero;
+                in.cf[q] = K.rk_gt1 ? cfp[q][o] : cx<T>{};
             }
-            in.th = NTH ? P.cth[o] : zero;
+            in.th = NTH ? P.cth[o] : cx<T>{};
             in.cp = P.cp[o];
             return in;
         };
@@ -663,13 +666,13 @@ __device__ __forceinline__ void cn3_solve(const CnArgs &A, const CnPtrs<T, NLT> 
         T cprod[3];
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
-            fm[q] = a >= 1 ? fldp[q][oa - ps] : zero;
+            fm[q] = a >= 1 ? fldp[q][oa - ps] : cx<T>{};
             f0[q] = fldp[q][oa];
             gl[q] = zero;
             cprod[q] = T(1);
         }
-        cx<T> thm = (a >= 1 && NTH) ? P.cth[oa - ps] : zero;
-        cx<T> cpm = a >= 1 ? P.cp[oa - ps] : zero;
+        cx<T> thm = (a >= 1 && NTH) ? P.cth[oa - ps] : cx<T>{};
+        cx<T> cpm = a >= 1 ? P.cp[oa - ps] : cx<T>{};
 #pragma unroll
         for (int r = 0; r < RMAX; ++r) {
             const int j = a + r;
@@ -681,12 +684,12 @@ __device__ __forceinline__ void cn3_solve(const CnArgs &A, const CnPtrs<T, NLT> 
                     const T mult = tb(L_MULT);
                     const bool isbc = tb(L_ISBC) != T(0);
                     const bool cfr = tb(L_CFR) != T(0);
-                    const cx<T> fp = (j <= NY) ? cur.fp[q] : zero;
+                    const cx<T> fp = (j <= NY) ? cur.fp[q] : cx<T>{};
                     const bool use = cfr || !isbc;
-                    const cx<T> nlv = use ? cur.nl[q] : zero;
-                    const cx<T> cfo = use ? cur.cf[q] : zero;
+                    const cx<T> nlv = use ? cur.nl[q] : cx<T>{};
+                    const cx<T> cfo = use ? cur.cf[q] : cx<T>{};
                     // U1's partner is CU3, U3's CU1 (their own rows here)
-                    const cx<T> aux1 = q == 0 ? f0[1] : q == 1 ? f0[0] : zero;
+                    const cx<T> aux1 = q == 0 ? f0[1] : q == 1 ? f0[0] : cx<T>{};
                     cx<T> cfn, vec;
                     cn_rhs<T, NTH>(q, K, tb, f0[q], fm[q], fp, aux1, cur.th, thm, cur.cp, cpm, nlv, cfo, cfn, vec);
                     gl[q] = (r == 0) ? vec : cfma(mult, gl[q], vec);
@@ -697,7 +700,7 @@ __device__ __forceinline__ void cn3_solve(const CnArgs &A, const CnPtrs<T, NLT> 
 #pragma unroll
                 for (int q = 0; q < 3; ++q) {
                     fm[q] = f0[q];
-                    f0[q] = (j <= NY) ? cur.fp[q] : zero;
+                    f0[q] = (j <= NY) ? cur.fp[q] : cx<T>{};
                 }
                 thm = cur.th;
                 cpm = cur.cp;
@@ -828,7 +831,7 @@ __device__ __forceinline__ void colfused_body(const CnArgs &A, const RdArgs &Rd,
     __syncthreads();  // the carry arrays are reused below
     if (rows) X2[seg * MPW + ml] = u2s[0];
     __syncthreads();
-    const cx<T> u2nx = (rows && seg + 1 < nseg) ? X2[(seg + 1) * MPW + ml] : zero;  // U2*(b+1)
+    const cx<T> u2nx = (rows && seg + 1 < nseg) ? X2[(seg + 1) * MPW + ml] : cx<T>{};  // U2*(b+1)
 
     // ---- divergence of U* and the Poisson elimination, rows max(a,1)..min(b,NY) ----
     int s = 0, i = 0;
@@ -848,8 +851,16 @@ __device__ __forceinline__ void colfused_body(const CnArgs &A, const RdArgs &Rd,
     // U2* of the row after a + r: the next register, or the next segment's first row
     auto u2up = [&](int r) -> cx<T> { return (a + r < b) ? u2s[r + 1 < RMAX ? r + 1 : r] : u2nx; };
     cx<T> yv[RMAX];
-    T mr[RMAX], fr[RMAX];
+    T mr[RMAX], fr[RMAX];  // the Poisson multipliers; 1/pivot, then U/B
+    constexpr bool early = sizeof(T) == 8;  // see below
     if (rows) {
+        // FP64: all rows' coefficients in flight at once (rows clamped to
+        // 1..NY; 384 x 257 x 384: 1.17 -> 1.12 ms).  FP32 has no registers
+        // left for them at four waves per SIMD (0.67 -> 0.71 ms).
+        if constexpr (early) {
+#pragma unroll
+            for (int r = 0; r < RMAX; ++r) mr[r] = pm(max(1, min(min(a + r, b), NY)));
+        }
         cx<T> hl = zero;
         T cprod = T(1);
         bool first = true;
@@ -865,13 +876,17 @@ __device__ __forceinline__ void colfused_body(const CnArgs &A, const RdArgs &Rd,
                     vec = make_cx<T>((d1.re + (c2p.re - c2.re) * idf) + d3.re,
                                      (d1.im + (c2p.im - c2.im) * idf) + d3.im);
                 }
-                const T mu = j >= 2 ? pm(j) : T(0);
+                const T mu = j >= 2 ? (early ? mr[r] : pm(j)) : T(0);
                 hl = first ? vec : cfma(mu, hl, vec);
                 cprod = first ? mu : cprod * mu;
                 first = false;
                 yv[r] = hl;
                 mr[r] = mu;
             }
+        }
+        if constexpr (early) {
+#pragma unroll
+            for (int r = 0; r < RMAX; ++r) fr[r] = pv(max(1, min(min(a + r, b), NY)));
         }
         GL[seg * MPW + ml] = hl;
         Cm[seg * MPW + ml] = cprod;
@@ -897,7 +912,7 @@ __device__ __forceinline__ void colfused_body(const CnArgs &A, const RdArgs &Rd,
         for (int r = RMAX - 1; r >= 0; --r) {
             const int j = a + r;
             if (j <= b && j >= 1 && j <= NY) {
-                const T ip = pv(j);
+                const T ip = early ? fr[r] : pv(j);
                 const T u = (j == 1) ? u1row : T(Rd.rd[(long)j * 4 + 0]);
                 fr[r] = -u * ip;
                 if (first) {
