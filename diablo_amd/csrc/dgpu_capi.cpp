@@ -547,9 +547,16 @@ int32_t dgpu_create(const dgpu_params *p, dgpu_ctx **out)
         // FP64 kernels spill above 12 values per thread; the FP32 z kernels
         // are faster at 12 too (NZ = 384: four radix stages at twice the
         // resident columns beat three stages of 24 values)
-        const int emax = 12;
-        if (!dgpu::ip_plan_x(g.nx, ex ? std::atoi(ex) : 0, c->mixed ? 16 : 12, 64, c->ipx) ||
+        const int emax = 12, xmax = c->mixed ? 16 : 12;
+        if (!dgpu::ip_plan_x(g.nx, ex ? std::atoi(ex) : 0, xmax, 64, c->ipx) ||
             !dgpu::ip_plan_z(g.nz, ez ? std::atoi(ez) : 0, emax, c->ipz)) {
+            delete c;
+            return DGPU_E_ARG;
+        }
+        // no FP64 x kernel is built for 16 values per thread: such a request
+        // takes the default plan
+        if (c->ipx.e > xmax && !dgpu::ip_plan_x(g.nx, 0, xmax, 64, c->ipx) &&
+            !dgpu::ip_plan_x(g.nx, 0, xmax, 128, c->ipx)) {
             delete c;
             return DGPU_E_ARG;
         }
