@@ -16,6 +16,15 @@
 // Everything done on pair planes is pointwise in x and z, so the order never
 // matters (pair_slot gives it where natural order is wanted).
 //
+// The two rows of a pair are transformed together, and the round-off of a
+// complex transform is that of its larger half.  Halves whose magnitudes are
+// more than 2^10 apart (U3 and a scalar in a unit of its own) are brought to
+// 2^10 by a power of two, which is exact, and taken back where they come apart,
+// so what one field adds to the other's round-off is bounded: beside a passive
+// scalar of 1e6 the LES substep's CU3 was off by 1.3e-13 of its maximum, 3e-15
+// for a scalar of 1.  Nearer halves stay as they are: bringing U2 up to U1, whose
+// maximum is its mean, costs U1's fluctuations four times their round-off.
+//
 // Both kernels move 16 B per pair point and 16 B per kept row value: 384x257x384,
 // 6 pairs back in 1.23 ms (5.3 GB, 4.3 TB/s), 2 pairs forward in 0.43 (2.0 GB,
 // 4.7 TB/s), near the rate of a copy; three waves per SIMD hide the loads (at two,
@@ -48,6 +57,49 @@ __device__ __forceinline__ RowOf row_of(long r, int nz, int nplanes, long nrows)
     return o;
 }
 
+// Largest magnitudes so far of the values of rows A and B, as the high words
+// of the doubles (ordered as the values are; NaN and infinity above all).
+struct PairMax {
+    int a = 0, b = 0;
+    __device__ __forceinline__ static int hi(double x) { return __double2hiint(x) & 0x7fffffff; }
+    __device__ __forceinline__ void take_a(double x) { a = max(a, hi(x)); }
+    __device__ __forceinline__ void take_b(double x) { b = max(b, hi(x)); }
+};
+
+// Row B goes in times `up`, the halves come out times a and b: `up` is the
+// power of two that brings the larger of the rows' largest values down to 2^10
+// times the other (1 where they are nearer, or one is not finite), and a row of
+// zeros comes out as zeros.
+struct PairScale {
+    double up, a, b;
+};
+__device__ __forceinline__ double pow2(int k) { return __hiloint2double((k + 1023) << 20, 0); }
+
+// From every thread of the row: TT lanes of a wave, or through the two words ex
+// (zero on entry) of a row that does not divide one.
+__device__ __forceinline__ PairScale pair_balance(PairMax m, int TT, bool wave_rows, int *ex)
+{
+    int ea = m.a >> 20, eb = m.b >> 20;
+    if (wave_rows) {
+        int e = (ea << 16) | eb;  // two halves of 11 bits
+        for (int h = TT >> 1; h > 0; h >>= 1) {
+            const int o = __shfl_xor(e, h);
+            e = (max(e >> 16, o >> 16) << 16) | max(e & 0xffff, o & 0xffff);
+        }
+        ea = e >> 16;
+        eb = e & 0xffff;
+    } else {
+        atomicMax(&ex[0], ea);
+        atomicMax(&ex[1], eb);
+        __syncthreads();
+        ea = ex[0];
+        eb = ex[1];
+    }
+    const bool scaled = ea != 0 && eb != 0 && ea != 0x7ff && eb != 0x7ff;
+    const int d = scaled ? ea - eb : 0, k = max(-1000, min(1000, d - max(-10, min(10, d))));
+    return {pow2(k), ea ? 1.0 : 0.0, eb ? pow2(-k) : 0.0};
+}
+
 }  // namespace
 
 template <int E, int PID>
@@ -67,8 +119,10 @@ __global__ void __launch_bounds__(128) k_pairs_inv(IpLen frt, const cx<double> *
     cx<double> *row = reinterpret_cast<cx<double> *>(smem_raw) + p * nx;
     cx<double> *tw = reinterpret_cast<cx<double> *>(smem_raw) + rb * nx;
     double *kxs = reinterpret_cast<double *>(tw + fx.twn);
+    int *ex = reinterpret_cast<int *>(kxs + mk) + 2 * p;
     for (int e = tid; e < fx.twn; e += blockDim.x) tw[e] = twg[e];
     for (int e = tid; e < mk; e += blockDim.x) kxs[e] = kxv[e];
+    if (th == 0) ex[0] = ex[1] = 0;
     __syncthreads();
     const bool wave_rows = (64 % TT) == 0;
     auto row_sync = [&]() {
@@ -80,23 +134,38 @@ __global__ void __launch_bounds__(128) k_pairs_inv(IpLen frt, const cx<double> *
         const long at = ((long)(j0 + o.plane) * nz + o.zp) * ld;
         const cx<double> *za = zt + src.a[o.pair] * zt_fs + at, *zb = zt + max(src.b[o.pair], 0) * zt_fs + at;
         const bool hasb = src.b[o.pair] >= 0, da = src.da[o.pair], db = src.db[o.pair];
-        // stage 0: the spectrum of a + i b from the Hermitian halves of both
-        // rows; C2R ignores Im of the DC term
+        // the Hermitian halves of both rows; C2R ignores Im of the DC term
+        cx<double> A[E], B[E];
+        PairMax m;
+        ip_groups<E, R0>(fx, 0, th, [&](int u, int b0, int) {
+#pragma unroll
+            for (int q = 0; q < R0; ++q) {
+                const int f = b0 + q * fx.span[0];
+                const int kk = f < mk ? f : (f > nx - mk ? nx - f : -1), kc = max(kk, 0);
+                cx<double> a = za[kc], b = hasb ? zb[kc] : make_cx(0.0, 0.0);
+                const double kx = kxs[kc];
+                if (da) a = make_cx(-kx * a.im, kx * a.re);
+                if (db) b = make_cx(-kx * b.im, kx * b.re);
+                if (kk < 0) a = b = make_cx(0.0, 0.0);
+                if (f == 0) a.im = b.im = 0.0;
+                if (f > nx - mk) {
+                    a.im = -a.im;
+                    b.im = -b.im;
+                }
+                m.take_a(a.re);
+                m.take_a(a.im);
+                m.take_b(b.re);
+                m.take_b(b.im);
+                A[u * R0 + q] = a;
+                B[u * R0 + q] = b;
+            }
+        });
+        const PairScale sc = pair_balance(m, TT, wave_rows, ex);
+        // stage 0: the spectrum of a + i b
         ip_stage<double, E, R0, +1, true>(
             fx, 0, tw, th,
-            [&](int, int f) {
-                const int kk = f < mk ? f : (f > nx - mk ? nx - f : -1), kc = max(kk, 0);
-                cx<double> A = za[kc], B = hasb ? zb[kc] : make_cx(0.0, 0.0);
-                const double kx = kxs[kc];
-                if (da) A = make_cx(-kx * A.im, kx * A.re);
-                if (db) B = make_cx(-kx * B.im, kx * B.re);
-                if (kk < 0) A = B = make_cx(0.0, 0.0);
-                if (f == 0) A.im = B.im = 0.0;
-                if (f > nx - mk) {
-                    A.im = -A.im;
-                    B.im = -B.im;
-                }
-                return make_cx(A.re - B.im, A.im + B.re);
+            [&](int idx, int) {
+                return make_cx(A[idx].re - sc.up * B[idx].im, A[idx].im + sc.up * B[idx].re);
             },
             [&](int, int pos, cx<double> v) { row[ip_swz(fx, pos)] = v; });
         row_sync();
@@ -110,9 +179,10 @@ __global__ void __launch_bounds__(128) k_pairs_inv(IpLen frt, const cx<double> *
             ip_stage<double, E, R, +1, true>(
                 fx, S - 1, tw, th, [&](int, int pos) { return row[ip_swz(fx, pos)]; },
                 [&](int idx, int, cx<double> v) {
-                    if (o.ok) out[idx * TT] = v;
+                    if (o.ok) out[idx * TT] = make_cx(v.re * sc.a, v.im * sc.b);
                 });
         });
+        if (!wave_rows && th == 0) ex[0] = ex[1] = 0;
         row_sync();
     }
 }
@@ -131,7 +201,9 @@ __global__ void __launch_bounds__(128) k_pairs_fwd(IpLen frt, const cx<double> *
     __builtin_assume(th >= 0 && th < TT);
     cx<double> *row = reinterpret_cast<cx<double> *>(smem_raw) + p * nx;
     cx<double> *tw = reinterpret_cast<cx<double> *>(smem_raw) + rb * nx;
+    int *ex = reinterpret_cast<int *>(tw + fx.twn) + 2 * p;
     for (int e = tid; e < fx.twn; e += blockDim.x) tw[e] = twg[e];
+    if (th == 0) ex[0] = ex[1] = 0;
     __syncthreads();
     const bool wave_rows = (64 % TT) == 0;
     auto row_sync = [&]() {
@@ -141,10 +213,20 @@ __global__ void __launch_bounds__(128) k_pairs_fwd(IpLen frt, const cx<double> *
     for (int k = 0; k < reps; ++k) {
         const RowOf o = row_of(((long)blockIdx.x * reps + k) * rb + p, nz, nplanes, nrows);
         const cx<double> *in = src.p[o.pair] + ((long)(j0 + o.plane) * nz + o.zp) * nx + th;
+        cx<double> v[E];
+        PairMax m;
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = in[e * TT];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            m.take_a(v[e].re);
+            m.take_b(v[e].im);
+        }
+        const PairScale sc = pair_balance(m, TT, wave_rows, ex);
         with_radix<E>(fx.radix[S - 1], [&](auto rc) {
             constexpr int R = decltype(rc)::value;
             ip_stage<double, E, R, -1, false>(
-                fx, S - 1, tw, th, [&](int idx, int) { return in[idx * TT]; },
+                fx, S - 1, tw, th, [&](int idx, int) { return make_cx(v[idx].re, v[idx].im * sc.up); },
                 [&](int, int pos, cx<double> v) { row[ip_swz(fx, pos)] = v; });
         });
         row_sync();
@@ -154,12 +236,13 @@ __global__ void __launch_bounds__(128) k_pairs_fwd(IpLen frt, const cx<double> *
         });
         cx<double> *o0 = wt + ((long)(j0 + o.plane) * nz + o.zp) * ld;
         const int fa = out.a[o.pair], fb = out.b[o.pair];
-        const double h = 0.5 / nx;
+        const double ha = 0.5 / nx * sc.a, hb = 0.5 / nx * sc.b;
         x_split<double, E>(fx, row, tw, th, mk, [&](int kp, cx<double> Zk, cx<double> Zn) {
             if (!o.ok) return;
-            if (fa >= 0) o0[fa * wt_fs + kp] = make_cx((Zk.re + Zn.re) * h, (Zk.im - Zn.im) * h);
-            if (fb >= 0) o0[fb * wt_fs + kp] = make_cx((Zk.im + Zn.im) * h, -(Zk.re - Zn.re) * h);
+            if (fa >= 0) o0[fa * wt_fs + kp] = make_cx((Zk.re + Zn.re) * ha, (Zk.im - Zn.im) * ha);
+            if (fb >= 0) o0[fb * wt_fs + kp] = make_cx((Zk.im + Zn.im) * hb, -(Zk.re - Zn.re) * hb);
         });
+        if (!wave_rows && th == 0) ex[0] = ex[1] = 0;
         row_sync();
     }
 }
@@ -181,7 +264,7 @@ PairGrid pair_grid(const IpLen &fx, int mk, long nrows)
     const long groups = (nrows + q.rb - 1) / q.rb;
     q.reps = (int)std::min<long>(8, std::max<long>(1, groups / 2048));
     q.blocks = (groups + q.reps - 1) / q.reps;
-    q.lds = sizeof(cx<double>) * ((size_t)q.rb * fx.n + fx.twn) + sizeof(double) * mk;
+    q.lds = sizeof(cx<double>) * ((size_t)q.rb * fx.n + fx.twn) + sizeof(double) * mk + 2 * sizeof(int) * q.rb;
     return q;
 }
 
