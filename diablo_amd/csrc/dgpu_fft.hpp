@@ -55,6 +55,20 @@ DGPU_HD cx<T> cmul(cx<T> a, cx<T> b)
 {
     return make_cx(a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re);
 }
+// a b + c, rounded once
+DGPU_HD double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+DGPU_HD float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+// cmul with the fused product named.  FIX below: where a sum of two products
+// leaves open which of them is fused into it, the code says which.  The
+// compiler otherwise chooses anew in every copy of a function, and the planes
+// that the x kernel transforms before its sweep, in it, in a batch or on a
+// compile-time plan differ in the last bit.
+template <typename T>
+DGPU_HD cx<T> cmul_fix(cx<T> a, cx<T> b)
+{
+#pragma clang fp contract(off)
+    return make_cx(fma_(a.re, b.re, -(a.im * b.im)), fma_(a.im, b.re, a.re * b.im));
+}
 template <typename T>
 DGPU_HD cx<T> scale(cx<T> a, T s) { return make_cx(a.re * s, a.im * s); }
 template <typename T>
@@ -84,7 +98,7 @@ DGPU_HD int div_magic(int t, unsigned magic)
     return magic ? (int)(((unsigned long long)(unsigned)t * magic) >> 32) : t;
 }
 
-template <typename T, int R, int SIGN>
+template <typename T, int R, int SIGN, bool FIX = false>
 DGPU_HD void butterfly(cx<T> *v)
 {
     if constexpr (R == 2) {
@@ -136,8 +150,15 @@ DGPU_HD void butterfly(cx<T> *v)
         butterfly<T, 3, SIGN>(o);
         const T h = T(0.5);
         const T s = T(SIGN) * T(0.86602540378443864676372317075294);
-        const cx<T> o1 = make_cx(h * o[1].re - s * o[1].im, h * o[1].im + s * o[1].re);     // o1 * w6
-        const cx<T> o2 = make_cx(-h * o[2].re - s * o[2].im, -h * o[2].im + s * o[2].re);   // o2 * w6^2
+        cx<T> o1 = make_cx(h * o[1].re - s * o[1].im, h * o[1].im + s * o[1].re);     // o1 * w6
+        cx<T> o2 = make_cx(-h * o[2].re - s * o[2].im, -h * o[2].im + s * o[2].re);   // o2 * w6^2
+        if constexpr (FIX) {
+#pragma clang fp contract(off)
+            o1 = make_cx(fma_(h, o[1].re, -(s * o[1].im)),
+                         SIGN > 0 ? fma_(s, o[1].re, h * o[1].im) : fma_(h, o[1].im, s * o[1].re));
+            o2 = make_cx(SIGN > 0 ? fma_(-h, o[2].re, -(s * o[2].im)) : fma_(-s, o[2].im, -h * o[2].re),
+                         fma_(s, o[2].re, -h * o[2].im));
+        }
         v[0] = e[0] + o[0];
         v[3] = e[0] - o[0];
         v[1] = e[1] + o1;
@@ -207,7 +228,7 @@ DGPU_HD int ip_swz(const IpLen &f, int pos)
 
 // Twiddle + butterfly of one group (values v[0..R-1] at positions
 // base + q L_i); tw points at the stage's table, k is the group offset.
-template <typename T, int R, int SIGN, bool DIF>
+template <typename T, int R, int SIGN, bool DIF, bool FIX = false>
 DGPU_HD void ip_group(cx<T> *v, const cx<T> *__restrict__ tw, int k)
 {
     cx<T> w[R];
@@ -218,12 +239,12 @@ DGPU_HD void ip_group(cx<T> *v, const cx<T> *__restrict__ tw, int k)
     }
     if (!DIF) {
 #pragma unroll
-        for (int q = 1; q < R; ++q) v[q] = cmul(v[q], w[q]);
+        for (int q = 1; q < R; ++q) v[q] = FIX ? cmul_fix(v[q], w[q]) : cmul(v[q], w[q]);
     }
-    butterfly<T, R, SIGN>(v);
+    butterfly<T, R, SIGN, FIX>(v);
     if (DIF) {
 #pragma unroll
-        for (int q = 1; q < R; ++q) v[q] = cmul(v[q], w[q]);
+        for (int q = 1; q < R; ++q) v[q] = FIX ? cmul_fix(v[q], w[q]) : cmul(v[q], w[q]);
     }
 }
 
@@ -245,7 +266,7 @@ DGPU_HD void ip_groups(const IpLen &f, int i, int th, F &&fn)
 // One stage with arbitrary sources and sinks: ld(idx, pos) gives the value at
 // position pos (idx = u*R + q is its slot in this thread's E values),
 // st(idx, pos, v) takes the result.  All loads come before any store.
-template <typename T, int E, int R, int SIGN, bool DIF, class Ld, class St>
+template <typename T, int E, int R, int SIGN, bool DIF, bool FIX = false, class Ld, class St>
 DGPU_HD void ip_stage(const IpLen &f, int i, const cx<T> *__restrict__ tw, int th, Ld &&ld, St &&st)
 {
     constexpr int NB = E / R;
@@ -262,10 +283,10 @@ DGPU_HD void ip_stage(const IpLen &f, int i, const cx<T> *__restrict__ tw, int t
         // the last stage of a DIF (first of a DIT) transform: every group has
         // k = 0, whose twiddles are all 1
 #pragma unroll
-        for (int u = 0; u < NB; ++u) butterfly<T, R, SIGN>(v + u * R);
+        for (int u = 0; u < NB; ++u) butterfly<T, R, SIGN, FIX>(v + u * R);
     } else {
 #pragma unroll
-        for (int u = 0; u < NB; ++u) ip_group<T, R, SIGN, DIF>(v + u * R, tw + f.twoff[i], kk[u]);
+        for (int u = 0; u < NB; ++u) ip_group<T, R, SIGN, DIF, FIX>(v + u * R, tw + f.twoff[i], kk[u]);
     }
 #pragma unroll
     for (int u = 0; u < NB; ++u) {
@@ -426,7 +447,7 @@ DGPU_HD bool ip_bits_apart(const IpLen &f, int i)
 
 // In-place stage i on one swizzled row x[ip_swz(pos)] (LDS).  CP: the plan is
 // known at compile time.
-template <typename T, int E, int SIGN, bool DIF, bool CP = false>
+template <typename T, int E, int SIGN, bool DIF, bool CP = false, bool FIX = false>
 DGPU_HD void ip_stage_row(cx<T> *x, const IpLen &f, int i, const cx<T> *__restrict__ tw, int th)
 {
     with_radix<E>(f.radix[i], [&](auto rc) {
@@ -443,17 +464,17 @@ DGPU_HD void ip_stage_row(cx<T> *x, const IpLen &f, int i, const cx<T> *__restri
             for (int e = 0; e < E; ++e) v[e] = at(e / R, e % R);
             if (L == 1) {
 #pragma unroll
-                for (int u = 0; u < NB; ++u) butterfly<T, R, SIGN>(v + u * R);
+                for (int u = 0; u < NB; ++u) butterfly<T, R, SIGN, FIX>(v + u * R);
             } else {
 #pragma unroll
                 for (int u = 0; u < NB; ++u)
-                    ip_group<T, R, SIGN, DIF>(v + u * R, tw + f.twoff[i], wide ? k0 + u * f.t : k0);
+                    ip_group<T, R, SIGN, DIF, FIX>(v + u * R, tw + f.twoff[i], wide ? k0 + u * f.t : k0);
             }
 #pragma unroll
             for (int e = 0; e < E; ++e) at(e / R, e % R) = v[e];
             return;
         }
-        ip_stage<T, E, R, SIGN, DIF>(
+        ip_stage<T, E, R, SIGN, DIF, FIX>(
             f, i, tw, th, [&](int, int pos) { return x[ip_swz(f, pos)]; },
             [&](int, int pos, cx<T> v) { x[ip_swz(f, pos)] = v; });
     });

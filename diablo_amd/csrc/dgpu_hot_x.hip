@@ -92,7 +92,7 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
     const bool lin = CP && ip_bits_apart<E, R0>(fx, 0);
     auto dif0 = [&](cx<T> *row) {
         const int s0 = ip_swz(fx, th);
-        ip_stage<T, E, R0, +1, true>(
+        ip_stage<T, E, R0, +1, true, true>(
             fx, 0, tw, th,
             [&](int idx, int f) {
                 cx<T> A = pa[idx], B = pb[idx];
@@ -121,8 +121,8 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
             va[q] = row[lin ? ip_slot(fx, sa, q * L0) : ip_swz(fx, ga + q * L0)];
             vb[q] = row[lin ? ip_slot(fx, sb, q * L0) : ip_swz(fx, gb + q * L0)];
         }
-        ip_group<T, R0, -1, false>(va, tw + fx.twoff[0], ga);
-        ip_group<T, R0, -1, false>(vb, tw + fx.twoff[0], gb);
+        ip_group<T, R0, -1, false, true>(va, tw + fx.twoff[0], ga);
+        ip_group<T, R0, -1, false, true>(vb, tw + fx.twoff[0], gb);
         const T h = T(0.5) / T(nx);
         cx<T> *o0 = wt + (long)j * wt_ps + zrow;
         // Outputs of pair row r (field slots of wt): G1 | G2 | G3, H1 | H2, H3
@@ -135,12 +135,13 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
         const long off2 = (long)(r == 2 ? 1 : 5) * wt_fs;
         const bool two = r == 2 || r == 3, xa1 = r == 3 || r == 5;
         auto emit = [&](int kp, cx<T> Zk, cx<T> Zn) {
+#pragma clang fp contract(off)
             if (!zvalid) return;
             const cx<T> Xa = make_cx<T>((Zk.re + Zn.re) * h, (Zk.im - Zn.im) * h);
             const cx<T> Xb = make_cx<T>((Zk.im + Zn.im) * h, -(Zk.re - Zn.re) * h);
             const T kx = kxs[kp];
             // -(i kx Xa + Xb)
-            const cx<T> G = make_cx<T>(kx * Xa.im - Xb.re, -kx * Xa.re - Xb.im);
+            const cx<T> G = make_cx<T>(fma_(kx, Xa.im, -Xb.re), fma_(-kx, Xa.re, -Xb.im));
             const cx<T> nXa = make_cx<T>(-Xa.re, -Xa.im), nXb = make_cx<T>(-Xb.re, -Xb.im);
             if constexpr (sizeof(T) == 4) {
                 o0[off1 + kp] = xa1 ? nXa : G;
@@ -179,6 +180,7 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
         const int extra = npos % nthr;
         const int e0 = extra ? (tid + nthr - extra) % nthr : tid;
         for (int e = e0; e < npos; e += nthr) {
+#pragma clang fp contract(off)
             const int zq = e / nx, x = e - zq * nx;
             cx<T> *const zw = base + zq * zsz;
             const cx<T> *wm = zw + ((j - 1) % 3) * npi * nx, *w0 = zw + (j % 3) * npi * nx,
@@ -192,10 +194,12 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
             const T p0 = u3 * u1;                                                      // U1*U3
             const T p1 = u1 * u1;                                                      // U1*U1
             const T p2 = u3 * u3;                                                      // U3*U3
-            const T p3 = ((dyfj * u1 + dyfm * u1m) * r2dy) * u2;                 // U1*U2 at GY
-            const T p4 = ((dyfj * u3 + dyfm * u3m) * r2dy) * u2;                 // U3*U2 at GY
-            const T p5 = (u1p * u2p + u1 * u2p - u1 * u2 - u1m * u2) * r2dyf;    // d/dy(U1 U2)
-            const T p6 = (u3p * u2p + u3 * u2p - u3 * u2 - u3m * u2) * r2dyf;    // d/dy(U3 U2)
+            const T p3 = (fma_(dyfj, u1, dyfm * u1m) * r2dy) * u2;               // U1*U2 at GY
+            const T p4 = (fma_(dyfj, u3, dyfm * u3m) * r2dy) * u2;               // U3*U2 at GY
+            // up u2p + u0 u2p, less u0 u2 + um u2
+            auto less = [&](T f, T u0, T um) { return fma_(-um, u2, fma_(-u0, u2, f)); };
+            const T p5 = less(fma_(u1p, u2p, u1 * u2p), u1, u1m) * r2dyf;        // d/dy(U1 U2)
+            const T p6 = less(fma_(u3, u2p, u3p * u2p), u3, u3m) * r2dyf;        // d/dy(U3 U2)
             const T sp = u2 + u2p, sm = u2 + u2m;
             const T p7 = (T(0.25) * (sp * sp) - T(0.25) * (sm * sm)) * rdy;      // d/dy(U2 U2)
             fq[0 * nx + x] = make_cx<T>(p1, p5);
@@ -206,7 +210,7 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
                 const T t0 = b0.im, tm = bm.im, tp = bp.im;
                 const T p8 = t0 * u1;
                 const T p9 = t0 * u3;
-                const T p10 = (tp * u2p + t0 * u2p - t0 * u2 - tm * u2) * r2dyf;
+                const T p10 = less(fma_(t0, u2p, tp * u2p), t0, tm) * r2dyf;
                 fq[4 * nx + x] = make_cx<T>(p8, p10);
                 fq[5 * nx + x] = make_cx<T>(p9, T(0));
             }
@@ -224,7 +228,7 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
     if (pro) dif0(slot_row(pro_plane, pro_pair));
     __syncthreads();
     stage_loop<CP>(1, S, [&](int s) {
-        if (pro) ip_stage_row<T, E, +1, true, CP>(slot_row(pro_plane, pro_pair), fx, s, tw, th);
+        if (pro) ip_stage_row<T, E, +1, true, CP, true>(slot_row(pro_plane, pro_pair), fx, s, tw, th);
         __syncthreads();
     });
     if (dif_row) {
@@ -268,8 +272,8 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
                 asm volatile("" : "+v"(th));
                 __builtin_assume(th >= 0 && th < TT);
             }
-            if (inv) ip_stage_row<T, E, +1, true, CP>(drow, fx, s + 1, tw, th);
-            if (fwd) ip_stage_row<T, E, -1, false, CP>(frow, fx, S - 1 - s, tw, th);
+            if (inv) ip_stage_row<T, E, +1, true, CP, true>(drow, fx, s + 1, tw, th);
+            if (fwd) ip_stage_row<T, E, -1, false, CP, true>(frow, fx, S - 1 - s, tw, th);
             row_sync();
         });
         if (fwd) dit_out(frow, p - npi, j - 1);
