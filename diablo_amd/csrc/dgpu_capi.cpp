@@ -1961,11 +1961,23 @@ int32_t dgpu_rk_chan_1(dgpu_ctx *c, int32_t rk_step, double time, const double *
     return DGPU_OK;
 }
 
+// What the autotuners report of planes per block: rounded up to a power of two
+// from `least` to 64.
+static int reported_chunk(int xchunk, int least)
+{
+    int r = least;
+    while (r < xchunk && r < 64) r *= 2;
+    return r;
+}
+
 // Launch-shape autotuner: times `steps` RK3 steps (after one untimed step)
 // of this context's own state (with time step delta_t) for each candidate -- planes per block of the
 // fused x kernel, and for mixed contexts with NX, NZ <= 256 the FFT or the
-// MFMA z transforms -- and keeps the fastest.  The state is copied aside
-// before and put back after, so tuning does not advance the run.
+// MFMA z transforms -- and keeps the fastest.  The context's own shape is the
+// first candidate, so tuning does not leave it slower than it was
+// (64x65x64 FP64 194 -> 205 us and 32x33x32 132 -> 188 when it was not
+// among them).  The state is copied aside before and put back after, so tuning
+// does not advance the run.
 int32_t dgpu_autotune(dgpu_ctx *c, int32_t steps, double delta_t, int32_t *xchunk_out, int32_t *zdft_out,
                       double *ms_per_step)
 {
@@ -2015,7 +2027,13 @@ int32_t dgpu_autotune(dgpu_ctx *c, int32_t steps, double delta_t, int32_t *xchun
     };
     // x-kernel planes per block and the z transforms, then the column shape
     // (LES runs keep the column stage of the LES substep)
-    const int chunks[] = {4, 8, 16, 32, 64};
+    std::vector<int> chunks{xchunk0};
+    int jlo = 2;
+    for (int n = 0; n < c->g.nth; ++n) jlo = std::min(jlo, c->jstart_th[n]);
+    for (int xc : {1, 2, 3, 4, 6, 8, 16, 32, 64}) {
+        xc = std::min(xc, c->g.ny - jlo + 1);
+        if (std::find(chunks.begin(), chunks.end(), xc) == chunks.end()) chunks.push_back(xc);
+    }
     int best_x = xchunk0, best_c = colnw0, best_f = colfuse0;
     bool best_z = zdft0;
     double best = 1e300;
@@ -2067,7 +2085,7 @@ int32_t dgpu_autotune(dgpu_ctx *c, int32_t steps, double delta_t, int32_t *xchun
     if (e1) (void)hipEventDestroy(e1);
     (void)hipFree(backup);
     if (rc) return rc;
-    if (xchunk_out) *xchunk_out = c->xchunk;
+    if (xchunk_out) *xchunk_out = reported_chunk(c->xchunk, 4);
     if (zdft_out) *zdft_out = c->zdft ? 1 : 0;
     if (ms_per_step) *ms_per_step = best;
     return DGPU_OK;
@@ -2782,12 +2800,6 @@ int32_t dgpu_ensemble_autotune(dgpu_ensemble *e, int32_t steps, const double *h_
         }
         return DGPU_OK;
     };
-    auto set_shape = [&](int xc, int nw) {
-        for (dgpu_ctx *c : e->m) {
-            c->xchunk = xc;
-            c->colnw = nw;
-        }
-    };
     // wall time per step of the current shapes, from the saved states
     auto time_shape = [&](double &ms) -> int {
         if (int rc = restore()) return rc;
@@ -2802,18 +2814,32 @@ int32_t dgpu_ensemble_autotune(dgpu_ensemble *e, int32_t steps, const double *h_
         ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count() / steps;
         return DGPU_OK;
     };
-    const int xc0 = e->m[0]->xchunk, nw0 = e->m[0]->colnw;
-    int best_x = xc0, best_w = nw0;
-    double best = 1e300;
-    int rc = DGPU_OK;
-    const int chunks[] = {8, 16, 32, 64};
+    // 0: every member's own shape, the first candidate
+    std::vector<int> own_x, own_w;
+    for (const dgpu_ctx *c : e->m) {
+        own_x.push_back(c->xchunk);
+        own_w.push_back(c->colnw);
+    }
+    auto set_shape = [&](int xc, int nw) {
+        for (int i = 0; i < n; ++i) {
+            e->m[i]->xchunk = xc ? xc : own_x[i];
+            e->m[i]->colnw = nw < 0 ? own_w[i] : nw;
+        }
+    };
+    const int nw0 = e->m[0]->colnw;
+    int best_x = 0, best_w = -1;
+    double best = 0.0;
+    int rc = time_shape(best);
+    const int chunks[] = {0, 8, 16, 32, 64};
     const int waves[] = {4, 8, 16};
     for (int xc : chunks) {
+        if (rc) break;
         for (int nw : waves) {
             if (nw0 == 0 && nw != waves[0]) continue;  // the sweeps were chosen: x chunks only
             bool fits = true;
             for (const dgpu_ctx *c : e->m) fits = fits && column_shape_fits(c, nw);
             const int w = (nw0 == 0 || !fits) ? nw0 : nw;
+            if (!xc && std::all_of(own_w.begin(), own_w.end(), [&](int v) { return v == w; })) continue;
             set_shape(xc, w);
             double ms = 0.0;
             if ((rc = time_shape(ms))) break;
@@ -2823,9 +2849,8 @@ int32_t dgpu_ensemble_autotune(dgpu_ensemble *e, int32_t steps, const double *h_
                 best_w = w;
             }
         }
-        if (rc) break;
     }
-    set_shape(rc == DGPU_OK ? best_x : xc0, rc == DGPU_OK ? best_w : nw0);
+    set_shape(rc == DGPU_OK ? best_x : 0, rc == DGPU_OK ? best_w : -1);
     const int rr = restore();
     if (rc == DGPU_OK) rc = rr;
     free_all();
@@ -2833,8 +2858,10 @@ int32_t dgpu_ensemble_autotune(dgpu_ensemble *e, int32_t steps, const double *h_
         if (e->err.empty()) e->err = "ensemble autotune";
         return rc;
     }
-    if (xchunk_out) *xchunk_out = best_x;
-    if (waves_out) *waves_out = best_w;
+    std::vector<int> xs;
+    for (const dgpu_ctx *c : e->m) xs.push_back(c->xchunk);
+    if (xchunk_out) *xchunk_out = reported_chunk(*std::max_element(xs.begin(), xs.end()), 8);
+    if (waves_out) *waves_out = e->m[0]->colnw;
     if (ms_per_step) *ms_per_step = best;
     return DGPU_OK;
 }

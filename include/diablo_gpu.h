@@ -312,15 +312,15 @@ int32_t dgpu_get_column_shape(const dgpu_ctx *ctx, int32_t *waves, int32_t *fuse
 
 /* Launch-shape autotuner (no counterpart in the reference): times `steps` RK3
  * steps of size delta_t (after one untimed step) of the context's own state
- * for each candidate -- planes per block of the fused x kernel (4..64), and
- * for mixed contexts with NX, NZ <= 256 the FFT or the MFMA z transforms;
- * then, with those fixed, the column shape (dgpu_set_column_shape: 4, 8 or
+ * for each candidate -- the context's own planes per block of the fused x
+ * kernel and 1 to 64, and for mixed contexts with NX, NZ <= 256 the FFT or
+ * the MFMA z transforms; then, with those fixed, the column shape (dgpu_set_column_shape: 4, 8 or
  * 16 waves per block, unless the sweeps are selected; with the FP32 state
  * and in FP64 also the fused column kernel on and off) -- keeps the fastest and puts
  * the state back as it was (the run does not advance).
- * Outputs (may be NULL): the chosen planes per block, whether the MFMA z
- * transforms are on, and the best ms per step.  Not with a COURANT request
- * pending.  Allocates a copy of the state while it runs. */
+ * Outputs (may be NULL): the chosen planes per block, rounded up to 4, 8, 16,
+ * 32 or 64, whether the MFMA z transforms are on, and the best ms per step.
+ * Not with a COURANT request pending.  Allocates a copy of the state while it runs. */
 int32_t dgpu_autotune(dgpu_ctx *ctx, int32_t steps, double delta_t, int32_t *xchunk, int32_t *zdft,
                       double *ms_per_step);
 
@@ -367,13 +367,15 @@ int32_t dgpu_ensemble_synchronize(dgpu_ensemble *ens);
 
 /* Ensemble launch-shape autotuner (no counterpart in the reference): times
  * `steps` RK3 steps (after one untimed step, wall clock between ensemble
- * synchronisations) of the members' own states for each candidate -- planes
- * per block of the batched x kernel (8..64, every member) and the column
- * shape (dgpu_set_column_shape's waves: 4, 8, 16, every member; the fused
- * setting of each member stays) -- keeps the fastest and puts every
+ * synchronisations) of the members' own states for each candidate -- the
+ * members' own shapes, then planes per block of the batched x kernel (their
+ * own and 8..64, every member) and the column shape (dgpu_set_column_shape's
+ * waves: 4, 8, 16, every member; the fused setting of each member stays) --
+ * keeps the fastest and puts every
  * member's state back (the run does not advance).  h_bar, beta_bar and
  * zeta_bar as for dgpu_ensemble_rk_chan_1.  Outputs (may be NULL): the
- * planes per block, the waves, the best ms per step.  Not with a member's
+ * largest planes per block, rounded up to 8, 16, 32 or 64, the first member's
+ * waves, the best ms per step.  Not with a member's
  * COURANT request pending.  Allocates a copy of every member's state while
  * it runs. */
 int32_t dgpu_ensemble_autotune(dgpu_ensemble *ens, int32_t steps, const double *h_bar, const double *beta_bar,
