@@ -134,6 +134,7 @@ struct dgpu_ctx {
 struct dgpu_ens_group {
     std::vector<int> idx;
     int max_planes = 0, max_span = 0, max_zf = 0;  // tallest member: NY+2, x-sweep planes, z-forward planes
+    int xchunk = 64;  // planes per block of the batched x kernel
     void *d_zinv = nullptr, *d_xf = nullptr, *d_zf = nullptr, *d_scat = nullptr;
     void *d_col[3] = {nullptr, nullptr, nullptr};   // column descriptors per RK stage
     void *d_cols[3] = {nullptr, nullptr, nullptr};  // low-mode columns (FP32 state)
@@ -584,9 +585,9 @@ int32_t dgpu_create(const dgpu_params *p, dgpu_ctx **out)
         if (xc && std::atoi(xc) > 0) {
             c->xchunk = std::atoi(xc);
         } else {
-            const int jlo = g.nth ? std::min(2, c->jstart_th[0]) : 2;
-            c->xchunk = c->mixed ? dgpu::xfused_auto_chunk<float>(g, c->ipx, jlo, g.ny)
-                                 : dgpu::xfused_auto_chunk<double>(g, c->ipx, jlo, g.ny);
+            const int planes = g.ny - (g.nth ? std::min(2, c->jstart_th[0]) : 2) + 1;
+            c->xchunk = c->mixed ? dgpu::xfused_auto_chunk<float>(g, c->ipx, &planes, 1, 1.0)
+                                 : dgpu::xfused_auto_chunk<double>(g, c->ipx, &planes, 1, 1.0);
         }
     }
     int rc = 0;
@@ -2269,6 +2270,33 @@ static int upload(void **dptr, const std::vector<D> &h)
     return DGPU_OK;
 }
 
+// Planes per block of each group's batched x kernel, by the rule of a single
+// run over all the group's planes (a fixed 64 in FP64, 32 in FP32 before: three
+// members of 64x{33,65,97}x64 had 48 blocks, 1096 us a step against
+// 351, mixed 763 against 357).  Groups on streams of their own run at the same
+// time: each counts on its share of the points.
+static void ens_group_chunks(dgpu_ensemble *e)
+{
+    const char *xc = std::getenv("DGPU_XCHUNK");
+    double all = 0.0;
+    auto points = [](const dgpu_ctx *c) { return (double)c->g.nx * c->g.nz * c->g.ny; };
+    for (const dgpu_ctx *c : e->m) all += points(c);
+    for (auto &gr : e->groups) {
+        const dgpu_ctx *c0 = e->m[gr.idx[0]];
+        std::vector<int> planes;
+        double own = 0.0;
+        for (int i : gr.idx) {
+            planes.push_back(e->m[i]->g.ny - member_jlo(e->m[i]) + 1);
+            own += points(e->m[i]);
+        }
+        const double share = e->group_streams ? own / all : 1.0;
+        const int n = (int)planes.size();
+        gr.xchunk = xc && std::atoi(xc) > 0 ? std::atoi(xc)
+                    : c0->mixed ? dgpu::xfused_auto_chunk<float>(c0->g, c0->ipx, planes.data(), n, share)
+                                : dgpu::xfused_auto_chunk<double>(c0->g, c0->ipx, planes.data(), n, share);
+    }
+}
+
 // Groups the members by (NX, NZ, N_TH) and writes the transform descriptors
 // (they do not change between steps).  Members of different precisions keep
 // the per-member path.
@@ -2304,10 +2332,7 @@ static int ens_build_groups(dgpu_ensemble *e)
         std::vector<dgpu::ZfDesc<float, float>> zf32;
         std::vector<dgpu::ScatDesc<double, float>> sc;
         for (int i : gr.idx) {
-            dgpu_ctx *c = e->m[i];
-            // the group's launches fill the GPU with whole sweeps of many
-            // members: longer chunks than a member alone would take
-            if (!std::getenv("DGPU_XCHUNK")) c->xchunk = mixed ? 32 : 64;
+            const dgpu_ctx *c = e->m[i];
             const int jlo = member_jlo(c), ny = c->g.ny;
             gr.max_planes = std::max(gr.max_planes, ny + 2);
             gr.max_span = std::max(gr.max_span, ny - jlo + 1);
@@ -2353,6 +2378,7 @@ static int ens_build_groups(dgpu_ensemble *e)
                 return DGPU_E_HIP;
         e->group_streams = true;
     }
+    ens_group_chunks(e);
     e->batched = true;
     return DGPU_OK;
 }
@@ -2458,7 +2484,7 @@ static int ens_enqueue_batched(dgpu_ensemble *e, int rk_step)
                                                        (const dgpu::ZinvDesc<double, double> *)gr.d_zinv, nm,
                                                        gr.max_planes, c0->ld, nin);
             dgpu::launch_xfused_ip_batch<double>(s, g, c0->ipx, twx, (const dgpu::XfDesc<double> *)gr.d_xf, nm,
-                                                 gr.max_span, c0->ld, c0->xchunk);
+                                                 gr.max_span, c0->ld, gr.xchunk);
             dgpu::launch_zfwd_nl_ip_batch<double, double>(s, g, c0->ipz, twz,
                                                           (const dgpu::ZfDesc<double, double> *)gr.d_zf, nm,
                                                           gr.max_zf, c0->ld, nin);
@@ -2473,7 +2499,7 @@ static int ens_enqueue_batched(dgpu_ensemble *e, int rk_step)
                                                           (const dgpu::ZinvDesc<float, double> *)gr.d_zinv, nm,
                                                           gr.max_planes, c0->ld, nin);
             dgpu::launch_xfused_ip_batch<float>(s, g, c0->ipx, twx, (const dgpu::XfDesc<float> *)gr.d_xf, nm,
-                                                gr.max_span, c0->ld, c0->xchunk);
+                                                gr.max_span, c0->ld, gr.xchunk);
             dgpu::launch_zfwd_nl_ip_batch<float, float>(s, g, c0->ipz, twz,
                                                         (const dgpu::ZfDesc<float, float> *)gr.d_zf, nm, gr.max_zf,
                                                         c0->ld, nin);
@@ -2726,6 +2752,7 @@ int32_t dgpu_ensemble_rk_chan_1(dgpu_ensemble *e, int32_t rk_step, const double 
     if (!graphable) return enqueue_all(false);
     std::vector<int> shape;
     for (const dgpu_ctx *c : e->m) shape.insert(shape.end(), {c->xchunk, c->colnw, c->colfuse, c->zdft ? 1 : 0});
+    for (const auto &gr : e->groups) shape.push_back(gr.xchunk);
     if (!(e->gexec[k] && e->gkey[k] == key && e->gshape[k] == shape)) {
         if (e->gexec[k]) {
             (void)hipGraphExecDestroy(e->gexec[k]);
@@ -2755,8 +2782,8 @@ int32_t dgpu_ensemble_rk_chan_1(dgpu_ensemble *e, int32_t rk_step, const double 
     return DGPU_OK;
 }
 
-// Ensemble launch shapes: every member's x-kernel planes per block (the
-// batched x launch of a group takes its first member's) and column shape,
+// Ensemble launch shapes: the x-kernel planes per block of every group (or
+// member, where there are no batched launches) and the members' column shape,
 // timed over the ensemble's own states, which are put back afterwards.
 int32_t dgpu_ensemble_autotune(dgpu_ensemble *e, int32_t steps, const double *h_bar, const double *beta_bar,
                                const double *zeta_bar, int32_t *xchunk_out, int32_t *waves_out, double *ms_per_step)
@@ -2814,23 +2841,25 @@ int32_t dgpu_ensemble_autotune(dgpu_ensemble *e, int32_t steps, const double *h_
         ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count() / steps;
         return DGPU_OK;
     };
-    // 0: every member's own shape, the first candidate
+    // the x kernels' planes per block: the groups', or the members' where they
+    // run one by one.  0: as they are, the first candidate
+    std::vector<int *> x;
+    if (e->batched)
+        for (auto &gr : e->groups) x.push_back(&gr.xchunk);
+    else
+        for (dgpu_ctx *c : e->m) x.push_back(&c->xchunk);
     std::vector<int> own_x, own_w;
-    for (const dgpu_ctx *c : e->m) {
-        own_x.push_back(c->xchunk);
-        own_w.push_back(c->colnw);
-    }
+    for (const int *v : x) own_x.push_back(*v);
+    for (const dgpu_ctx *c : e->m) own_w.push_back(c->colnw);
     auto set_shape = [&](int xc, int nw) {
-        for (int i = 0; i < n; ++i) {
-            e->m[i]->xchunk = xc ? xc : own_x[i];
-            e->m[i]->colnw = nw < 0 ? own_w[i] : nw;
-        }
+        for (size_t i = 0; i < x.size(); ++i) *x[i] = xc ? xc : own_x[i];
+        for (int i = 0; i < n; ++i) e->m[i]->colnw = nw < 0 ? own_w[i] : nw;
     };
     const int nw0 = e->m[0]->colnw;
     int best_x = 0, best_w = -1;
     double best = 0.0;
     int rc = time_shape(best);
-    const int chunks[] = {0, 8, 16, 32, 64};
+    const int chunks[] = {0, 2, 4, 8, 16, 32, 64};
     const int waves[] = {4, 8, 16};
     for (int xc : chunks) {
         if (rc) break;
@@ -2858,9 +2887,9 @@ int32_t dgpu_ensemble_autotune(dgpu_ensemble *e, int32_t steps, const double *h_
         if (e->err.empty()) e->err = "ensemble autotune";
         return rc;
     }
-    std::vector<int> xs;
-    for (const dgpu_ctx *c : e->m) xs.push_back(c->xchunk);
-    if (xchunk_out) *xchunk_out = reported_chunk(*std::max_element(xs.begin(), xs.end()), 8);
+    int most = 0;
+    for (const int *v : x) most = std::max(most, *v);
+    if (xchunk_out) *xchunk_out = reported_chunk(most, 8);
     if (waves_out) *waves_out = e->m[0]->colnw;
     if (ms_per_step) *ms_per_step = best;
     return DGPU_OK;

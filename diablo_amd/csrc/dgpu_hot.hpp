@@ -134,8 +134,9 @@ __device__ __forceinline__ void x_split(const IpLen &fx, const cx<T> *row, const
 // Id of the compile-time plan equal to f, or 0 (dgpu_hot_z.hip).
 int const_plan_id(const IpLen &f);
 
-// Planes per block of a sweeping kernel (dgpu_hot_x.hip).
-int sweep_rule(long rows, int planes, long slots);
+// Planes per block of a sweeping kernel over `runs` fields of so many planes,
+// alone on the device or among others (dgpu_hot_x.hip).
+int sweep_rule(long rows, const int *planes, int runs, long slots, bool among = false);
 
 // Blocks of a kernel that the whole device holds at once.
 template <class K>

@@ -482,21 +482,29 @@ static int xfused_zrows(const IpLen &fx, int nz, int mk)
 // pass), and an iteration takes nearly the same time whether a CU holds one
 // block or all that fit, so up to one full round only the chunk's length
 // counts.  Beyond it a round that is partly empty costs a whole one while the
-// rounds are few; over many rounds blocks even that out by half.  On small
+// rounds are few; over many rounds blocks even that out by half.  Among other
+// launches (the groups of an ensemble) what a round leaves empty they fill: the
+// iterations of all blocks, and a block at the end.  On small
 // grids the former fixed 64 (FP64) / 32 planes left most CUs without a block:
-// one RK3 step at 64x65x64 FP64 1502 -> 219 us (2 planes), 96x81x108 1984 ->
-// 520, 192x129x192 2819 -> 1840; at 384x257x384 the rule gives the 64 (FP64)
-// and 32 (FP32) planes measured best there.
-int sweep_rule(long rows, int planes, long slots)
+// one RK3 step at 64x65x64 FP64 1005 -> 159 us (2 planes; the 64 were one block
+// of 63 a row), 192x129x192 2819 -> 1840, three members of 64x{33,65,97}x64
+// 1096 -> 351; at 384x257x384 the rule gives the 64 (FP64) and 32 (FP32) planes
+// measured best there.
+int sweep_rule(long rows, const int *planes, int runs, long slots, bool among)
 {
-    int best = planes;
+    const int most = *std::max_element(planes, planes + runs);
+    int best = most;
     double best_cost = 1e300;
-    for (int n = 1; n <= planes; ++n) {
-        const int c = (planes + n - 1) / n;
-        const long blocks = rows * ((planes + c - 1) / c);
-        const double r = (double)blocks / (double)slots, up = std::ceil(r);
-        const double rounds = r <= 3.0 ? std::max(1.0, up) : r + 0.5 * (up - r);
-        const double cost = rounds * (c + 1.5);
+    for (int n = 1; n <= most; ++n) {
+        const int c = (most + n - 1) / n;
+        long blocks = 0, swept = 0;
+        for (int r = 0; r < runs; ++r) {
+            blocks += rows * ((planes[r] + c - 1) / c);
+            swept += rows * planes[r];
+        }
+        const double block = c + 1.5, r = (double)blocks / (double)slots, up = std::ceil(r);
+        const double cost = among ? std::max(block, (swept + 1.5 * blocks) / (double)slots + block)
+                                  : (r <= 3.0 ? std::max(1.0, up) : r + 0.5 * (up - r)) * block;
         if (cost < best_cost * (1.0 - 1e-9)) {
             best_cost = cost;
             best = c;
@@ -505,11 +513,17 @@ int sweep_rule(long rows, int planes, long slots)
     return best;
 }
 
-// pick: nothing is launched, *pick receives the rule's planes per block
+// pick: nothing is launched, pick->chunk receives the rule's planes per block
+struct XPick {
+    const int *planes;  // of each run of the launch
+    int runs;
+    double share;       // of the device that the launch has to itself
+    int chunk;
+};
 template <typename T, int E, int NTH, int PID>
 static void xfused_ip_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, int ld, const cx<T> *zt,
                         long zt_fs, cx<T> *wt, long wt_fs, const double *dy, const double *dyf, const double *kx,
-                        int jlo, int jhi, int chunk, int *pick)
+                        int jlo, int jhi, int chunk, XPick *pick)
 {
     using C = XCount<NTH>;
     const int zr = xfused_zrows<T, NTH>(fx, g.nz, g.mk);
@@ -523,8 +537,9 @@ static void xfused_ip_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T
         attr = true;
     }
     if (pick) {
-        *pick = sweep_rule((g.nz + zr - 1) / zr, jhi - jlo + 1,
-                            kernel_slots(&k_xfused_ip<T, E, NTH, PID>, threads, lds));
+        const long slots = kernel_slots(&k_xfused_ip<T, E, NTH, PID>, threads, lds);
+        pick->chunk = sweep_rule((g.nz + zr - 1) / zr, pick->planes, pick->runs,
+                                 std::max(1L, (long)(slots * pick->share)), pick->share < 1.0);
         return;
     }
     const int nchunks = (jhi - jlo + 1 + chunk - 1) / chunk;
@@ -539,7 +554,7 @@ static void xfused_ip_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T
 template <typename T>
 static void xfused_ip_any(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, int ld, const cx<T> *zt,
                           long zt_fs, cx<T> *wt, long wt_fs, const double *dy, const double *dyf, const double *kx,
-                          int jlo, int jhi, int chunk, int *pick)
+                          int jlo, int jhi, int chunk, XPick *pick)
 {
     if (g.nth == 1 && with_pid(const_plan_id(fx), XPids<T>{}, [&](auto pc) {
             constexpr int P = decltype(pc)::value;
@@ -578,11 +593,11 @@ void launch_xfused_ip(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> 
 }
 
 template <typename T>
-int xfused_auto_chunk(const Geo &g, const IpLen &fx, int jlo, int jhi)
+int xfused_auto_chunk(const Geo &g, const IpLen &fx, const int *planes, int runs, double share)
 {
-    int c = 0;
-    xfused_ip_any<T>(nullptr, g, fx, nullptr, 0, nullptr, 0, nullptr, 0, nullptr, nullptr, nullptr, jlo, jhi, 1, &c);
-    return c > 0 ? c : 32;
+    XPick p{planes, runs, share, 0};
+    xfused_ip_any<T>(nullptr, g, fx, nullptr, 0, nullptr, 0, nullptr, 0, nullptr, nullptr, nullptr, 0, 0, 1, &p);
+    return p.chunk > 0 ? p.chunk : 32;
 }
 
 template <typename T, int E, int NTH, int PID>
@@ -668,8 +683,8 @@ void launch_vmax_ip(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *t
     DGPU_DISPATCH_IPE(fx.e, (vmax_ip_e<T, EE>(s, g, fx, tw, ld, zt, zt_fs, part, out)));
 }
 
-template int xfused_auto_chunk<double>(const Geo &, const IpLen &, int, int);
-template int xfused_auto_chunk<float>(const Geo &, const IpLen &, int, int);
+template int xfused_auto_chunk<double>(const Geo &, const IpLen &, const int *, int, double);
+template int xfused_auto_chunk<float>(const Geo &, const IpLen &, const int *, int, double);
 template void launch_vmax_ip<double>(hipStream_t, const Geo &, const IpLen &, const cx<double> *, int,
                                      const cx<double> *, long, double *, double *);
 template void launch_vmax_ip<float>(hipStream_t, const Geo &, const IpLen &, const cx<float> *, int,

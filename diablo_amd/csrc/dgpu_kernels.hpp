@@ -167,9 +167,10 @@ template <typename T>
 void launch_xfused_ip(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, int ld, const cx<T> *zt,
                       long zt_fs, cx<T> *wt, long wt_fs, const double *dy, const double *dyf, const double *kx,
                       int jlo, int jhi, int chunk);
-// Planes per block of launch_xfused_ip by its rule (dgpu_hot_x.hip).
+// Planes per block of launch_xfused_ip, or of its batch over `runs` members, by
+// the rule (dgpu_hot_x.hip), for a launch that has `share` of the device.
 template <typename T>
-int xfused_auto_chunk(const Geo &g, const IpLen &fx, int jlo, int jhi);
+int xfused_auto_chunk(const Geo &g, const IpLen &fx, const int *planes, int runs, double share);
 template <typename T, typename TOUT>
 void launch_zfwd_nl_ip(hipStream_t s, const Geo &g, const IpLen &fz, const cx<T> *tw, const cx<T> *wt, long wt_fs,
                        int ld, cx<TOUT> *const *nl, const double *kz, int jlo, int jhi, int nout);

@@ -398,7 +398,8 @@ static void les_prod_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<do
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_les_prod<E, NTH, PID, LM, WIDE>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     const long rows = (g.nz + a.zr - 1) / a.zr;
-    a.chunk = sweep_rule(rows, a.jhi - a.jlo + 1, kernel_slots(&k_les_prod<E, NTH, PID, LM, WIDE>, threads, lds));
+    const int planes = a.jhi - a.jlo + 1;
+    a.chunk = sweep_rule(rows, &planes, 1, kernel_slots(&k_les_prod<E, NTH, PID, LM, WIDE>, threads, lds));
     const int nchunks = (a.jhi - a.jlo + a.chunk) / a.chunk;
     hipLaunchKernelGGL((k_les_prod<E, NTH, PID, LM, WIDE>), dim3((unsigned)rows, nchunks), dim3(threads), lds, s, fx, tw, g.mk,
                        ld, a);

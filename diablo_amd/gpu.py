@@ -494,8 +494,8 @@ class GpuEnsemble:
 
     def autotune(self, steps: int = 2) -> dict:
         """Times the batched launch shapes on the members' states (every
-        member's x-kernel planes per block and column waves), keeps the
-        fastest; the states are left as they were."""
+        group's x-kernel planes per block, every member's column waves), keeps
+        the fastest; the states are left as they were."""
         xc, w, ms = C.c_int32(0), C.c_int32(0), C.c_double(0.0)
         self._chk(self.L.dgpu_ensemble_autotune(self.h, steps, _dp(self.h_bar), _dp(self.beta_bar),
                                                 _dp(self.zeta_bar), C.byref(xc), C.byref(w), C.byref(ms)),

@@ -368,8 +368,8 @@ int32_t dgpu_ensemble_synchronize(dgpu_ensemble *ens);
 /* Ensemble launch-shape autotuner (no counterpart in the reference): times
  * `steps` RK3 steps (after one untimed step, wall clock between ensemble
  * synchronisations) of the members' own states for each candidate -- the
- * members' own shapes, then planes per block of the batched x kernel (their
- * own and 8..64, every member) and the column shape (dgpu_set_column_shape's
+ * shapes as they are, then planes per block of the batched x kernel (as they
+ * are and 2..64, every group) and the column shape (dgpu_set_column_shape's
  * waves: 4, 8, 16, every member; the fused setting of each member stays) --
  * keeps the fastest and puts every
  * member's state back (the run does not advance).  h_bar, beta_bar and
