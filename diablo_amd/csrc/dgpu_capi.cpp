@@ -86,7 +86,8 @@ struct dgpu_ctx {
     cx<double> *d_zt = nullptr, *d_wt = nullptr;
     long zfs = 0;  // complex elements per intermediate field: (NY+2)*NZ*ld
     double *d_fort = nullptr;  // Fortran-layout planes on the device
-    dgpu::Staging staging;     // pinned slots of the host entry points
+    dgpu::Staging own_staging;  // pinned slots of the host entry points
+    dgpu::Staging *staging = &own_staging;  // an ensemble member's: the ensemble's
     double *d_gyf = nullptr;    // GYF (0:NY+1), part of d_vec
     double *d_stats = nullptr;  // dgpu_stats_chan output
     double *d_noalloc = nullptr;  // this GPU's fixed array of dgpu_stats_chan_noalloc
@@ -161,6 +162,7 @@ struct dgpu_ensemble {
     // and joined back into the ensemble stream (DGPU_ENS_STREAMS=0: one stream)
     bool group_streams = false;
     hipEvent_t gfork = nullptr;
+    dgpu::Staging staging;  // of all members
     std::string err;
 };
 }
@@ -795,7 +797,7 @@ int32_t dgpu_destroy(dgpu_ctx *c)
     }
     if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
     if (c->ev_join) (void)hipEventDestroy(c->ev_join);
-    c->staging.release();
+    c->own_staging.release();
     if (c->stream && c->own_stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return DGPU_OK;
@@ -1415,7 +1417,7 @@ int32_t dgpu_set_field(dgpu_ctx *c, int32_t field, const double *a)
     c->master_dirty = true;
     const HostPlanes h(c->g, 0, c->g.ny + 1);
     const size_t row = sizeof(cx<double>) * h.mk;
-    HIPCHK(c, c->staging.run(
+    HIPCHK(c, c->staging->run(
                   c->stream, h.chunks, h.per * h.bytes,
                   [=](int i, char *slot, hipStream_t s) {
                       char *p = slot;
@@ -1434,7 +1436,7 @@ int32_t dgpu_get_field(dgpu_ctx *c, int32_t field, double *a)
     if (!src) return fail(c, DGPU_E_ARG, "unknown field id");
     if (int rc = to_master(c)) return rc;
     const HostPlanes h(c->g, 0, c->g.ny + 1);
-    HIPCHK(c, c->staging.run(
+    HIPCHK(c, c->staging->run(
                   c->stream, h.chunks, h.per * h.bytes,
                   [=](int i, char *slot, hipStream_t s) {
                       return hipMemcpyAsync(slot, src + h.lo(i) * h.ps, sizeof(cx<double>) * h.ps * h.count(i),
@@ -2131,7 +2133,7 @@ int32_t dgpu_fft_xz_to_fourier(dgpu_ctx *c, double *v, int32_t jmin, int32_t jma
     const HostPlanes h(g, jmin, jmax);
     // the transforms of one chunk run beside the copies of the others; only the
     // kept slots come back (192x129x192: the pair of calls 7.2 -> 3.0 ms)
-    HIPCHK(c, c->staging.run(
+    HIPCHK(c, c->staging->run(
                   c->stream, h.chunks, h.per * h.bytes,
                   [=](int i, char *slot, hipStream_t s) {
                       const int j = h.lo(i), np = h.count(i);
@@ -2160,7 +2162,7 @@ int32_t dgpu_fft_xz_to_physical(dgpu_ctx *c, double *vv, int32_t jmin, int32_t j
     if (int rc = ensure_fort(c)) return rc;
     const HostPlanes h(g, jmin, jmax);
     const long in_ps = (long)(g.nx / 2 + 1) * g.mz;  // the rows K = 0..TNKZ of a plane, whole
-    HIPCHK(c, c->staging.run(
+    HIPCHK(c, c->staging->run(
                   c->stream, h.chunks, h.per * h.bytes,
                   [=](int i, char *slot, hipStream_t s) {
                       const int j = h.lo(i), np = h.count(i), nxp = c->g.nx / 2;
@@ -2615,6 +2617,7 @@ int32_t dgpu_ensemble_destroy(dgpu_ensemble *e)
     for (auto &ge : e->gexec)
         if (ge) (void)hipGraphExecDestroy(ge);
     for (auto *c : e->m) dgpu_destroy(c);
+    e->staging.release();
     for (auto ev : e->join)
         if (ev) (void)hipEventDestroy(ev);
     if (e->fork) (void)hipEventDestroy(e->fork);
@@ -2644,7 +2647,10 @@ int32_t dgpu_ensemble_create(const dgpu_params *members, int32_t n, dgpu_ensembl
         dgpu_ensemble_destroy(e);
         return DGPU_E_HIP;
     }
-    for (dgpu_ctx *c : e->m) c->ens_stream = e->main;
+    for (dgpu_ctx *c : e->m) {
+        c->ens_stream = e->main;
+        c->staging = &e->staging;
+    }
     e->join.assign(n, nullptr);
     for (int i = 0; i < n; ++i)
         if (hipEventCreateWithFlags(&e->join[i], hipEventDisableTiming) != hipSuccess) {

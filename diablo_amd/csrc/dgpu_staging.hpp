@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <atomic>
 #include <exception>
+#include <mutex>
 #include <system_error>
 #include <thread>
 
@@ -21,7 +22,9 @@ namespace dgpu {
 // bytes all use the caller's.
 // Slots and streams are made on first use, kept with the context and given back
 // by release(); threads live for one call, and an array of one chunk starts
-// none.
+// none.  The members of an ensemble share one (a set of slots each is 16 MB of
+// pinned memory a member, 1 GB for 64); calls that come together follow each
+// other.
 class Staging {
 public:
     // planes of `bytes` each that make a chunk
@@ -34,6 +37,7 @@ public:
     template <typename In, typename Out>
     hipError_t run(hipStream_t main, int n, size_t bytes, In in, Out out)
     {
+        std::lock_guard<std::mutex> one(call_);
         int workers = 0, streams = 1;
         if (hipError_t e = reserve(n, bytes, workers, streams)) return e;
         int dev = 0;
@@ -123,6 +127,7 @@ private:
         return hipSuccess;
     }
 
+    std::mutex call_;
     char *slot_[kWorkers] = {};
     hipEvent_t done_[kWorkers] = {};
     size_t size_ = 0;

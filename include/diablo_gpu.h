@@ -128,7 +128,9 @@ const char *dgpu_last_error(const dgpu_ctx *ctx);
 
 /* Copies the kept Fourier slots of one Fortran-layout field to the device
  * (set) or back (get).  get writes every slot of planes 0..NY+1: kept slots
- * get the state, the rest zero. */
+ * get the state, the rest zero.  These and the transforms of host arrays below
+ * go through up to 8 pinned slots of 2 MB (a plane where that is more), made on
+ * first use and held until dgpu_destroy; an ensemble's members share one set. */
 int32_t dgpu_set_field(dgpu_ctx *ctx, int32_t field, const double *fortran_array);
 int32_t dgpu_get_field(dgpu_ctx *ctx, int32_t field, double *fortran_array);
 
