@@ -2208,13 +2208,28 @@ static int fort_to_fourier(dgpu_ctx *c, double *buf, int j0, int j1)
     return check_launch(c, "zfwd_pack(planes)");
 }
 
+// POISSON_P_CHAN runs once a start, so what it keeps is bounded: its six whole
+// pair planes up to this size, Zt's memory instead beyond it.  In Zt's the same
+// takes four runs: 64x65x64 61 us of its own against 121, 128x129x128 (206 MB)
+// 186 against 196, but 192x129x192 (464 MB) 412 against 404 and 384x257x384
+// (3.7 GB) 2817 against 2936.
+static const size_t kOwnPairs = size_t(256) << 20;
+
 int32_t dgpu_poisson_p_chan(dgpu_ctx *c)
 {
     if (!c) return DGPU_E_ARG;
     if (int rc = to_master(c)) return rc;
     c->master_dirty = true;
     const dgpu::Geo &g = c->g;
-    if (int rc = ensure_pairs(c, 6)) return rc;
+    // The pair planes of the call, 5 (2 per + 2) and the sums' per for a run of
+    // `per` plane pairs: Zt's memory, in as few runs as it allows, or the
+    // context's own (six whole pairs) where those are small or Zt is.
+    const long pp = pair_plane(c), room = c->zfs * (3 + g.nth) / pp;
+    const int np = g.ny / 2;
+    const bool own = sizeof(cx<double>) * 6 * pair_fs(c) <= kOwnPairs || room < 21;
+    if (int rc = ensure_pairs(c, own ? 6 : 0)) return rc;
+    cx<double> *const work = own ? c->d_pairs : c->d_zt;
+    const int most = own ? np : (int)((room - 10) / 11), runs = (np + most - 1) / most, per = (np + runs - 1) / runs;
     const cx<double> *twz = c->d_iptw + c->ipx.twn;
     cx<double> *cs = c->nl[1], *scr = c->nl[0];
     // CU1-3 and their z derivatives (Wt fields 0-2, 3-5), with the x
@@ -2228,16 +2243,22 @@ int32_t dgpu_poisson_p_chan(dgpu_ctx *c)
     dgpu::launch_zinv_src(c->stream, g, c->ipz, twz, z, c->d_wt, c->zfs, c->ld, c->d_kx, c->d_kz, 0, g.ny + 2);
     if (int rc = check_launch(c, "zinv(poisson)")) return rc;
     const dgpu::PairSrc src{{0, 2, 1, 3, 5}, {1, 0, 2, 4, -1}, {0, 0, 1, 0, 0}, {0, 1, 1, 0, 0}, 5};
-    if (int rc = pairs_x(c, src, c->d_wt, 0)) return rc;
-    dgpu::PairDst pr{};
-    for (int q = 0; q < 5; ++q) pr.p[q] = pair_buf(c, q);
-    dgpu::launch_pp_rhs(c->stream, g, pr, pair_buf(c, 5), c->d_dyf);
-    if (int rc = check_launch(c, "pp_rhs")) return rc;
-    // rows 2 + 2q and 3 + 2q: the two rows of pair plane q, Wt fields 0 and 1
-    const dgpu::PairDst sum{{pair_buf(c, 5)}};
-    dgpu::launch_pairs_fwd(c->stream, g, c->ipx64, c->d_pairtw, c->ld, sum, c->d_wt, c->zfs,
-                           dgpu::PairOut{{0}, {1}, 1}, 0, g.ny / 2);
-    if (int rc = check_launch(c, "x forward(poisson)")) return rc;
+    // Rows 2 + 2q and 3 + 2q share pair plane q of the sums, whose transforms are
+    // Wt fields 0 and 1, plane q: planes that the runs to come do not read (theirs
+    // begin at 1 + 2q).
+    for (int q0 = 0; q0 < np; q0 += per) {
+        const int q1 = std::min(np, q0 + per), j0 = 1 + 2 * q0, n = std::min(2 + 2 * q1, g.ny + 1) - j0 + 1;
+        dgpu::PairDst pr{};
+        for (int q = 0; q < 5; ++q) pr.p[q] = work + ((long)q * (2 * per + 2) - j0) * pp;
+        dgpu::launch_pairs_inv(c->stream, g, c->ipx64, c->d_pairtw, c->ld, c->d_wt, c->zfs, src, pr, c->d_kx, j0, n);
+        if (int rc = check_launch(c, "x inverse(poisson)")) return rc;
+        const dgpu::PairDst sum{{work + (5L * (2 * per + 2) - q0) * pp}};
+        dgpu::launch_pp_rhs(c->stream, g, pr, sum.p[0], c->d_dyf, q0, q1);
+        if (int rc = check_launch(c, "pp_rhs")) return rc;
+        dgpu::launch_pairs_fwd(c->stream, g, c->ipx64, c->d_pairtw, c->ld, sum, c->d_wt, c->zfs,
+                               dgpu::PairOut{{0}, {1}, 1}, q0, q1 - q0);
+        if (int rc = check_launch(c, "x forward(poisson)")) return rc;
+    }
     dgpu::Geo g2 = g;
     g2.ps = 2 * g.ps;
     dgpu::launch_zfwd_dst(c->stream, g2, c->ipz, twz, c->d_wt, c->zfs, c->ld,

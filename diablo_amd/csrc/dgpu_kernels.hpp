@@ -288,8 +288,9 @@ void launch_pairs_inv(hipStream_t s, const Geo &g, const IpLen &fx, const cx<dou
                       int j0, int nplanes);
 void launch_pairs_fwd(hipStream_t s, const Geo &g, const IpLen &fx, const cx<double> *tw, int ld, const PairDst &src,
                       cx<double> *wt, long wt_fs, const PairOut &out, int j0, int nplanes);
-// POISSON_P_CHAN's right-hand sides, rows 2.. two by two (dgpu_poisson.hip)
-void launch_pp_rhs(hipStream_t s, const Geo &g, const PairDst &pr, cx<double> *out, const double *dyf);
+// POISSON_P_CHAN's right-hand sides, rows 2 + 2 qlo .. 1 + 2 qhi two by two (dgpu_poisson.hip)
+void launch_pp_rhs(hipStream_t s, const Geo &g, const PairDst &pr, cx<double> *out, const double *dyf, int qlo,
+                   int qhi);
 // where pair planes keep x index i of a row, and row z
 int pair_slot(const IpLen &f, int i);
 int pair_zpos(const IpLen &f, int k);

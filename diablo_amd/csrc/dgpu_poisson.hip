@@ -7,7 +7,7 @@
 // tridiagonal solve per (kx,kz) mode.  The reference transforms each of its
 // six products back; here they are summed first and two planes' sums share one
 // complex x transform: nine inverse real transforms and one forward a plane.
-// 192x129x192: 1031 -> 500 us for the whole call, of which the solve 179 -> 48.
+// 192x129x192: 1031 -> 404 us for the whole call, of which the solve 179 -> 48.
 // The solve rows that are read (1..NY) carry the same matrix as REM_DIV_CHAN's
 // (for/channel.f:1126-1143 vs 1399-1440, boundary rows for/mpi.f:1293-1369),
 // so the context's precomputed Poisson factorisation is reused.
@@ -17,15 +17,15 @@ namespace dgpu {
 
 // pairs: 0 (U1, U2), 1 (U3, dU1/dx), 2 (dU2/dx, dU3/dx), 3 (dU1/dz, dU2/dz),
 // 4 (dU3/dz, -).  out plane q: the right-hand sides of rows 2 + 2q and 3 + 2q
-// (0 beyond NY).  A thread owns one position and a chunk of plane pairs; the
-// planes it has read roll through its registers.
+// (0 beyond NY), q = qlo..qhi-1.  A thread owns one position and a chunk of plane
+// pairs; the planes it has read roll through its registers.
 __global__ void __launch_bounds__(256) k_pp_rhs(Geo g, PairDst pr, cx<double> *__restrict__ out,
-                                                const double *__restrict__ dyf, int chunk)
+                                                const double *__restrict__ dyf, int qlo, int qhi, int chunk)
 {
     const long n = (long)g.nx * g.nz;
     const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= n) return;
-    const int NY = g.ny, q0 = blockIdx.y * chunk, q1 = min(q0 + chunk, NY / 2);
+    const int NY = g.ny, q0 = qlo + blockIdx.y * chunk, q1 = min(q0 + chunk, qhi);
     auto at = [&](int q, int j) { return pr.p[q][(long)min(j, NY + 1) * n + e]; };
     const int j0 = 2 + 2 * q0;
     double um = at(0, j0 - 1).re, wm = at(1, j0 - 1).re;
@@ -50,12 +50,13 @@ __global__ void __launch_bounds__(256) k_pp_rhs(Geo g, PairDst pr, cx<double> *_
     }
 }
 
-void launch_pp_rhs(hipStream_t s, const Geo &g, const PairDst &pr, cx<double> *out, const double *dyf)
+void launch_pp_rhs(hipStream_t s, const Geo &g, const PairDst &pr, cx<double> *out, const double *dyf, int qlo,
+                   int qhi)
 {
     const long n = (long)g.nx * g.nz;
     const int chunk = 8;  // 16 planes: one in nine read twice
-    hipLaunchKernelGGL(k_pp_rhs, dim3((unsigned)((n + 255) / 256), (g.ny / 2 + chunk - 1) / chunk), dim3(256), 0, s, g,
-                       pr, out, dyf, chunk);
+    hipLaunchKernelGGL(k_pp_rhs, dim3((unsigned)((n + 255) / 256), (qhi - qlo + chunk - 1) / chunk), dim3(256), 0, s, g,
+                       pr, out, dyf, qlo, qhi, chunk);
 }
 
 // Buoyancy term, the tridiagonal solve and CP (for/channel.f:1373-1449).  The

@@ -153,7 +153,10 @@ int32_t dgpu_rem_div_chan(dgpu_ctx *ctx);
 /* POISSON_P_CHAN (for/channel.f:1217-1453): CP from the device-resident
  * CU1..3 and CTH.  Rows 1..NY of CP are written (as in the reference); the
  * reference's use of CF1..3 as scratch is not reproduced (device scratch is
- * used instead, CF is left unchanged).  Synchronises before returning. */
+ * used instead, CF is left unchanged).  The first call allocates work planes of
+ * 96 NX NZ (NY+2) bytes where these are 256 MB or less (or NY below 20), held
+ * until dgpu_destroy; larger runs use the context's transform buffers.
+ * Synchronises before returning. */
 int32_t dgpu_poisson_p_chan(dgpu_ctx *ctx);
 
 /* APPLY_BC_VEL_MPI (for/mpi.f:1371-1385 -> for/channel.f:2285-2492) on the
