@@ -107,6 +107,7 @@ struct dgpu_ctx {
     cx<double> *d_pairs = nullptr;
     int npairs = 0;
     double *d_les = nullptr;   // LES: NU_T, wall rows, saved rows, per-row constants
+    int les_chunk = 0;         // planes per block of k_les_prod
     bool les = false, les_model = false;  // input.dat's LES; les_chan called in each substep
     // CN tables: [stage 0..2][sys][NY+2][kRow]
     double *d_cn = nullptr;
@@ -1268,6 +1269,7 @@ static int ensure_les(dgpu_ctx *c)
     void *mem = nullptr;
     HIPCHK(c, hipMalloc(&mem, bytes));
     c->d_les = reinterpret_cast<double *>(mem);
+    c->les_chunk = dgpu::les_prod_auto_chunk(g, c->ipx64, g.nth ? std::min(2, c->jstart_th[0]) : 2, NY);
     // NU_T starts at zero; its rows outside k_les_prod's stay zero
     HIPCHK(c, hipMemsetAsync(mem, 0, bytes, c->stream));
     // per-row constants; filter widths with -2 C_SMAG^2 absorbed
@@ -1335,7 +1337,8 @@ static int les_terms(dgpu_ctx *c, int jlo, bool force)
     for (int q = 0; q < src.n; ++q) a.pr[q] = pair_buf(c, q);
     a.bc = m.bc; a.nut = m.nut; a.wt = c->d_wt; a.wt_fs = c->zfs; a.tab = m.tab;
     a.cu1 = c->cu[0]; a.cu3 = c->cu[2]; a.kx = c->d_kx; a.ps = g.ps;
-    a.ny = g.ny; a.nz = g.nz; a.jlo = jlo; a.jhi = g.ny; a.force = force ? 1 : 0;
+    a.ny = g.ny; a.nz = g.nz; a.jlo = jlo; a.jhi = g.ny;
+    a.chunk = c->les_chunk; a.force = force ? 1 : 0;
     dgpu::launch_les_prod(c->stream, g, c->ipx64, c->d_pairtw, c->ld, a);
     if (int rc = check_launch(c, "les_prod")) return rc;
     if (!force) {

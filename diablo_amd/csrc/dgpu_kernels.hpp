@@ -308,9 +308,11 @@ struct LesProd {
     const cx<double> *cu1, *cu3;  // mean profiles: mode 0
     const double *kx;
     long ps;
-    int ny, nz, jlo, jhi, chunk, zr, force;
+    int ny, nz, jlo, jhi, chunk, zr, force;  // chunk: planes per block
 };
 void launch_les_prod(hipStream_t s, const Geo &g, const IpLen &fx, const cx<double> *tw, int ld, const LesProd &a);
+// Planes per block of launch_les_prod by the rule.
+int les_prod_auto_chunk(const Geo &g, const IpLen &fx, int jlo, int jhi);
 void launch_les_addcf(hipStream_t s, const Geo &g, cx<double> *cf, const cx<double> *f);
 void launch_les_nut_out(hipStream_t s, const Geo &g, const double *nut, const int *zpos, const int *slot,
                         double *fort);

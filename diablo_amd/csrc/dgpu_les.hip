@@ -376,15 +376,20 @@ __global__ void __launch_bounds__(WIDE ? 768 : 384) __attribute__((amdgpu_waves_
     }
 }
 
+// pick: nothing is launched, *pick receives the rule's planes per block (the x
+// kernel's, dgpu_hot_x.hip: this kernel's blocks run c + 2 iterations, and the
+// rule's shape is within 4 % of the best of 1, 2, 3, 4, 5, 6, 8, 11, 16, 22, 32, 43,
+// 64 and 129 planes, whole LES steps at eleven sizes from 32x33x32 to 384x257x384).
 // LM: threads a position is shared out over, in units of the transforms' own
 // (2: one position a thread up to 12 values a transform thread).  WIDE: rows of
 // more than 384 threads (NX above 512 or so), one unit.
 template <int E, int NTH, int PID, int LM = (E > XCount<NTH>::npo ? 2 : 1), bool WIDE = false>
-static void les_prod_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<double> *tw, int ld, LesProd a)
+static void les_prod_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<double> *tw, int ld, LesProd a,
+                       int *pick)
 {
     constexpr int npo = XCount<NTH>::npo;
     if constexpr (!WIDE && PID == 0)
-        if (LM * npo * fx.t > 384) return les_prod_e<E, NTH, PID, 1, true>(s, g, fx, tw, ld, a);
+        if (LM * npo * fx.t > 384) return les_prod_e<E, NTH, PID, 1, true>(s, g, fx, tw, ld, a, pick);
     // short rows are packed as in the fused x kernel
     const size_t stash =  // a z row's
         WIDE ? 0 : sizeof(double) * kStash * ((E + LM * npo - 1) / (LM * npo)) * LM * npo * fx.t;
@@ -398,25 +403,44 @@ static void les_prod_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<do
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_les_prod<E, NTH, PID, LM, WIDE>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     const long rows = (g.nz + a.zr - 1) / a.zr;
-    const int planes = a.jhi - a.jlo + 1;
-    a.chunk = sweep_rule(rows, &planes, 1, kernel_slots(&k_les_prod<E, NTH, PID, LM, WIDE>, threads, lds));
+    if (pick) {
+        const int planes = a.jhi - a.jlo + 1;
+        *pick = sweep_rule(rows, &planes, 1, kernel_slots(&k_les_prod<E, NTH, PID, LM, WIDE>, threads, lds));
+        return;
+    }
     const int nchunks = (a.jhi - a.jlo + a.chunk) / a.chunk;
     hipLaunchKernelGGL((k_les_prod<E, NTH, PID, LM, WIDE>), dim3((unsigned)rows, nchunks), dim3(threads), lds, s, fx, tw, g.mk,
                        ld, a);
 }
 
-void launch_les_prod(hipStream_t s, const Geo &g, const IpLen &fx, const cx<double> *tw, int ld, const LesProd &a)
+static void les_prod_any(hipStream_t s, const Geo &g, const IpLen &fx, const cx<double> *tw, int ld,
+                         const LesProd &a, int *pick)
 {
     if (g.nth == 1 && with_pid(const_plan_id(fx), XPids64{}, [&](auto pc) {
             constexpr int P = decltype(pc)::value;
-            les_prod_e<kConstPlanSpecs[P].e, 1, P>(s, g, fx, tw, ld, a);
+            les_prod_e<kConstPlanSpecs[P].e, 1, P>(s, g, fx, tw, ld, a, pick);
         }))
         return;
     if (g.nth == 0) {
-        DGPU_DISPATCH_XE64(fx.e, (les_prod_e<EE, 0, 0>(s, g, fx, tw, ld, a)));
+        DGPU_DISPATCH_XE64(fx.e, (les_prod_e<EE, 0, 0>(s, g, fx, tw, ld, a, pick)));
     } else {
-        DGPU_DISPATCH_XE64(fx.e, (les_prod_e<EE, 1, 0>(s, g, fx, tw, ld, a)));
+        DGPU_DISPATCH_XE64(fx.e, (les_prod_e<EE, 1, 0>(s, g, fx, tw, ld, a, pick)));
     }
+}
+
+void launch_les_prod(hipStream_t s, const Geo &g, const IpLen &fx, const cx<double> *tw, int ld, const LesProd &a)
+{
+    les_prod_any(s, g, fx, tw, ld, a, nullptr);
+}
+
+int les_prod_auto_chunk(const Geo &g, const IpLen &fx, int jlo, int jhi)
+{
+    LesProd a{};
+    a.jlo = jlo;
+    a.jhi = jhi;
+    int c = 0;
+    les_prod_any(nullptr, g, fx, nullptr, 0, a, &c);
+    return c > 0 ? c : jhi - jlo + 1;
 }
 
 // CF1-3 (rows 2..NY) += the SGS force in the nonlinear-term slots x, y, z.
