@@ -49,7 +49,7 @@ struct dgpu_ctx {
     int ld = 0;      // row length of the intermediates (>= mk, multiple of 8)
     int xchunk = 64; // planes per block of the fused x kernel (xfused_auto_chunk's at creation)
     int colnw = 8;   // waves per block of the segmented column kernels; 0: whole-column sweeps
-    int colfuse = -1;     // fused column kernel: -1 where NY >= 160 (FP64: at 8 waves), 0 never, 1 where it fits
+    int colfuse = -1;     // fused column kernel: -1 where it is faster (fused_waves), 0 never, 1 where it fits
     // mixed paths: FP32 transforms, intermediates and nonlinear terms
     int mixed = 0;
     // DGPU_MIXED: FP32 working state [slot][j][K][I] (same slots as d_state's
@@ -1613,23 +1613,28 @@ static int seg_waves(const dgpu_ctx *c, int ny, bool fp32)
 }
 // The fused column kernel (dgpu_colseg.hip): the context's shape where the
 // column fits it, else 0.
-// Left to itself (colfuse -1) the fused kernel runs from NY = 160 up (six or
-// more rows per segment): on shorter columns its four solves in a row are
-// mostly barriers, and the separate kernels are faster.  In FP64 only at 8
-// waves: its 252 VGPRs and 131 KB of LDS (NY = 257) leave one block per CU,
-// and at 4 waves that is too few wavefronts (1.73 ms against 1.22 at 8 and
-// 1.24 for the two kernels, 384 x 257 x 384).
+// Left to itself (colfuse -1) the fused kernel runs where it is the faster:
+// - on tall columns, NY >= 160 (six or more rows per segment; on shorter ones
+//   its four solves in a row are mostly barriers).  In FP64 only at 8 waves: its
+//   236 VGPRs and 131 KB of LDS (NY = 257) leave one block per CU, and at 4 waves
+//   that is too few wavefronts (384 x 257 x 384: 1.73 ms where 8 waves took 1.22
+//   and the two kernels 1.24; 8 waves take 1.12 now);
+// - with the FP32 state also on the short columns that it cuts into 16 segments
+//   (NY <= 142): the 64-member ensemble 17.13k -> 17.65k Mpts*substeps/s against
+//   the two kernels;
+// - at 8 waves, on any column it fits, from 8192 modes up: a block is 32 modes at
+//   16 segments, 23 at 22 and 17 at 30, so that is one or two for each of the 256
+//   CUs, and the barriers of one block hide behind another's loads (a step of
+//   256x97x256 in FP64 1826 -> 1637 us, 384x129x384 5165 -> 4772, 384x150x384
+//   with the FP32 state 3200 -> 2936; even at 192x97x192, 8385 modes, and 474 ->
+//   478 and 230 -> 301 at 128 and 64).  In FP32 only this line decides at 142 <
+//   NY < 160: there the error of a step against 64 bits is 1.00 to 1.02 times that
+//   of the two kernels in L2 (192x{143,150,159}x192, both decks, three starts
+//   each; in the one value with the largest error 0.8 to 1.2 times, for the
+//   pressure 0.7 to 2.8).
 static int fused_waves(const dgpu_ctx *c, int ny)
 {
     if (!c->colnw) return 0;
-    // tall columns; with the FP32 state also the short ones the fused kernel
-    // cuts into 16 segments (NY <= 142): the 64-member ensemble 17.13k ->
-    // 17.65k Mpts*substeps/s against the two kernels.  Any column where the
-    // modes alone give a block or more per CU (one block is 32 of them): the
-    // barriers of one block then hide behind another's loads (8 waves, a step
-    // of 256x97x256 in FP64 1826 -> 1637 us, 384x129x384 5165 -> 4772,
-    // 384x150x384 with the FP32 state 3200 -> 2936; even at 192x97x192, and
-    // 474 -> 478 and 230 -> 301 at 128 and 64).
     const bool many = c->g.ps >= 8192 && c->colnw == 8;
     const bool auto_on =
         many || (ny >= 160 && (c->f32state || c->colnw == 8)) || (c->f32state && ny + 2 <= 144);

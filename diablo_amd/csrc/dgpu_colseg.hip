@@ -143,7 +143,6 @@ __device__ __forceinline__ void cn_rhs(int q, const CnMode<T> &K, TB &&tb, cx<T>
                                        cx<T> aux2, cx<T> thm, cx<T> cp0, cx<T> cpm, cx<T> nlv, cx<T> cfo,
                                        cx<T> &cfn, cx<T> &vec)
 {
-    const cx<T> zero = make_cx<T>(0, 0);
     const T visc = (q == SYS_TH0) ? K.nupr * K.pw : K.nu * K.pw;
     cfn = make_cx<T>(-(visc * f0.re), -(visc * f0.im));
     if (q == SYS_U1) {
@@ -1122,7 +1121,7 @@ void launch_remdiv_seg_batch(hipStream_t s, int nw, const Geo &g, int max_ny, co
 }
 
 // The fused column kernel (fused_nseg(NY) segments of at most 9 rows), FP32
-// state or FP64 (there at two waves per SIMD: 252 VGPRs, and the three
+// state or FP64 (there at two waves per SIMD: 236 VGPRs, and the three
 // systems' tables take 81 KB of LDS at NY = 257, so 4 or 8 waves per block).
 // A round of resident blocks is latency-bound, so the mode count per block
 // sets the number of rounds: at 384x257x384 (33153 modes, one FP64 block of
@@ -1142,7 +1141,7 @@ static size_t colfused_lds(int ny, int nw)
 template <typename T>
 bool colfused_supported(int ny, int nw)
 {
-    // FP64 blocks of 16 waves would hold its 252 VGPRs in 128 (spills)
+    // FP64 blocks of 16 waves would hold its 236 VGPRs in 128 (spills)
     const int nseg = fused_nseg(ny);
     return (nw == 4 || nw == 8 || (nw == 16 && sizeof(T) == 4)) && ny >= 4 && (ny + 2 + nseg - 1) / nseg <= 9 &&
            colfused_lds<T>(ny, nw) <= 150 * 1024;

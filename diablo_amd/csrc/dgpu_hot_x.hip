@@ -484,12 +484,12 @@ static int xfused_zrows(const IpLen &fx, int nz, int mk)
 // counts.  Beyond it a round that is partly empty costs a whole one while the
 // rounds are few; over many rounds blocks even that out by half.  Among other
 // launches (the groups of an ensemble) what a round leaves empty they fill: the
-// iterations of all blocks, and a block at the end.  On small
-// grids the former fixed 64 (FP64) / 32 planes left most CUs without a block:
-// one RK3 step at 64x65x64 FP64 1005 -> 159 us (2 planes; the 64 were one block
-// of 63 a row), 192x129x192 2819 -> 1840, three members of 64x{33,65,97}x64
-// 1096 -> 351; at 384x257x384 the rule gives the 64 (FP64) and 32 (FP32) planes
-// measured best there.
+// iterations of all blocks, and a block at the end.  On small grids the former
+// fixed 64 (FP64) / 32 planes left most CUs without a block: one RK3 step at
+// 64x65x64 FP64 1005 -> 159 us (2 planes; the 64 were one block a row),
+// 192x129x192 2819 -> 1840, three members of 64x{33,65,97}x64 1096 -> 351; at
+// 384x257x384 the rule gives the 64 (FP64) and 32 (FP32) planes measured best
+// there.
 int sweep_rule(long rows, const int *planes, int runs, long slots, bool among)
 {
     const int most = *std::max_element(planes, planes + runs);

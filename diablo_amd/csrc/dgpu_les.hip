@@ -157,10 +157,11 @@ __global__ void k_les_bc_put(Geo g, cx<double> *__restrict__ p0, cx<double> *__r
 // values are on their way.  tab[j*8 + {0..6}]: 1/DYF, 1/DY, 1/(2 DYF),
 // DYF(j-1)/(2 DY), DYF(j)/(2 DY), -2 C^2 DELTA^2 on GYF, on GY.
 // force: the SGS force alone (dgpu_les_chan), no products and no scalar.
-// 384x257x384: 1.92 ms (5.6 GB: six pairs in, NU_T and eight row fields out, 2.9
-// TB/s; three waves per SIMD; 2.29 ms with two positions a thread, 256 registers
-// and 44 of them spilled); it replaces the x kernel (1.30 ms), nine plane transforms (2.9 ms) and seven pointwise
-// kernels (2.9 ms) of the Fortran-layout form.  Substep 18.1 -> 10.0 ms.
+// 384x257x384: 1.90-1.95 ms (counted 3.7 GB read, 1.9 written: six pairs in, NU_T
+// and eight row fields out, 2.9 TB/s; three waves per SIMD; 2.29 ms with two
+// positions a thread, 256 registers and 44 of them spilled); it replaces the x
+// kernel (1.30 ms), nine plane transforms (2.9 ms) and seven pointwise kernels
+// (2.9 ms) of the Fortran-layout form, a substep of 18.1 ms, now 7.9.
 // -------------------------------------------------------------------------
 constexpr int kStash = 8;
 template <int E, int NTH, int PID, int LM, bool WIDE>
@@ -551,7 +552,7 @@ __global__ void __launch_bounds__(512) k_les_cn_seg(Geo g, LesCnSet set, const d
     constexpr int NS = 32, NC = 16;
     __shared__ double eq[NS][6][NC];  // x(a): G, C, F; x(b): g, c, f -- then x(b+1), x(a-1)
     const int col = threadIdx.x & (NC - 1), seg = threadIdx.x / NC;
-    const long n = 2L * g.nx * g.nz;  // doubles a pair plane (a multiple of 16: NX, NZ are even and NX*NZ*2 >= 32)
+    const long n = 2L * g.nx * g.nz;  // doubles a pair plane; the last block's columns beyond it are off
     const long e0 = (long)blockIdx.x * NC + col;
     const bool on = e0 < n;
     const long e = on ? e0 : n - 1;

@@ -26,9 +26,11 @@
 // maximum is its mean, costs U1's fluctuations four times their round-off.
 //
 // Both kernels move 16 B per pair point and 16 B per kept row value: 384x257x384,
-// 6 pairs back in 1.23 ms (5.3 GB, 4.3 TB/s), 2 pairs forward in 0.43 (2.0 GB,
-// 4.7 TB/s), near the rate of a copy; three waves per SIMD hide the loads (at two,
-// before the dealiasing gap was known at compile time, 1.99 ms).  The standalone
+// 6 pairs back in 1.25-1.28 ms (counted 2.4 GB read, 3.7 written, 4.8 TB/s), 2 pairs
+// forward in 0.43 (1.2 + 0.8 GB, 4.7 TB/s), near the rate of a copy.  k_pairs_inv
+// holds both rows until their scale is known: 198 registers, two waves per SIMD
+// (1.23 ms at three without it; 25 to 32 registers spill when held to three, and
+// reading the rows twice, once for the scale, takes 1.77).  The standalone
 // transforms they replace took 0.33 ms per field and direction (Fortran-layout
 // planes, one real row per complex transform).
 #include "dgpu_hot.hpp"

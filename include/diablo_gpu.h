@@ -305,7 +305,7 @@ int32_t dgpu_set_zdft(dgpu_ctx *ctx, int32_t on);
  * FP64); 0 keeps the two kernels; -1 (the default; environment
  * DGPU_COLFUSE) fuses from NY = 160 up (in FP64 only at 8 waves) and, with
  * the FP32 state, up to NY = 142 (16 segments there, 22 up to NY = 196,
- * else 30); in both, at 8 waves, also any NY with 8192 (kx,kz) modes or more.  With the
+ * else 30); at 8 waves also at any NY from 8192 (kx,kz) modes up.  With the
  * FP32 state the fused kernel rounds differently from the two kernels (30
  * segments, not 16), within FP32 round-off; in FP64 (30 against 32
  * segments) they agree to round-off.  An RK stage 3 with a COURANT request runs the
