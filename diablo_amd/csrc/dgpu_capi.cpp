@@ -589,7 +589,7 @@ int32_t dgpu_create(const dgpu_params *p, dgpu_ctx **out)
             c->xchunk = std::atoi(xc);
         } else {
             const int planes = g.ny - (g.nth ? std::min(2, c->jstart_th[0]) : 2) + 1;
-            c->xchunk = c->mixed ? dgpu::xfused_auto_chunk<float>(g, c->ipx, &planes, 1, 1.0)
+            c->xchunk = c->mixed ? dgpu::xfused_auto_chunk<float>(g, c->ipx, &planes, 1, 1.0, c->f32state)
                                  : dgpu::xfused_auto_chunk<double>(g, c->ipx, &planes, 1, 1.0);
         }
     }
@@ -1677,7 +1677,7 @@ static int rk_enqueue(dgpu_ctx *c, int rk_step, double time, double temp1, doubl
         {
             TimerScope t(c, 1);
             dgpu::launch_xfused_ip<float>(c->stream, g, c->ipx, twx, c->ld, c->d_ztf, c->zfs, c->d_wtf, c->zfs,
-                                          c->d_dy, c->d_dyf, c->d_kx, jlo, g.ny, c->xchunk);
+                                          c->d_dy, c->d_dyf, c->d_kx, jlo, g.ny, c->xchunk, c->f32state);
         }
         if (int rc = check_launch(c, "xfused")) return rc;
         {
@@ -2323,7 +2323,7 @@ static void ens_group_chunks(dgpu_ensemble *e)
         const double share = e->group_streams ? own / all : 1.0;
         const int n = (int)planes.size();
         gr.xchunk = xc && std::atoi(xc) > 0 ? std::atoi(xc)
-                    : c0->mixed ? dgpu::xfused_auto_chunk<float>(c0->g, c0->ipx, planes.data(), n, share)
+                    : c0->mixed ? dgpu::xfused_auto_chunk<float>(c0->g, c0->ipx, planes.data(), n, share, c0->f32state)
                                 : dgpu::xfused_auto_chunk<double>(c0->g, c0->ipx, planes.data(), n, share);
     }
 }
@@ -2530,7 +2530,7 @@ static int ens_enqueue_batched(dgpu_ensemble *e, int rk_step)
                                                           (const dgpu::ZinvDesc<float, double> *)gr.d_zinv, nm,
                                                           gr.max_planes, c0->ld, nin);
             dgpu::launch_xfused_ip_batch<float>(s, g, c0->ipx, twx, (const dgpu::XfDesc<float> *)gr.d_xf, nm,
-                                                gr.max_span, c0->ld, gr.xchunk);
+                                                gr.max_span, c0->ld, gr.xchunk, f32);
             dgpu::launch_zfwd_nl_ip_batch<float, float>(s, g, c0->ipz, twz,
                                                         (const dgpu::ZfDesc<float, float> *)gr.d_zf, nm, gr.max_zf,
                                                         c0->ld, nin);

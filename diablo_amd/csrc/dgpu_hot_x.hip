@@ -26,8 +26,15 @@ namespace dgpu {
 // twiddles, the kept modes' KX.  Transform positions sit at swizzled slots
 // (ip_swz) of their rows; the products read and write slot by slot, which is
 // position by position in the same permutation for every row.
+//
+// FIX: the fused product of every sum of two is named (dgpu_fft.hpp), so the
+// results are the same bits for any number of planes per block, single or
+// batched, on run-time or compile-time plans.  DGPU_MIXED_F64STATE runs leave
+// it to the compiler: their FP64 state carries this kernel's FP32 round-off, so
+// other forms of it move their results by 1e-5 of a nonlinear term, where an FP64
+// or an FP32 state moves by its own round-off.
 // -------------------------------------------------------------------------
-template <typename T, int E, int NTH, bool CP, bool MZ>
+template <typename T, int E, int NTH, bool CP, bool MZ, bool FIX>
 __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__restrict__ twg, int mk_rt, int ld,
                                             const cx<T> *__restrict__ zt, long zt_fs, long zt_ps,
                                             cx<T> *__restrict__ wt, long wt_fs, long wt_ps,
@@ -50,6 +57,8 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
     // thread's inputs and outputs lie in the dealiasing gap is known: their
     // loads, selects and stores go
     const int mk = CP ? nx / 3 + 1 : mk_rt;
+    // a b + c d with the first product fused into the second
+    auto sum2 = [](T a, T b, T c, T d) { return FIX ? fma_(a, b, c * d) : a * b + c * d; };
     const int tid = threadIdx.x, nthr = blockDim.x;
     const int pg = tid / TT, zs = MZ ? pg / nrow : 0;
     const int p = pg - zs * nrow;
@@ -92,7 +101,7 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
     const bool lin = CP && ip_bits_apart<E, R0>(fx, 0);
     auto dif0 = [&](cx<T> *row) {
         const int s0 = ip_swz(fx, th);
-        ip_stage<T, E, R0, +1, true, true>(
+        ip_stage<T, E, R0, +1, true, FIX>(
             fx, 0, tw, th,
             [&](int idx, int f) {
                 cx<T> A = pa[idx], B = pb[idx];
@@ -121,8 +130,8 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
             va[q] = row[lin ? ip_slot(fx, sa, q * L0) : ip_swz(fx, ga + q * L0)];
             vb[q] = row[lin ? ip_slot(fx, sb, q * L0) : ip_swz(fx, gb + q * L0)];
         }
-        ip_group<T, R0, -1, false, true>(va, tw + fx.twoff[0], ga);
-        ip_group<T, R0, -1, false, true>(vb, tw + fx.twoff[0], gb);
+        ip_group<T, R0, -1, false, FIX>(va, tw + fx.twoff[0], ga);
+        ip_group<T, R0, -1, false, FIX>(vb, tw + fx.twoff[0], gb);
         const T h = T(0.5) / T(nx);
         cx<T> *o0 = wt + (long)j * wt_ps + zrow;
         // Outputs of pair row r (field slots of wt): G1 | G2 | G3, H1 | H2, H3
@@ -135,13 +144,13 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
         const long off2 = (long)(r == 2 ? 1 : 5) * wt_fs;
         const bool two = r == 2 || r == 3, xa1 = r == 3 || r == 5;
         auto emit = [&](int kp, cx<T> Zk, cx<T> Zn) {
-#pragma clang fp contract(off)
             if (!zvalid) return;
             const cx<T> Xa = make_cx<T>((Zk.re + Zn.re) * h, (Zk.im - Zn.im) * h);
             const cx<T> Xb = make_cx<T>((Zk.im + Zn.im) * h, -(Zk.re - Zn.re) * h);
             const T kx = kxs[kp];
             // -(i kx Xa + Xb)
-            const cx<T> G = make_cx<T>(fma_(kx, Xa.im, -Xb.re), fma_(-kx, Xa.re, -Xb.im));
+            const cx<T> G = FIX ? make_cx<T>(fma_(kx, Xa.im, -Xb.re), fma_(-kx, Xa.re, -Xb.im))
+                                : make_cx<T>(kx * Xa.im - Xb.re, -kx * Xa.re - Xb.im);
             const cx<T> nXa = make_cx<T>(-Xa.re, -Xa.im), nXb = make_cx<T>(-Xb.re, -Xb.im);
             if constexpr (sizeof(T) == 4) {
                 o0[off1 + kp] = xa1 ? nXa : G;
@@ -180,7 +189,6 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
         const int extra = npos % nthr;
         const int e0 = extra ? (tid + nthr - extra) % nthr : tid;
         for (int e = e0; e < npos; e += nthr) {
-#pragma clang fp contract(off)
             const int zq = e / nx, x = e - zq * nx;
             cx<T> *const zw = base + zq * zsz;
             const cx<T> *wm = zw + ((j - 1) % 3) * npi * nx, *w0 = zw + (j % 3) * npi * nx,
@@ -194,12 +202,12 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
             const T p0 = u3 * u1;                                                      // U1*U3
             const T p1 = u1 * u1;                                                      // U1*U1
             const T p2 = u3 * u3;                                                      // U3*U3
-            const T p3 = (fma_(dyfj, u1, dyfm * u1m) * r2dy) * u2;               // U1*U2 at GY
-            const T p4 = (fma_(dyfj, u3, dyfm * u3m) * r2dy) * u2;               // U3*U2 at GY
-            // up u2p + u0 u2p, less u0 u2 + um u2
-            auto less = [&](T f, T u0, T um) { return fma_(-um, u2, fma_(-u0, u2, f)); };
-            const T p5 = less(fma_(u1p, u2p, u1 * u2p), u1, u1m) * r2dyf;        // d/dy(U1 U2)
-            const T p6 = less(fma_(u3, u2p, u3p * u2p), u3, u3m) * r2dyf;        // d/dy(U3 U2)
+            const T p3 = (sum2(dyfj, u1, dyfm, u1m) * r2dy) * u2;                // U1*U2 at GY
+            const T p4 = (sum2(dyfj, u3, dyfm, u3m) * r2dy) * u2;                // U3*U2 at GY
+            // a u2p + b u2p, less u0 u2 + um u2
+            auto less = [&](T f, T u0, T um) { return FIX ? fma_(-um, u2, fma_(-u0, u2, f)) : f - u0 * u2 - um * u2; };
+            const T p5 = less(sum2(u1p, u2p, u1, u2p), u1, u1m) * r2dyf;         // d/dy(U1 U2)
+            const T p6 = less(FIX ? sum2(u3, u2p, u3p, u2p) : sum2(u3p, u2p, u3, u2p), u3, u3m) * r2dyf;  // d/dy(U3 U2)
             const T sp = u2 + u2p, sm = u2 + u2m;
             const T p7 = (T(0.25) * (sp * sp) - T(0.25) * (sm * sm)) * rdy;      // d/dy(U2 U2)
             fq[0 * nx + x] = make_cx<T>(p1, p5);
@@ -210,7 +218,7 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
                 const T t0 = b0.im, tm = bm.im, tp = bp.im;
                 const T p8 = t0 * u1;
                 const T p9 = t0 * u3;
-                const T p10 = less(fma_(t0, u2p, tp * u2p), t0, tm) * r2dyf;
+                const T p10 = less(FIX ? sum2(t0, u2p, tp, u2p) : sum2(tp, u2p, t0, u2p), t0, tm) * r2dyf;
                 fq[4 * nx + x] = make_cx<T>(p8, p10);
                 fq[5 * nx + x] = make_cx<T>(p9, T(0));
             }
@@ -228,7 +236,7 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
     if (pro) dif0(slot_row(pro_plane, pro_pair));
     __syncthreads();
     stage_loop<CP>(1, S, [&](int s) {
-        if (pro) ip_stage_row<T, E, +1, true, CP, true>(slot_row(pro_plane, pro_pair), fx, s, tw, th);
+        if (pro) ip_stage_row<T, E, +1, true, CP, FIX>(slot_row(pro_plane, pro_pair), fx, s, tw, th);
         __syncthreads();
     });
     if (dif_row) {
@@ -272,8 +280,8 @@ __device__ __forceinline__ void xfused_body(const IpLen &fx, const cx<T> *__rest
                 asm volatile("" : "+v"(th));
                 __builtin_assume(th >= 0 && th < TT);
             }
-            if (inv) ip_stage_row<T, E, +1, true, CP, true>(drow, fx, s + 1, tw, th);
-            if (fwd) ip_stage_row<T, E, -1, false, CP, true>(frow, fx, S - 1 - s, tw, th);
+            if (inv) ip_stage_row<T, E, +1, true, CP, FIX>(drow, fx, s + 1, tw, th);
+            if (fwd) ip_stage_row<T, E, -1, false, CP, FIX>(frow, fx, S - 1 - s, tw, th);
             row_sync();
         });
         if (fwd) dit_out(frow, p - npi, j - 1);
@@ -303,7 +311,7 @@ constexpr bool xf_multi(int pid)
 // FP32 with the 384 plan: four resident blocks per CU (LDS holds four FP32
 // windows at NX = 384, 40 KB each) at the cost of a few spilled registers;
 // FP64 stays at the two its LDS allows.
-template <typename T, int E, int NTH, int PID>
+template <typename T, int E, int NTH, int PID, bool FIX>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && PID == 17 ? 4 : 2)))
 k_xfused_ip(IpLen fx, const cx<T> *__restrict__ twg, int mk, int ld,
                                                     const cx<T> *__restrict__ zt, long zt_fs, long zt_ps,
@@ -312,19 +320,19 @@ k_xfused_ip(IpLen fx, const cx<T> *__restrict__ twg, int mk, int ld,
                                                     const double *__restrict__ kxv, int jlo, int jhi, int chunk,
                                                     int zr, int nz)
 {
-    xfused_body<T, E, NTH, PID != 0, xf_multi<T>(PID)>(plan_ref<PID>(fx), twg, mk, ld, zt, zt_fs, zt_ps, wt, wt_fs, wt_ps,
+    xfused_body<T, E, NTH, PID != 0, xf_multi<T>(PID), FIX>(plan_ref<PID>(fx), twg, mk, ld, zt, zt_fs, zt_ps, wt, wt_fs, wt_ps,
                                                      dy, dyf, kxv, jlo, jhi, chunk, blockIdx.x, blockIdx.y, zr, nz);
 }
 
 // grid (z-row groups, chunks of the tallest member, members)
-template <typename T, int E, int NTH, int PID>
+template <typename T, int E, int NTH, int PID, bool FIX>
 __global__ void __launch_bounds__(512) k_xfused_ip_batch(const XfDesc<T> *__restrict__ d, IpLen fx,
                                                           const cx<T> *__restrict__ twg, int mk, int ld, long ps,
                                                           int chunk, int zr, int nz)
 {
     const XfDesc<T> D = d[blockIdx.z];
     if ((int)blockIdx.y * chunk > D.jhi - D.jlo) return;
-    xfused_body<T, E, NTH, PID != 0, xf_multi<T>(PID)>(plan_ref<PID>(fx), twg, mk, ld, D.zt, D.zt_fs, ps, D.wt, D.wt_fs,
+    xfused_body<T, E, NTH, PID != 0, xf_multi<T>(PID), FIX>(plan_ref<PID>(fx), twg, mk, ld, D.zt, D.zt_fs, ps, D.wt, D.wt_fs,
                                                     ps, D.dy, D.dyf, D.kx, D.jlo, D.jhi, chunk, blockIdx.x, blockIdx.y, zr,
                                                     nz);
 }
@@ -520,7 +528,18 @@ struct XPick {
     double share;       // of the device that the launch has to itself
     int chunk;
 };
-template <typename T, int E, int NTH, int PID>
+// fn(std::integral_constant<bool, named>): the kernels that leave the fused
+// products open exist in FP32 only
+template <typename T, class F>
+static void with_named(bool named, F &&fn)
+{
+    if constexpr (sizeof(T) == 4) {
+        if (!named) return fn(std::false_type{});
+    }
+    fn(std::true_type{});
+}
+
+template <typename T, int E, int NTH, int PID, bool FIX>
 static void xfused_ip_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, int ld, const cx<T> *zt,
                         long zt_fs, cx<T> *wt, long wt_fs, const double *dy, const double *dyf, const double *kx,
                         int jlo, int jhi, int chunk, XPick *pick)
@@ -532,44 +551,44 @@ static void xfused_ip_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T
         sizeof(cx<T>) * ((size_t)zr * fx.n * (3 * C::npi + C::npo) + fx.twn) + sizeof(T) * g.mk;
     static bool attr = false;
     if (!attr) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_xfused_ip<T, E, NTH, PID>),
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_xfused_ip<T, E, NTH, PID, FIX>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         attr = true;
     }
     if (pick) {
-        const long slots = kernel_slots(&k_xfused_ip<T, E, NTH, PID>, threads, lds);
+        const long slots = kernel_slots(&k_xfused_ip<T, E, NTH, PID, FIX>, threads, lds);
         pick->chunk = sweep_rule((g.nz + zr - 1) / zr, pick->planes, pick->runs,
                                  std::max(1L, (long)(slots * pick->share)), pick->share < 1.0);
         return;
     }
     const int nchunks = (jhi - jlo + 1 + chunk - 1) / chunk;
     const long ps = (long)g.nz * ld;
-    hipLaunchKernelGGL((k_xfused_ip<T, E, NTH, PID>), dim3((g.nz + zr - 1) / zr, nchunks), dim3(threads), lds, s, fx,
+    hipLaunchKernelGGL((k_xfused_ip<T, E, NTH, PID, FIX>), dim3((g.nz + zr - 1) / zr, nchunks), dim3(threads), lds, s, fx,
                        tw, g.mk, ld, zt, zt_fs, ps, wt, wt_fs, ps, dy, dyf, kx, jlo, jhi, chunk, zr, g.nz);
 }
 
 
 // The x kernels are built for the compile-time plans with one scalar; other
 // shapes run on run-time plans.
-template <typename T>
+template <typename T, bool FIX>
 static void xfused_ip_any(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, int ld, const cx<T> *zt,
                           long zt_fs, cx<T> *wt, long wt_fs, const double *dy, const double *dyf, const double *kx,
                           int jlo, int jhi, int chunk, XPick *pick)
 {
     if (g.nth == 1 && with_pid(const_plan_id(fx), XPids<T>{}, [&](auto pc) {
             constexpr int P = decltype(pc)::value;
-            xfused_ip_e<T, kConstPlanSpecs[P].e, 1, P>(s, g, fx, tw, ld, zt, zt_fs, wt, wt_fs, dy, dyf, kx, jlo, jhi,
-                                                       chunk, pick);
+            xfused_ip_e<T, kConstPlanSpecs[P].e, 1, P, FIX>(s, g, fx, tw, ld, zt, zt_fs, wt, wt_fs, dy, dyf, kx, jlo,
+                                                            jhi, chunk, pick);
         }))
         return;
 #define DGPU_XF(EE_)                                                                                             \
     do {                                                                                                         \
         if (g.nth == 0)                                                                                          \
-            xfused_ip_e<T, EE_, 0, 0>(s, g, fx, tw, ld, zt, zt_fs, wt, wt_fs, dy, dyf, kx, jlo, jhi, chunk,      \
-                                      pick);                                                                     \
+            xfused_ip_e<T, EE_, 0, 0, FIX>(s, g, fx, tw, ld, zt, zt_fs, wt, wt_fs, dy, dyf, kx, jlo, jhi, chunk, \
+                                           pick);                                                                \
         else                                                                                                     \
-            xfused_ip_e<T, EE_, 1, 0>(s, g, fx, tw, ld, zt, zt_fs, wt, wt_fs, dy, dyf, kx, jlo, jhi, chunk,      \
-                                      pick);                                                                     \
+            xfused_ip_e<T, EE_, 1, 0, FIX>(s, g, fx, tw, ld, zt, zt_fs, wt, wt_fs, dy, dyf, kx, jlo, jhi, chunk, \
+                                           pick);                                                                \
     } while (0)
     switch (fx.e) {
     case 4: DGPU_XF(4); break;
@@ -587,20 +606,26 @@ static void xfused_ip_any(hipStream_t s, const Geo &g, const IpLen &fx, const cx
 template <typename T>
 void launch_xfused_ip(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, int ld, const cx<T> *zt,
                       long zt_fs, cx<T> *wt, long wt_fs, const double *dy, const double *dyf, const double *kx,
-                      int jlo, int jhi, int chunk)
+                      int jlo, int jhi, int chunk, bool named)
 {
-    xfused_ip_any<T>(s, g, fx, tw, ld, zt, zt_fs, wt, wt_fs, dy, dyf, kx, jlo, jhi, chunk, nullptr);
+    with_named<T>(named, [&](auto fix) {
+        xfused_ip_any<T, decltype(fix)::value>(s, g, fx, tw, ld, zt, zt_fs, wt, wt_fs, dy, dyf, kx, jlo, jhi, chunk,
+                                               nullptr);
+    });
 }
 
 template <typename T>
-int xfused_auto_chunk(const Geo &g, const IpLen &fx, const int *planes, int runs, double share)
+int xfused_auto_chunk(const Geo &g, const IpLen &fx, const int *planes, int runs, double share, bool named)
 {
     XPick p{planes, runs, share, 0};
-    xfused_ip_any<T>(nullptr, g, fx, nullptr, 0, nullptr, 0, nullptr, 0, nullptr, nullptr, nullptr, 0, 0, 1, &p);
+    with_named<T>(named, [&](auto fix) {
+        xfused_ip_any<T, decltype(fix)::value>(nullptr, g, fx, nullptr, 0, nullptr, 0, nullptr, 0, nullptr, nullptr,
+                                               nullptr, 0, 0, 1, &p);
+    });
     return p.chunk > 0 ? p.chunk : 32;
 }
 
-template <typename T, int E, int NTH, int PID>
+template <typename T, int E, int NTH, int PID, bool FIX>
 static void xfused_ip_batch_e(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, const XfDesc<T> *d,
                               int nmem, int max_span, int ld, int chunk)
 {
@@ -611,30 +636,30 @@ static void xfused_ip_batch_e(hipStream_t s, const Geo &g, const IpLen &fx, cons
         sizeof(cx<T>) * ((size_t)zr * fx.n * (3 * C::npi + C::npo) + fx.twn) + sizeof(T) * g.mk;
     static bool attr = false;
     if (!attr) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_xfused_ip_batch<T, E, NTH, PID>),
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&k_xfused_ip_batch<T, E, NTH, PID, FIX>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         attr = true;
     }
     dim3 grid((g.nz + zr - 1) / zr, (max_span + chunk - 1) / chunk, nmem);
-    hipLaunchKernelGGL((k_xfused_ip_batch<T, E, NTH, PID>), grid, dim3(threads), lds, s, d, fx, tw, g.mk, ld,
+    hipLaunchKernelGGL((k_xfused_ip_batch<T, E, NTH, PID, FIX>), grid, dim3(threads), lds, s, d, fx, tw, g.mk, ld,
                        (long)g.nz * ld, chunk, zr, g.nz);
 }
 
-template <typename T>
-void launch_xfused_ip_batch(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, const XfDesc<T> *d,
-                            int nmem, int max_span, int ld, int chunk)
+template <typename T, bool FIX>
+static void xfused_ip_batch_any(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, const XfDesc<T> *d,
+                                int nmem, int max_span, int ld, int chunk)
 {
     if (g.nth == 1 && with_pid(const_plan_id(fx), XPids<T>{}, [&](auto pc) {
             constexpr int P = decltype(pc)::value;
-            xfused_ip_batch_e<T, kConstPlanSpecs[P].e, 1, P>(s, g, fx, tw, d, nmem, max_span, ld, chunk);
+            xfused_ip_batch_e<T, kConstPlanSpecs[P].e, 1, P, FIX>(s, g, fx, tw, d, nmem, max_span, ld, chunk);
         }))
         return;
 #define DGPU_XFB(EE_)                                                                               \
     do {                                                                                            \
         if (g.nth == 0)                                                                             \
-            xfused_ip_batch_e<T, EE_, 0, 0>(s, g, fx, tw, d, nmem, max_span, ld, chunk);            \
+            xfused_ip_batch_e<T, EE_, 0, 0, FIX>(s, g, fx, tw, d, nmem, max_span, ld, chunk);       \
         else                                                                                        \
-            xfused_ip_batch_e<T, EE_, 1, 0>(s, g, fx, tw, d, nmem, max_span, ld, chunk);            \
+            xfused_ip_batch_e<T, EE_, 1, 0, FIX>(s, g, fx, tw, d, nmem, max_span, ld, chunk);       \
     } while (0)
     switch (fx.e) {
     case 4: DGPU_XFB(4); break;
@@ -647,6 +672,15 @@ void launch_xfused_ip_batch(hipStream_t s, const Geo &g, const IpLen &fx, const 
     default: break;
     }
 #undef DGPU_XFB
+}
+
+template <typename T>
+void launch_xfused_ip_batch(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, const XfDesc<T> *d,
+                            int nmem, int max_span, int ld, int chunk, bool named)
+{
+    with_named<T>(named, [&](auto fix) {
+        xfused_ip_batch_any<T, decltype(fix)::value>(s, g, fx, tw, d, nmem, max_span, ld, chunk);
+    });
 }
 
 int vmax_rows_per_block(const IpLen &fx) { return 256 / (2 * fx.t); }
@@ -683,20 +717,20 @@ void launch_vmax_ip(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *t
     DGPU_DISPATCH_IPE(fx.e, (vmax_ip_e<T, EE>(s, g, fx, tw, ld, zt, zt_fs, part, out)));
 }
 
-template int xfused_auto_chunk<double>(const Geo &, const IpLen &, const int *, int, double);
-template int xfused_auto_chunk<float>(const Geo &, const IpLen &, const int *, int, double);
+template int xfused_auto_chunk<double>(const Geo &, const IpLen &, const int *, int, double, bool);
+template int xfused_auto_chunk<float>(const Geo &, const IpLen &, const int *, int, double, bool);
 template void launch_vmax_ip<double>(hipStream_t, const Geo &, const IpLen &, const cx<double> *, int,
                                      const cx<double> *, long, double *, double *);
 template void launch_vmax_ip<float>(hipStream_t, const Geo &, const IpLen &, const cx<float> *, int,
                                     const cx<float> *, long, double *, double *);
 template void launch_xfused_ip_batch<double>(hipStream_t, const Geo &, const IpLen &, const cx<double> *,
-                                             const XfDesc<double> *, int, int, int, int);
+                                             const XfDesc<double> *, int, int, int, int, bool);
 template void launch_xfused_ip_batch<float>(hipStream_t, const Geo &, const IpLen &, const cx<float> *,
-                                            const XfDesc<float> *, int, int, int, int);
+                                            const XfDesc<float> *, int, int, int, int, bool);
 template void launch_xfused_ip<double>(hipStream_t, const Geo &, const IpLen &, const cx<double> *, int,
                                        const cx<double> *, long, cx<double> *, long, const double *, const double *,
-                                       const double *, int, int, int);
+                                       const double *, int, int, int, bool);
 template void launch_xfused_ip<float>(hipStream_t, const Geo &, const IpLen &, const cx<float> *, int,
                                       const cx<float> *, long, cx<float> *, long, const double *, const double *,
-                                      const double *, int, int, int);
+                                      const double *, int, int, int, bool);
 }  // namespace dgpu

@@ -163,14 +163,16 @@ struct ZfDesc {
 template <typename T, typename TIN>
 void launch_zinv_ip(hipStream_t s, const Geo &g, const IpLen &fz, const cx<T> *tw, const cx<TIN> *in, long in_fs,
                     long in_ps, cx<T> *out, long out_fs, long out_ps, int ld, int j0, int nplanes, int nfields);
+// named: the fused product of each sum is named (dgpu_hot_x.hip); false only in
+// FP32, for a DGPU_MIXED_F64STATE run.
 template <typename T>
 void launch_xfused_ip(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, int ld, const cx<T> *zt,
                       long zt_fs, cx<T> *wt, long wt_fs, const double *dy, const double *dyf, const double *kx,
-                      int jlo, int jhi, int chunk);
+                      int jlo, int jhi, int chunk, bool named = true);
 // Planes per block of launch_xfused_ip, or of its batch over `runs` members, by
 // the rule (dgpu_hot_x.hip), for a launch that has `share` of the device.
 template <typename T>
-int xfused_auto_chunk(const Geo &g, const IpLen &fx, const int *planes, int runs, double share);
+int xfused_auto_chunk(const Geo &g, const IpLen &fx, const int *planes, int runs, double share, bool named = true);
 template <typename T, typename TOUT>
 void launch_zfwd_nl_ip(hipStream_t s, const Geo &g, const IpLen &fz, const cx<T> *tw, const cx<T> *wt, long wt_fs,
                        int ld, cx<TOUT> *const *nl, const double *kz, int jlo, int jhi, int nout);
@@ -179,7 +181,7 @@ void launch_zinv_ip_batch(hipStream_t s, const Geo &g, const IpLen &fz, const cx
                           int nmem, int max_planes, int ld, int nfields);
 template <typename T>
 void launch_xfused_ip_batch(hipStream_t s, const Geo &g, const IpLen &fx, const cx<T> *tw, const XfDesc<T> *d,
-                            int nmem, int max_span, int ld, int chunk);
+                            int nmem, int max_span, int ld, int chunk, bool named = true);
 template <typename T, typename TOUT>
 void launch_zfwd_nl_ip_batch(hipStream_t s, const Geo &g, const IpLen &fz, const cx<T> *tw, const ZfDesc<T, TOUT> *d,
                              int nmem, int max_planes, int ld, int nout);

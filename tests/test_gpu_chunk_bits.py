@@ -48,3 +48,34 @@ def test_bits_of_the_x_kernel(monkeypatch, size, precision):
     ens.synchronize()
     _same(ens.members[0].state(), ref, "ensemble")
     ens.close()
+
+
+@pytest.mark.parametrize("size", SIZES)
+def test_f64state_keeps_its_accuracy(monkeypatch, size):
+    """mixed_f64state runs have x kernels of their own, whose bits may depend on
+    the planes per block: the state stays within FP32 round-off of the nonlinear
+    terms (64 eps of them, and they move the state by at most a tenth of itself
+    in two steps: 8e-7) of the FP64 run for any number of planes."""
+    nx, ny, nz = size
+    print(size, flush=True)
+    cfg = case.channel_case(nx, ny, nz, kick=0.3, streak=0.1)
+    start = case.initial_physical(cfg)
+
+    def run(precision, chunk):
+        if chunk:
+            monkeypatch.setenv("DGPU_XCHUNK", str(chunk))
+        else:
+            monkeypatch.delenv("DGPU_XCHUNK", raising=False)
+        g = gpu.GpuChannel(cfg, precision=precision)
+        g.initialize(*start)
+        g.step(2)
+        s = g.state()
+        g.close()
+        return s
+
+    ref = run("fp64", 0)
+    for chunk in (0, 1, 3, 64):
+        s = run("mixed_f64state", chunk)
+        for k in ("CU1", "CU3", "CTH0"):
+            err = np.linalg.norm(s[k] - ref[k]) / np.linalg.norm(ref[k])
+            assert err <= 8e-7, (chunk, k, err)
