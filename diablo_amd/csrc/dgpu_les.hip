@@ -161,7 +161,7 @@ __global__ void k_les_bc_put(Geo g, cx<double> *__restrict__ p0, cx<double> *__r
 // and eight row fields out, 2.9 TB/s; three waves per SIMD; 2.29 ms with two
 // positions a thread, 256 registers and 44 of them spilled); it replaces the x
 // kernel (1.30 ms), nine plane transforms (2.9 ms) and seven pointwise kernels
-// (2.9 ms) of the Fortran-layout form, a substep of 18.1 ms, now 7.9.
+// (2.9 ms) of the Fortran-layout form, a substep of 18.1 ms, now 8.1.
 // -------------------------------------------------------------------------
 constexpr int kStash = 8;
 template <int E, int NTH, int PID, int LM, bool WIDE>
